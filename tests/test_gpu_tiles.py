@@ -1,0 +1,45 @@
+"""Tiled kernels at the sizes where a tile can go wrong (bit-exact against numpy)."""
+import numpy as np
+import pytest
+
+from conftest import gdl
+
+pytestmark = pytest.mark.gpu
+
+M32 = np.uint64(0xffffffff)
+
+
+def runs_of(lengths, gap=1):
+    """Sorted keys whose prefixes 0, gap, 2 gap, ... have runs of these lengths."""
+    lengths = np.asarray(lengths, dtype=np.int64)
+    p = np.repeat(np.arange(lengths.size, dtype=np.uint64) * np.uint64(gap), lengths)
+    j = np.arange(lengths.sum()) - np.repeat(np.cumsum(lengths) - lengths, lengths)
+    return gdl.pack(p, j)
+
+
+# a wave reads spans of 256 keys (1024 from 2^22 keys on); the last run of a
+# span is followed past it, 64 keys, then doubling distances
+INDEX_RUNS = {
+    "one": [1], "wave": [64], "span": [256], "span+1": [257], "ends": [255, 1, 256, 2, 254, 3],
+    "ones": [1] * 1025, "past64": [200, 56 + 64, 1], "past65": [200, 56 + 65, 1],
+    "doubling": [1] + [255 + 64 * (1 << k) + d for k in range(6) for d in (-1, 0, 1)],
+    "hub": [3, 1_000_001, 7], "mixed": [(i * i) % 97 + 1 for i in range(3000)],
+    "long": [1500, 1024, 1023, 1025, 1, 4096] * 400 + [63, 64, 65] * 1500,
+    "long_hub": [5, (1 << 22) + 3, 2],
+}
+
+
+@pytest.mark.parametrize("gap", [1, 100_003])
+@pytest.mark.parametrize("name", INDEX_RUNS)
+def test_index_runs_at_span_edges(ctx, name, gap):
+    lengths = np.asarray(INDEX_RUNS[name], dtype=np.int64)
+    keys = runs_of(lengths, gap)
+    d = ctx.to_device(keys)
+    idx = ctx.index_build(d, 1)
+    assert idx.n_distinct == lengths.size and idx.max_run == lengths.max()
+    q = np.arange(lengths.size, dtype=np.uint64) * np.uint64(gap)
+    b, c = ctx.index_lookup(idx, d, q)
+    assert np.array_equal(c.astype(np.int64), lengths)
+    assert np.array_equal(b.astype(np.int64), np.cumsum(lengths) - lengths)
+    ctx.index_free(idx)
+    d.free()
