@@ -43,3 +43,38 @@ def test_index_runs_at_span_edges(ctx, name, gap):
     assert np.array_equal(b.astype(np.int64), np.cumsum(lengths) - lengths)
     ctx.index_free(idx)
     d.free()
+
+
+def np_join_runs(inner, outer):
+    p = inner >> np.uint64(32)
+    lo = np.searchsorted(p, outer >> np.uint64(32))
+    cnt = np.searchsorted(p, outer >> np.uint64(32), side="right") - lo
+    oi = np.repeat(np.arange(outer.size), cnt)
+    ii = np.repeat(lo - (np.cumsum(cnt) - cnt), cnt) + np.arange(oi.size)
+    return inner[ii], outer[oi], cnt
+
+
+# run lengths of the inner prefixes, and which prefix each outer tuple asks for
+# (a prefix past the last one has no run): tiles are 2048 outputs, a block's
+# threads take 256 outer tuples at a time
+JOIN_SHAPES = {
+    "one": ([1], [0]), "tile": ([2048], [0]), "tile+1": ([2048, 1], [0, 1]),
+    "ends_at_tile": ([1024, 1024, 5], [0, 1, 2, 0, 1, 2]),
+    "holes": ([3, 2045, 2], [9] * 300 + [0] + [9] * 700 + [1] + [9] * 5 + [2] * 2000 + [9] * 900),
+    "ones": ([1] * 50, [i % 57 for i in range(5000)]),
+    "hub": ([100_000, 1, 2], [1] * 10 + [0] + [2] * 600 + [7] * 600 + [0, 0, 1]),
+    "words": ([63, 64, 65, 1, 128], [i % 6 for i in range(1000)]),
+    "all_missing_but_last": ([4], [5] * 3000 + [0]),
+    # enough tiles for a block to take several
+    "many": ([i % 40 for i in range(1, 4000)], [(i * 7919) % 4100 for i in range(600_000)]),
+}
+
+
+@pytest.mark.parametrize("name", JOIN_SHAPES)
+def test_join_outputs_at_tile_edges(ctx, name):
+    lengths, asks = JOIN_SHAPES[name]
+    inner = runs_of(lengths)
+    outer = gdl.pack(np.asarray(asks), np.arange(len(asks)))
+    ik, ok, _ = np_join_runs(inner, outer)
+    got = ctx.join(inner, outer, (1, 3))  # (inner c1, outer c1)
+    assert np.array_equal(got, ((ik & M32) << np.uint64(32)) | (ok & M32))
