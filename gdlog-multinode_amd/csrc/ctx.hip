@@ -12,7 +12,7 @@ namespace gdl {
 const char *kKernelNames[K_NUM] = {
     "rs_upsweep",   "rs_rowscan",   "rs_downsweep", "rs_oneblock",   "key_bits",
     "scan_reduce",  "scan_top",     "scan_down",    "compact_count", "compact_write",
-    "merge_count",  "merge_write",  "idx_count",    "idx_build",     "idx_lookup",
+    "merge",  "idx_count",    "idx_build",     "idx_lookup",
     "join_count",   "join_materialize", "project",  "fill",          "hs_insert_new",
     "hs_rehash",    "join_insert",  "hs_extract",   "seg_hist",      "mask_cols",
     "linear_body",  "segment_labels", "scatter_by_key", "dense_setup", "dense_expand",
@@ -134,6 +134,34 @@ gdl_status read_u64(gdl_ctx *ctx, const u64 *d, u64 *h, int count) {
                                 ctx->stream));
     GDL_HIP(ctx, hipStreamSynchronize(ctx->stream));
     memcpy(h, ctx->h_pinned, sizeof(u64) * count);
+    return GDL_OK;
+}
+
+gdl_status read_result(gdl_ctx *ctx, u64 *h) {
+    GDL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    *h = *(volatile u64 *)result_word(ctx);
+    return GDL_OK;
+}
+
+gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out) {
+    if (tiles > ctx->tile_cap) {
+        // outside the caching allocator: it lives as long as the context
+        const u64 cap = std::max<u64>({tiles, 2 * ctx->tile_cap, kTilesMin});
+        uint64_t *p = nullptr;
+        GDL_HIP(ctx, hipMalloc((void **)&p, (kTileWordsAt + cap) * sizeof(u64)));
+        if (ctx->d_tiles) (void)hipFree(ctx->d_tiles);  // waits for the device
+        ctx->d_tiles = p;
+        ctx->tile_cap = cap;
+        ctx->tile_epoch = 255;
+    }
+    if (ctx->tile_epoch >= 255) {
+        GDL_HIP(ctx, hipMemsetAsync(ctx->d_tiles, 0, (kTileWordsAt + ctx->tile_cap) * sizeof(u64),
+                                    ctx->stream));
+        ctx->tile_epoch = 0;
+    }
+    out->ticket = (unsigned int *)ctx->d_tiles;
+    out->words = (unsigned long long *)ctx->d_tiles + kTileWordsAt;
+    out->epoch = ++ctx->tile_epoch;
     return GDL_OK;
 }
 
@@ -343,7 +371,8 @@ gdl_status gdl_ctx_create(const gdl_config *cfg_in, gdl_ctx **out) {
         gdl_ctx_destroy(ctx);
         return GDL_ERR_HIP;
     }
-    if (noalloc_setup(ctx) != GDL_OK) {
+    TileLook look;  // its memory comes with the context
+    if (tile_look(ctx, kTilesMin, &look) != GDL_OK || noalloc_setup(ctx) != GDL_OK) {
         gdl_ctx_destroy(ctx);
         return GDL_ERR_HIP;
     }
@@ -362,6 +391,7 @@ gdl_status gdl_ctx_destroy(gdl_ctx *ctx) {
     for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
     delete ctx->alloc;
     if (ctx->d_err) (void)hipFree(ctx->d_err);
+    if (ctx->d_tiles) (void)hipFree(ctx->d_tiles);
     if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
     if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

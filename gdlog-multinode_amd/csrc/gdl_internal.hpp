@@ -61,8 +61,7 @@ enum KernelId {
     K_SCAN_DOWN,
     K_COMPACT_COUNT,
     K_COMPACT_WRITE,
-    K_MERGE_COUNT,
-    K_MERGE_WRITE,
+    K_MERGE,
     K_IDX_COUNT,
     K_IDX_BUILD,
     K_IDX_LOOKUP,
@@ -113,6 +112,9 @@ struct gdl_ctx {
     char *h_stage = nullptr;       // pinned staging for bulk copies (gdl::Staging)
     size_t h_stage_cap = 0;
     uint32_t *d_err = nullptr;     // kernel-side error word
+    uint64_t *d_tiles = nullptr;   // running sums of single-pass kernels (gdl::TileLook)
+    uint64_t tile_cap = 0;         // tiles d_tiles has room for
+    uint32_t tile_epoch = 0;       // the last call's tag, 0..255
     int cu_count = 0;
     gdl_tuning tune{GDL_DEFAULT_LOAD_FACTOR, 8, 8, 256};  // load_factor mirrors cfg.load_factor
     std::string last_error;
@@ -254,6 +256,23 @@ class Staging {
     std::vector<Pending> pending_;
 };
 
+// Running sums over the tiles of one kernel (tile_before below): a ticket
+// counter and a word per tile, kept with the context.  Every call tags its
+// words with an epoch of its own, so they are cleared once in 255 calls and
+// not before each; the calls of a context follow each other on its stream.
+struct TileLook {
+    unsigned long long *words;
+    unsigned int *ticket;
+    u32 epoch;
+};
+constexpr u64 kTileWordsAt = 16;  // the words' place in d_tiles, after the ticket's line
+constexpr u64 kTilesMin = 16384;
+gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out);
+// A pinned word that a kernel of the context's stream can write its result to
+// (no copy back to the host), and its value once the stream has been waited for.
+inline u64 *result_word(gdl_ctx *ctx) { return ctx->h_pinned + 63; }
+gdl_status read_result(gdl_ctx *ctx, u64 *h);
+
 // ---- internal entry points shared between translation units
 gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *d_out,
                                      u64 *total_host /* may be null: no sync */);
@@ -299,8 +318,6 @@ bool dense_join_insert(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner, const u64 
 gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
                      const u64 *d_delta, u64 n_delta, u64 **d_log, u64 *log_cap, u64 *log_end,
                      int max_bodies, u64 *h_new, u64 *h_raw, int *bodies);
-// Exclusive scans of two arrays in place in one launch (v[n] = total each).
-gdl_status scan_inplace2(gdl_ctx *ctx, u64 *v0, u64 *v1, u64 n, u64 *totals /* 2 */);
 
 inline unsigned grid_for(u64 n, u64 per_block) {
     u64 g = (n + per_block - 1) / per_block;
@@ -355,6 +372,69 @@ __device__ __forceinline__ u64 block_exclusive_scan(u64 v, u64 *s_wave, u64 *tot
     *total = s_wave[NW];
     __syncthreads();
     return res;
+}
+
+// A block's tile, in the order in which blocks start: every tile before it
+// belongs to a block that is running or done.  `s_tile` is a shared word.
+__device__ __forceinline__ u32 tile_ticket(const TileLook &look, u32 *s_tile) {
+    if (gridDim.x == 1) return 0;
+    if (threadIdx.x == 0) {
+        const u32 t = atomicAdd(look.ticket, 1u);
+        // the last ticket is out: back to 0 for the next kernel
+        if (t == gridDim.x - 1) atomicExch(look.ticket, 0u);
+        *s_tile = t;
+    }
+    __syncthreads();
+    return *s_tile;
+}
+
+// The sum of the aggregates of all tiles before `tile`, by one whole wave
+// (values below 2^54).  A tile's word says epoch (8 bits), state (2 bits: 1 =
+// its own aggregate, 2 = the sum up to and with it) and value in one 64-bit
+// store, so no other ordering is needed; loads and stores are of agent scope,
+// since tiles run on all XCDs.  The wave reads 64 predecessors at a time and
+// waits only for words of blocks that already run and publish their aggregate
+// without waiting for anything, so the wait ends.
+__device__ __forceinline__ u64 tile_before(const TileLook &look, u32 tile, u64 aggregate) {
+    const int lane = threadIdx.x & 63;
+    const u64 tag = (u64)look.epoch << 56, value = (1ull << 54) - 1;
+    auto put = [&](u64 state, u64 v) {
+        if (lane == 0)
+            __hip_atomic_store(&look.words[tile], (unsigned long long)(tag | (state << 54) | v),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (tile == 0) {
+        if (gridDim.x > 1) put(2, aggregate);
+        return 0;
+    }
+    put(1, aggregate);
+    u64 before = 0;
+    for (long long last = (long long)tile - 1;; last -= 64) {
+        const long long j = last - lane;
+        u64 w = 0;
+        u32 state = 2;  // before the first tile: a sum of 0
+        int first;
+        for (;;) {
+            if (j >= 0) {
+                w = __hip_atomic_load(&look.words[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                state = (w >> 56) == look.epoch ? (u32)(w >> 54) & 3u : 0u;
+            }
+            const u64 sums = __ballot(state == 2), none = __ballot(state == 0);
+            first = sums ? __ffsll((unsigned long long)sums) - 1 : 63;
+            // ready: a state for every tile up to the nearest sum
+            if (!(none & ((2ull << first) - 1ull))) {
+                first = sums ? first : 64;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        u64 v = j >= 0 && lane <= first ? w & value : 0;
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+        before += v;
+        if (first < 64) break;
+    }
+    put(2, before + aggregate);
+    return before;
 }
 
 __device__ __forceinline__ u32 key_col(u64 k, int c) {

@@ -5,175 +5,164 @@
 // A B-key is a duplicate exactly when the A-key consumed just before it is
 // equal (equal keys are adjacent in merge order and A goes first).
 //
-// Two launches per merge plus a scan of per-tile counts: count (per 2048-key
-// tile of the merged sequence: |U|, |D|) and write (LDS-staged, coalesced).
+// One launch: a block takes a tile of keys of the merged sequence, finds where its B-keys go among its A-keys, counts the duplicates, learns how many
+// the tiles before hold (tile_before), and writes its part of U and D.
 #include "gdl_internal.hpp"
 
 namespace gdl {
 
-constexpr int MG_B = 256;
-constexpr int MG_I = 8;
-constexpr int MG_TILE = MG_B * MG_I;
+constexpr int MG_I = 8;  // keys per thread
 
-// Number of A-keys among the first `diag` keys of the merge (A first on ties).
+// Number of A-keys among the first `diag` keys of the merge (A first on ties),
+// by a whole wave: 64 probes a round (5 rounds for 41M keys, where a thread's
+// binary search is 26 dependent loads).
 __device__ __forceinline__ u64 merge_path(const u64 *A, u64 na, const u64 *B, u64 nb, u64 diag) {
+    const int lane = threadIdx.x & 63;
     u64 lo = diag > nb ? diag - nb : 0;
     u64 hi = diag < na ? diag : na;
     while (lo < hi) {
-        const u64 mid = (lo + hi) >> 1;
-        if (A[mid] <= B[diag - 1 - mid]) lo = mid + 1;
-        else hi = mid;
+        const u64 step = (hi - lo + 63) / 64;
+        const u64 m = lo + (u64)lane * step;
+        const u64 past = ~__ballot(m < hi && A[m] <= B[diag - 1 - m]);
+        const int f = past ? __ffsll((unsigned long long)past) - 1 : 64;
+        if (f == 0) break;  // A[lo] comes after the diagonal
+        const u64 next = lo + (u64)f * step;
+        lo += (u64)(f - 1) * step + 1;
+        if (next < hi) hi = next;
     }
     return lo;
 }
 
-struct TileSplit {
-    u64 i0, j0;  // start of the tile in A and B
-    u32 la, lb;  // lengths in A and B
-};
+// The exclusive prefix sums of the population counts of N words, by one whole
+// wave; returns the total.
+template <int N>
+__device__ __forceinline__ u32 scan_words(const u64 *words, u32 *before) {
+    constexpr int PER = N > 64 ? N / 64 : 1;
+    const int lane = threadIdx.x & 63;
+    u32 c[PER], sum = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = lane * PER + j;
+        c[j] = i < N ? (u32)__popcll(words[i]) : 0;
+        sum += c[j];
+    }
+    u32 x = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const u32 y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    u32 at = x - sum;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = lane * PER + j;
+        if (i < N) before[i] = at;
+        at += c[j];
+    }
+    return __shfl(x, 63, 64);
+}
 
-// Loads the tile's A and B ranges into s (A at [0, la), B at [la, la + lb)),
-// and the A-key before the tile into *s_prev (s_has_prev = 0 if none).
-__device__ __forceinline__ TileSplit load_tile(const u64 *A, u64 na, const u64 *B, u64 nb, u64 *s,
-                                               u64 *s_split, u64 *s_prev, u32 *s_has_prev,
-                                               u32 *err) {
-    const int t = threadIdx.x;
-    const u64 d0 = (u64)blockIdx.x * MG_TILE;
-    const u64 tot = na + nb;
+// U (may be null) gets A u B, D (may be null) B \ A; *dups the duplicates'
+// number, so |U| = na + nb - *dups and |D| = nb - *dups.  Each B-key finds its
+// place among the tile's A-keys by a search in LDS and marks it in a bit
+// array; the output at w of the tile is then the B-key after as many B-keys as
+// are marked before w, or the A-key after the rest.  Consecutive lanes write
+// consecutive outputs.  41M + 2M keys: 0.235 ms, 2.9 TB/s (a count and a write
+// launch, each merging a thread's 8 keys one by one, took 0.245 + 0.309 ms).
+template <int MG_B>
+__global__ __launch_bounds__(MG_B) void k_merge(const u64 *A, u64 na, const u64 *B, u64 nb,
+                                                u64 *U, u64 *D, TileLook look, u64 *dups,
+                                                u32 *err) {
+    constexpr int MG_TILE = MG_B * MG_I, MG_W = MG_TILE / 64;
+    __shared__ u64 s[MG_TILE];
+    __shared__ u64 s_is_b[MG_W], s_dup[MG_W];
+    __shared__ u32 s_nb[MG_W], s_nd[MG_W];  // marks in the words before
+    __shared__ u64 s_split[2], s_before;
+    __shared__ u32 s_tile;
+    const int t = threadIdx.x, lane = t & 63;
+    const u32 tile = tile_ticket(look, &s_tile);
+    const u64 d0 = (u64)tile * MG_TILE, tot = na + nb;
     const u64 d1 = d0 + MG_TILE < tot ? d0 + MG_TILE : tot;
-    if (t == 0) s_split[0] = merge_path(A, na, B, nb, d0);
-    if (t == 64) s_split[1] = merge_path(A, na, B, nb, d1);
+    if (t < 128) {
+        const u64 i = merge_path(A, na, B, nb, t < 64 ? d0 : d1);
+        if (lane == 0) s_split[t >> 6] = i;
+    }
+    if (t < MG_W) s_is_b[t] = s_dup[t] = 0;
     __syncthreads();
-    TileSplit sp;
-    sp.i0 = s_split[0];
-    const u64 i1 = s_split[1];
-    sp.j0 = d0 - sp.i0;
+    const u64 i0 = s_split[0], j0 = d0 - i0;
     // sorted inputs give i0 <= i1 <= i0 + (d1 - d0); anything else is treated
     // as an empty tile so no LDS or global index leaves its buffer
-    if (i1 < sp.i0 || i1 - sp.i0 > d1 - d0) {
+    u32 la = 0, lb = 0;
+    if (s_split[1] < i0 || s_split[1] - i0 > d1 - d0) {
         if (t == 0) atomicOr(err, 4u);
-        sp.la = 0;
-        sp.lb = 0;
-        __syncthreads();
-        return sp;
+    } else {
+        la = (u32)(s_split[1] - i0);
+        lb = (u32)(d1 - d0) - la;
     }
-    sp.la = (u32)(i1 - sp.i0);
-    sp.lb = (u32)((d1 - i1) - sp.j0);
-    for (u32 x = t; x < sp.la; x += MG_B) s[x] = A[sp.i0 + x];
-    for (u32 x = t; x < sp.lb; x += MG_B) s[sp.la + x] = B[sp.j0 + x];
-    if (t == 0) {
-        *s_has_prev = sp.i0 > 0 ? 1u : 0u;
-        *s_prev = sp.i0 > 0 ? A[sp.i0 - 1] : 0;
+#pragma unroll
+    for (int r = 0; r < MG_I; ++r) {
+        const u32 x = r * MG_B + t;
+        if (x < la + lb) s[x] = x < la ? A[i0 + x] : B[j0 + (x - la)];
+    }
+    const bool has_prev = i0 > 0;
+    const u64 prev = has_prev ? A[i0 - 1] : 0;
+    __syncthreads();
+    u32 place[MG_I];  // of this thread's B-keys; bit 31: a duplicate
+#pragma unroll
+    for (int r = 0; r < MG_I; ++r) {
+        const u32 x = r * MG_B + t;
+        if (x >= lb) continue;
+        const u64 v = s[la + x];
+        u32 lo = 0, hi = la;  // A-keys <= v
+        while (lo < hi) {
+            const u32 mid = (lo + hi) >> 1;
+            if (s[mid] <= v) lo = mid + 1;
+            else hi = mid;
+        }
+        const bool dup = lo ? s[lo - 1] == v : has_prev && prev == v;
+        const u32 w = lo + x;
+        atomicOr((unsigned long long *)&s_is_b[w >> 6], 1ull << (w & 63));
+        if (dup) atomicOr((unsigned long long *)&s_dup[w >> 6], 1ull << (w & 63));
+        place[r] = w | (dup ? 1u << 31 : 0u);
     }
     __syncthreads();
-    return sp;
-}
-
-// Serial merge of this thread's MG_I merge steps inside the tile.  Bit r of
-// *is_u / *is_d says output r is a union / difference element; vals[r] holds it.
-__device__ __forceinline__ void thread_merge(const u64 *s, const TileSplit &sp, u64 prev,
-                                             bool has_prev, u64 *vals, u32 *is_u, u32 *is_d,
-                                             u32 *nu, u32 *nd) {
-    const u32 t = threadIdx.x;
-    const u32 tile_len = sp.la + sp.lb;
-    const u32 k0 = t * MG_I;
-    *is_u = 0;
-    *is_d = 0;
-    *nu = 0;
-    *nd = 0;
-    if (k0 >= tile_len) return;
-    const u32 steps = tile_len - k0 < (u32)MG_I ? tile_len - k0 : (u32)MG_I;
-    const u64 *sA = s;
-    const u64 *sB = s + sp.la;
-    // local merge path
-    u32 lo = k0 > sp.lb ? k0 - sp.lb : 0;
-    u32 hi = k0 < sp.la ? k0 : sp.la;
-    while (lo < hi) {
-        const u32 mid = (lo + hi) >> 1;
-        if (sA[mid] <= sB[k0 - 1 - mid]) lo = mid + 1;
-        else hi = mid;
+    if (t < 64) {
+        const u64 mine = scan_words<MG_W>(s_dup, s_nd);
+        const u64 before = tile_before(look, tile, mine);
+        if (t == 0) {
+            s_before = before;
+            if (tile == gridDim.x - 1) *dups = before + mine;
+        }
+    } else if (t < 128) {
+        scan_words<MG_W>(s_is_b, s_nb);
     }
-    u32 ia = lo, ib = k0 - lo;
-    u64 last_a = ia > 0 ? sA[ia - 1] : prev;
-    bool has_last = ia > 0 || has_prev;
+    __syncthreads();
+    const u64 before = s_before;
+    if (U) {
+        const u64 lt = lane_mask_lt();
 #pragma unroll
-    for (u32 r = 0; r < (u32)MG_I; ++r) {
-        if (r >= steps) break;
-        const bool take_a = ib >= sp.lb || (ia < sp.la && sA[ia] <= sB[ib]);
-        if (take_a) {
-            last_a = sA[ia++];
-            has_last = true;
-            vals[r] = last_a;
-            *is_u |= 1u << r;
-            ++*nu;
-        } else {
-            const u64 v = sB[ib++];
-            vals[r] = v;
-            if (!(has_last && last_a == v)) {
-                *is_u |= 1u << r;
-                *is_d |= 1u << r;
-                ++*nu;
-                ++*nd;
-            }
+        for (int r = 0; r < MG_I; ++r) {
+            const u32 w = r * MG_B + t;
+            if (w >= la + lb) continue;
+            const u64 is_b = s_is_b[w >> 6], dup = s_dup[w >> 6];
+            const u32 nb_at = s_nb[w >> 6] + (u32)__popcll(is_b & lt);
+            const u32 nd_at = s_nd[w >> 6] + (u32)__popcll(dup & lt);
+            const u64 at = d0 + w - nd_at - before;
+            if (!((dup >> lane) & 1ull) && at < tot)
+                __builtin_nontemporal_store(((is_b >> lane) & 1ull) ? s[la + nb_at] : s[w - nb_at],
+                                            &U[at]);
         }
     }
-}
-
-__global__ __launch_bounds__(MG_B) void k_merge_count(const u64 *A, u64 na, const u64 *B, u64 nb,
-                                                      u64 *tile_u, u64 *tile_d, u32 *err) {
-    __shared__ u64 s[MG_TILE];
-    __shared__ u64 s_split[2];
-    __shared__ u64 s_prev;
-    __shared__ u32 s_has_prev;
-    __shared__ u64 s_w[MG_B / 64 + 1];
-    const TileSplit sp = load_tile(A, na, B, nb, s, s_split, &s_prev, &s_has_prev, err);
-    u64 vals[MG_I];
-    u32 iu, id, nu, nd;
-    thread_merge(s, sp, s_prev, s_has_prev != 0, vals, &iu, &id, &nu, &nd);
-    u64 tu, td;
-    block_exclusive_scan<MG_B>(nu, s_w, &tu);
-    block_exclusive_scan<MG_B>(nd, s_w, &td);
-    if (threadIdx.x == 0) {
-        tile_u[blockIdx.x] = tu;
-        tile_d[blockIdx.x] = td;
-    }
-}
-
-// off_u / off_d: exclusive scans of the tile counts.  U or D may be null.
-__global__ __launch_bounds__(MG_B) void k_merge_write(const u64 *A, u64 na, const u64 *B, u64 nb,
-                                                      const u64 *off_u, const u64 *off_d, u64 *U,
-                                                      u64 *D, u32 *err) {
-    __shared__ u64 s[MG_TILE];
-    __shared__ u64 s_split[2];
-    __shared__ u64 s_prev;
-    __shared__ u32 s_has_prev;
-    __shared__ u64 s_w[MG_B / 64 + 1];
-    const TileSplit sp = load_tile(A, na, B, nb, s, s_split, &s_prev, &s_has_prev, err);
-    u64 vals[MG_I];
-    u32 iu, id, nu, nd;
-    thread_merge(s, sp, s_prev, s_has_prev != 0, vals, &iu, &id, &nu, &nd);
-    u64 tu, td;
-    const u64 pu = block_exclusive_scan<MG_B>(nu, s_w, &tu);
-    const u64 pd = block_exclusive_scan<MG_B>(nd, s_w, &td);
-    // s is free again (block_exclusive_scan ended with a barrier)
-    if (U) {
-        u32 k = 0;
-#pragma unroll
-        for (int r = 0; r < MG_I; ++r)
-            if ((iu >> r) & 1u) s[pu + k++] = vals[r];
-        __syncthreads();
-        const u64 base = off_u[blockIdx.x];
-        for (u32 x = threadIdx.x; x < (u32)tu; x += MG_B) U[base + x] = s[x];
-        __syncthreads();
-    }
     if (D) {
-        u32 k = 0;
 #pragma unroll
-        for (int r = 0; r < MG_I; ++r)
-            if ((id >> r) & 1u) s[pd + k++] = vals[r];
-        __syncthreads();
-        const u64 base = off_d[blockIdx.x];
-        for (u32 x = threadIdx.x; x < (u32)td; x += MG_B) D[base + x] = s[x];
+        for (int r = 0; r < MG_I; ++r) {
+            const u32 x = r * MG_B + t;
+            if (x >= lb || (place[r] >> 31)) continue;
+            const u32 w = place[r];
+            const u32 nd_at =
+                s_nd[w >> 6] + (u32)__popcll(s_dup[w >> 6] & ((1ull << (w & 63)) - 1ull));
+            const u64 at = j0 + x - nd_at - before;
+            if (at < nb) D[at] = s[la + x];  // (always, if the inputs are sorted)
+        }
     }
 }
 
@@ -185,33 +174,31 @@ static gdl_status merge_impl(gdl_ctx *ctx, const u64 *A, u64 na, const u64 *B, u
         if (n_d) *n_d = 0;
         return GDL_OK;
     }
-    const u64 nt = (tot + MG_TILE - 1) / MG_TILE;
-    if (nt > 0xffffffffull) return fail(ctx, GDL_ERR_OVERFLOW, "merge: too many tiles");
-    Scratch scr(ctx);
-    u64 *ou, *od, *totals;
-    GDL_TRY(scr.get(nt + 1, &ou));
-    GDL_TRY(scr.get(nt + 1, &od));
-    GDL_TRY(scr.get(2, &totals));
-    {
-        KTimer kt(ctx, K_MERGE_COUNT, 8.0 * tot);
-        hipLaunchKernelGGL(k_merge_count, dim3((unsigned)nt), dim3(MG_B), 0, ctx->stream, A, na, B,
-                           nb, ou, od, ctx->d_err);
-        GDL_TRY(check_launch(ctx, "k_merge_count"));
-    }
-    GDL_TRY(scan_inplace2(ctx, ou, od, nt, totals));
+    // Tickets come at 11 ns each (atomics on one word), so 41M + 2M keys in
+    // tiles of 2048 took 395 us, 240 of them in 21,000 tickets; in tiles of
+    // 8192 keys it takes 235 us.  Below 2^19 keys the smaller tiles spread over more CUs.
+    const bool big = tot >= 1ull << 19;
+    const u64 tile = (big ? 1024 : 256) * MG_I, nt = (tot + tile - 1) / tile;
+    if (nt > 0x7fffffffull) return fail(ctx, GDL_ERR_OVERFLOW, "merge: too many tiles");
+    TileLook look;
+    GDL_TRY(tile_look(ctx, nt, &look));
     {
         // algorithmic bytes: read A and B here; the U / D writes are added
         // below once their sizes are known
-        KTimer kt(ctx, K_MERGE_WRITE, 8.0 * tot);
-        hipLaunchKernelGGL(k_merge_write, dim3((unsigned)nt), dim3(MG_B), 0, ctx->stream, A, na, B,
-                           nb, ou, od, U, D, ctx->d_err);
-        GDL_TRY(check_launch(ctx, "k_merge_write"));
+        KTimer kt(ctx, K_MERGE, 8.0 * tot);
+        auto launch = [&](auto kern, int block) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream, A, na, B, nb,
+                               U, D, look, result_word(ctx), ctx->d_err);
+        };
+        if (big) launch(k_merge<1024>, 1024);
+        else launch(k_merge<256>, 256);
+        GDL_TRY(check_launch(ctx, "k_merge"));
     }
-    u64 h[2];
-    GDL_TRY(read_u64(ctx, totals, h, 2));
-    ctx->stats[K_MERGE_WRITE].alg_bytes += (U ? 8.0 * h[0] : 0.0) + (D ? 8.0 * h[1] : 0.0);
-    if (n_u) *n_u = h[0];
-    if (n_d) *n_d = h[1];
+    u64 dups = 0;
+    GDL_TRY(read_result(ctx, &dups));
+    ctx->stats[K_MERGE].alg_bytes += (U ? 8.0 * (tot - dups) : 0.0) + (D ? 8.0 * (nb - dups) : 0.0);
+    if (n_u) *n_u = tot - dups;
+    if (n_d) *n_d = nb - dups;
     return GDL_OK;
 }
 

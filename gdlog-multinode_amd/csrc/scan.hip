@@ -202,21 +202,6 @@ static gdl_status scan_top(gdl_ctx *ctx, u64 *v, u64 n, u64 *total_dev) {
     return check_launch(ctx, "k_scan_top");
 }
 
-gdl_status scan_inplace2(gdl_ctx *ctx, u64 *v0, u64 *v1, u64 n, u64 *totals) {
-    if (n > 262144) {
-        GDL_TRY(scan_inplace(ctx, v0, n));
-        GDL_TRY(scan_inplace(ctx, v1, n));
-        GDL_HIP(ctx, hipMemcpyAsync(totals, v0 + n, sizeof(u64), hipMemcpyDeviceToDevice,
-                                    ctx->stream));
-        GDL_HIP(ctx, hipMemcpyAsync(totals + 1, v1 + n, sizeof(u64), hipMemcpyDeviceToDevice,
-                                    ctx->stream));
-        return GDL_OK;
-    }
-    KTimer kt(ctx, K_SCAN_TOP, 32.0 * n);
-    hipLaunchKernelGGL(k_scan_top<1024>, dim3(2), dim3(1024), 0, ctx->stream, v0, v1, n, totals);
-    return check_launch(ctx, "k_scan_top");
-}
-
 template <typename T>
 static gdl_status exclusive_scan_impl(gdl_ctx *ctx, const T *d_in, u64 n, u64 *d_out,
                                       u64 *total_host) {

@@ -78,3 +78,34 @@ def test_join_outputs_at_tile_edges(ctx, name):
     ik, ok, _ = np_join_runs(inner, outer)
     got = ctx.join(inner, outer, (1, 3))  # (inner c1, outer c1)
     assert np.array_equal(got, ((ik & M32) << np.uint64(32)) | (ok & M32))
+
+
+def _sorted(rng, n, hi):
+    return np.sort(rng.choice(hi, size=n, replace=False)).astype(np.uint64) if n else \
+        np.zeros(0, np.uint64)
+
+
+# tiles are 2048 keys of the merged sequence; a tile may hold one side only,
+# and a duplicate may be the first key of a tile
+@pytest.mark.parametrize("na,nb,hi", [
+    (0, 1, 9), (1, 0, 9), (1, 1, 1), (2047, 1, 5000), (1024, 1024, 2048), (1024, 1024, 1024),
+    (2048, 2048, 2048), (2049, 2047, 4097), (5000, 5000, 5500), (100_000, 10, 10**6),
+    (10, 100_000, 10**6), (300_001, 299_999, 600_000), (700_000, 700_000, 700_000)])
+def test_merge_at_tile_edges(ctx, na, nb, hi):
+    rng = np.random.default_rng(na * 7 + nb)
+    a, b = _sorted(rng, na, hi), _sorted(rng, nb, hi)
+    for full, newt in ((a, b), (a, b + np.uint64(hi)), (a + np.uint64(hi), b)):
+        u, d = ctx.merge_diff(full, newt)
+        assert np.array_equal(u, np.union1d(full, newt))
+        assert np.array_equal(d, np.setdiff1d(newt, full))
+        assert np.array_equal(ctx.merge_union(full, newt), u)
+        assert np.array_equal(ctx.set_difference(newt, full), d)
+
+
+def test_tile_words_are_tagged_anew(ctx):
+    # the running sums' words are cleared once in 255 calls and tagged in between
+    a = np.arange(0, 60_000, 2, dtype=np.uint64)
+    for i in range(600):
+        n = 5000 + 97 * (i % 300)
+        b = np.arange(i % 7, 3 * n, 3, dtype=np.uint64)
+        assert ctx.set_difference(b, a).size == np.setdiff1d(b, a, assume_unique=True).size
