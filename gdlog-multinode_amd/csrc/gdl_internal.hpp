@@ -59,8 +59,8 @@ enum KernelId {
     K_SCAN_REDUCE,
     K_SCAN_TOP,
     K_SCAN_DOWN,
-    K_COMPACT_COUNT,
-    K_COMPACT_WRITE,
+    K_SCAN_ONE,
+    K_COMPACT,
     K_MERGE,
     K_IDX_COUNT,
     K_IDX_BUILD,

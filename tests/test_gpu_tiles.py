@@ -109,3 +109,30 @@ def test_tile_words_are_tagged_anew(ctx):
         n = 5000 + 97 * (i % 300)
         b = np.arange(i % 7, 3 * n, 3, dtype=np.uint64)
         assert ctx.set_difference(b, a).size == np.setdiff1d(b, a, assume_unique=True).size
+
+
+# tiles of 4096 keys, of 16384 from 2^20 keys on
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 4095, 4096, 4097, 12_289, (1 << 20) - 1, 1 << 20,
+                               (1 << 20) + 1, 2_000_003])
+@pytest.mark.parametrize("kind", ["none", "all", "half", "last", "tile_firsts"])
+def test_compaction_at_tile_edges(ctx, n, kind):
+    i = np.arange(n)
+    keep = {"none": i < 0, "all": i >= 0, "half": i % 2 == 1, "last": i == n - 1,
+            "tile_firsts": i % 4096 == 0}[kind]
+    # c0 == 7 where kept (a predicate on a column), c1 tells the keys apart
+    keys = gdl.pack(np.where(keep, 7, 8), i)
+    assert np.array_equal(ctx.filter(keys, gdl.PRED_EQ | 0x100, 0, 7), keys[keep])
+
+
+# one launch up to 2^22 values, three above; 2048 values a tile
+@pytest.mark.parametrize("n", [1, 8, 2047, 2048, 2049, 100_000, 1 << 22, (1 << 22) + 1])
+def test_join_offsets_at_tile_edges(ctx, n):
+    import ctypes
+    counts = (np.arange(n, dtype=np.uint64) * np.uint64(2654435761) & M32).astype(np.uint32)
+    counts[::3] = 0
+    d, o = ctx.to_device(counts, np.uint32), ctx.alloc(n + 1)
+    total = ctypes.c_uint64()
+    ctx._check(ctx.eng.gdl_join_scan(ctx.h, d.ptr, n, o.ptr, ctypes.byref(total)), "scan")
+    want = np.concatenate([[0], np.cumsum(counts.astype(np.uint64))]).astype(np.uint64)
+    assert np.array_equal(o.numpy(), want) and total.value == int(want[-1])
+    d.free(); o.free()
