@@ -10,7 +10,7 @@
 namespace gdl {
 
 const char *kKernelNames[K_NUM] = {
-    "rs_upsweep",   "rs_rowscan",   "rs_downsweep", "rs_oneblock",   "key_bits",
+    "rs_hist",      "rs_pass",      "rs_oneblock",   "key_bits",
     "scan_reduce",  "scan_top",     "scan_down",    "scan_one", "compact",
     "merge",  "idx_count",    "idx_build",     "idx_lookup",
     "join_count",   "join_materialize", "project",  "fill",          "hs_insert_new",

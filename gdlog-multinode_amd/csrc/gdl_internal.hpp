@@ -51,9 +51,8 @@ class Allocator {
 
 // ------------------------------------------------------------------ stats
 enum KernelId {
-    K_RS_UPSWEEP = 0,
-    K_RS_ROWSCAN,
-    K_RS_DOWNSWEEP,
+    K_RS_HIST = 0,
+    K_RS_PASS,
     K_RS_ONEBLOCK,
     K_KEY_BITS,
     K_SCAN_REDUCE,

@@ -1,8 +1,7 @@
 // Allocation-free sort + unique for callers that cannot allocate device
 // memory (code under HIP-graph capture, tight serving loops, harnesses that
 // forbid hipMalloc).  Its scratch -- the radix sort's ping-pong buffer and
-// digit histograms, the sorted copy ahead of the unique pass and the
-// compaction's tile counts -- lives in one file-scope device array of fixed
+// digit counts and the sorted copy ahead of the unique pass -- lives in one file-scope device array of fixed
 // size instead of the context allocator.
 //
 // Each GPU that loads this library holds the array until the process ends.
@@ -21,11 +20,11 @@ namespace gdl {
 
 static constexpr uint64_t kNoallocMaxKeys = GDL_NOALLOC_MAX_KEYS;
 // Worst case for kNoallocMaxKeys keys: the sorted copy (8n) and the radix
-// ping-pong buffer (8n), 2^9-bin digit counts per 4096-key tile, and the
-// compaction's tile counts, each piece 256-byte aligned.
+// ping-pong buffer (8n), two arrays of 2^9 digit counts per 4096-key tile, and
+// the passes' digit counts, each piece 256-byte aligned.
 static constexpr size_t kScratchBytes = 18u << 20;
-static_assert(kScratchBytes >= 16 * GDL_NOALLOC_MAX_KEYS + 4 * 512 * (GDL_NOALLOC_MAX_KEYS / 4096) +
-                                   (64u << 10),
+static_assert(kScratchBytes >= 16 * GDL_NOALLOC_MAX_KEYS +
+                                   2 * 4 * 512 * (GDL_NOALLOC_MAX_KEYS / 4096) + (64u << 10),
               "scratch array too small for the key limit");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];

@@ -136,3 +136,25 @@ def test_join_offsets_at_tile_edges(ctx, n):
     want = np.concatenate([[0], np.cumsum(counts.astype(np.uint64))]).astype(np.uint64)
     assert np.array_equal(o.numpy(), want) and total.value == int(want[-1])
     d.free(); o.free()
+
+
+# tiles of 2048 keys up to 2^18 keys, of 4096 up to 2^22, of 8192 above
+@pytest.mark.parametrize("n", [4097, 6144, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 1_000_001,
+                               1 << 22, (1 << 22) + 1, (1 << 22) + 8192])
+@pytest.mark.parametrize("kind", ["random36", "random32", "sorted", "reversed", "one_odd",
+                                  "few", "high_only"])
+def test_sort_at_tile_edges(ctx, n, kind):
+    rng = np.random.default_rng(n)
+    i = np.arange(n, dtype=np.uint64)
+    bits = 18 if kind == "random36" else 16 if kind == "random32" else 32
+    if kind.startswith("random"):
+        keys = gdl.pack(rng.integers(0, 1 << bits, n), rng.integers(0, 1 << bits, n))
+    elif kind == "one_odd":
+        keys = np.full(n, 0x0102030405060708, dtype=np.uint64)
+        keys[n // 2] = 0x0102030405060701
+    else:
+        keys = {"sorted": i * np.uint64(977), "reversed": i[::-1] * np.uint64(977),
+                "few": (i * np.uint64(7919)) % np.uint64(3) << np.uint64(40),
+                "high_only": gdl.pack(rng.integers(0, 1 << 31, n), np.zeros(n))}[kind]
+    assert np.array_equal(ctx.sort(keys, bits, bits), np.sort(keys))
+    assert np.array_equal(ctx.sort_unique(keys, -1, -1), np.unique(keys))
