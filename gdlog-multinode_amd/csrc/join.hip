@@ -354,28 +354,40 @@ __global__ __launch_bounds__(JB) void k_join_materialize(const u64 *inner, const
 constexpr u32 kStage = 256;
 constexpr u64 kHubRun = 32;  // longer inner runs may use the load-balanced variant
 
+// A cursor word counts the new keys (low bits) and, in a linear body, the
+// blocks that are done (from bit kDoneBit on), so that one atomic gives a
+// block its place in the output and tells it whether it is the last.
+constexpr int kDoneBit = 50;
+constexpr u64 kNewMask = (1ull << kDoneBit) - 1;
+
 // Writes stay below out_cap; a cursor past it tells the host the caller's
 // output bound was wrong.
 __device__ __forceinline__ void flush_stage(const u64 *stage, u32 n, u64 *out, u64 out_cap,
-                                            unsigned long long *cursor, int lane) {
+                                            unsigned long long *cursor, u64 base, int lane) {
     unsigned long long pos = 0;
-    if (lane == 0) pos = atomicAdd(cursor, (unsigned long long)n);
+    if (lane == 0) pos = base + (atomicAdd(cursor, (unsigned long long)n) & kNewMask);
     pos = __shfl(pos, 0, 64);
     for (u32 x = lane; x < n; x += 64)
         if (pos + x < out_cap) out[pos + x] = stage[x];
 }
 
 // End of a fused-join block: what the waves still stage goes out with one
-// cursor atomic for the whole block, and the produced count with one more
-// (instead of one of each per wave, all on the same two addresses).  Every
-// thread of the block calls it.
-template <int B>
-__device__ __forceinline__ void block_final_flush(u64 (*s_stage)[kStage], u32 staged,
+// cursor atomic for the whole block.  The produced count: one more atomic on
+// *produced_to (LIN = false), or a store to the block's own word there
+// (LIN = true, a linear body), which is at the device's coherence point before
+// the cursor says that the block is done: an agent-scope store that has been
+// waited for.  (A fence in its place writes the XCD's whole L2 back, in each of
+// a body's ~190 blocks.)  LIN returns whether this block is the last, and the
+// new keys of all blocks in *total.  Every thread of the block calls it.
+template <int B, bool LIN>
+__device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 staged,
                                                   u64 produced, u64 *out, u64 out_cap,
-                                                  unsigned long long *counters) {
+                                                  unsigned long long *cursor, u64 base,
+                                                  unsigned long long *produced_to, u64 *total) {
     __shared__ u32 s_cnt[B / 64];
     __shared__ u64 s_prod[B / 64];
-    __shared__ unsigned long long s_base;
+    __shared__ u64 s_base, s_total;
+    __shared__ bool s_last;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int d = 32; d >= 1; d >>= 1) produced += __shfl_xor(produced, d, 64);
     if (lane == 0) {
@@ -389,13 +401,18 @@ __device__ __forceinline__ void block_final_flush(u64 (*s_stage)[kStage], u32 st
             tot += s_cnt[v];
             prod += s_prod[v];
         }
-        s_base = tot ? atomicAdd(&counters[0], (unsigned long long)tot) : 0ull;
-        if (prod) atomicAdd(&counters[1], (unsigned long long)prod);
-        // release: both counter updates are ordered (device scope) before
-        // whatever this thread does next, so a caller that counts finished
-        // blocks after this function and reads the counters after an acquire
-        // fence sees them
-        __threadfence();
+        if constexpr (LIN) {
+            __hip_atomic_store(&produced_to[blockIdx.x], (unsigned long long)prod,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const u64 old = atomicAdd(cursor, (unsigned long long)((1ull << kDoneBit) | tot));
+            s_base = base + (old & kNewMask);
+            s_last = (old >> kDoneBit) == gridDim.x - 1;
+            s_total = (old & kNewMask) + tot;
+        } else {
+            if (prod) atomicAdd(produced_to, (unsigned long long)prod);
+            s_base = tot ? base + atomicAdd(cursor, (unsigned long long)tot) : 0;
+        }
     }
     __syncthreads();
     u64 off = s_base;
@@ -403,6 +420,11 @@ __device__ __forceinline__ void block_final_flush(u64 (*s_stage)[kStage], u32 st
     const u64 *stage = s_stage[w];
     for (u32 x = lane; x < staged; x += 64)
         if (off + x < out_cap) out[off + x] = stage[x];
+    if constexpr (LIN) {
+        *total = s_total;
+        return s_last;
+    }
+    return false;
 }
 
 // Target of a fused join's inserts: one hash set, or one set per fixpoint
@@ -444,13 +466,15 @@ __device__ __forceinline__ void load_segs(const HsSel &h, gdl_hs_seg *s_segs) {
 }
 
 // One block's share of a fused join + insert (the blocks of the grid stride
-// over the outer tuples); counters[0] is the output cursor, counters[1] the
-// produced-tuple count.
-template <int B, bool SEG>
-__device__ __forceinline__ void join_insert_blocks(
+// over the outer tuples): new keys go to out from base + *cursor on.  LIN,
+// produced_to, total and the result as in block_final_flush; counters[2] flags
+// a key outside the id bound.
+template <int B, bool SEG, bool LIN>
+__device__ __forceinline__ bool join_insert_blocks(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
-    u64 out_cap, unsigned long long *counters) {
+    u64 out_cap, unsigned long long *cursor, u64 out_base, unsigned long long *produced_to,
+    unsigned long long *outside, u64 *total_new) {
     __shared__ u64 s_excl[B], s_b[B], s_ok[B];
     __shared__ u64 s_stage[B / 64][kStage];
     __shared__ gdl_hs_seg s_segs[SEG ? kMaxSegs : 1];
@@ -493,7 +517,7 @@ __device__ __forceinline__ void join_insert_blocks(
                     ++produced;
                     const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, key);
                     if (sel.dom_bits && !bm_in_domain(key, sel.dom_bits))
-                        atomicOr(&counters[2], 1ull);
+                        atomicOr(outside, 1ull);
                     else if (hs.slots)
                         fresh = hs_insert_key((u64 *)hs.slots, hs.mask, key);
                 }
@@ -502,7 +526,7 @@ __device__ __forceinline__ void join_insert_blocks(
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage(stage, staged, out, out_cap, &counters[0], lane);
+                flush_stage(stage, staged, out, out_cap, cursor, out_base, lane);
                 staged = 0;
                 wave_sync_lds();
             }
@@ -511,7 +535,8 @@ __device__ __forceinline__ void join_insert_blocks(
         }
         wave_sync_lds();  // s_excl / s_b / s_ok are rewritten next round
     }
-    block_final_flush<B>(s_stage, staged, produced, out, out_cap, counters);
+    return block_final_flush<B, LIN>(s_stage, staged, produced, out, out_cap, cursor, out_base,
+                                     produced_to, total_new);
 }
 
 template <int B, bool SEG>
@@ -519,15 +544,16 @@ __global__ __launch_bounds__(B) void k_join_insert(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
     u64 out_cap, unsigned long long *counters) {
-    join_insert_blocks<B, SEG>(slots, n_slots, inner, n_inner, shift, outer, n_outer, arity, s0,
-                               s1, pop, plhs, prhs, sel, out, out_cap, counters);
+    u64 unused;
+    join_insert_blocks<B, SEG, false>(slots, n_slots, inner, n_inner, shift, outer, n_outer, arity,
+                                      s0, s1, pop, plhs, prhs, sel, out, out_cap, &counters[0], 0,
+                                      &counters[1], &counters[2], &unused);
 }
 
 // State of a stream-ordered linear fixpoint (gdl_fixpoint_linear) in device
-// memory.  cursor and produced come first: they are a body's counters.
+// memory.
 struct LinState {
-    unsigned long long cursor;    // log end while a body runs
-    unsigned long long produced;  // tuples the body produced
+    unsigned long long cursor;    // the running body's new keys and finished blocks (kDoneBit)
     u64 delta_begin, delta_end;   // the body's delta: log[delta_begin, delta_end)
     u64 size;                     // hash set members
     u64 hs_limit;                 // members the set may reach (a fraction of its capacity)
@@ -536,30 +562,25 @@ struct LinState {
     u64 delta_limit;              // a larger delta ends the chunk (the grid was sized smaller)
     u32 stop;                     // 0 run, 1 fixpoint, 2 grow first, 3 body limit, 4 overflow
     u32 body;                     // bodies finished in this call
-    u32 blocks_done;              // blocks of the running body that finished
     u32 max_bodies;
+    u32 pad_;
 };
 enum : u32 { kLinRun = 0, kLinFixpoint = 1, kLinGrow = 2, kLinLimit = 3, kLinOverflow = 4 };
 
 // End of a body (thread 0 of the last block to finish): record its counts,
-// move the delta window to the tuples it appended, and decide whether the
-// next enqueued body runs.  Every block releases its cursor / produced
-// updates (a device-scope fence) before it counts itself finished, and the
-// last block fences again before reading them, so the atomic reads below see
-// the final values; the plain stores reach the next body at its launch.
-__device__ void linear_epilogue(LinState *st, u64 *counts, u64 d1) {
-    const u64 end = atomicAdd(&st->cursor, 0ull);
-    const u64 produced = atomicAdd(&st->produced, 0ull);
+// move the delta window to the nd tuples it appended from d1 on, and decide
+// whether the next enqueued body runs.  The plain stores reach the next body
+// at its launch.
+__device__ void linear_epilogue(LinState *st, u64 *counts, u64 d1, u64 nd, u64 produced) {
+    const u64 end = d1 + nd;
     const u32 b = st->body;
-    const u64 nd = end > d1 ? end - d1 : 0;
     counts[2 * b] = nd;
     counts[2 * b + 1] = produced;
     const u64 size = st->size + nd;
     st->size = size;
     st->delta_begin = d1;
     st->delta_end = end;
-    st->produced = 0;
-    st->blocks_done = 0;
+    st->cursor = 0;
     st->body = b + 1;
     u32 stop = kLinRun;
     if (end > st->log_cap) stop = kLinOverflow;
@@ -572,26 +593,35 @@ __device__ void linear_epilogue(LinState *st, u64 *counts, u64 d1) {
 
 // One body of out := out U map(inner x delta) with FULL = hash set + append
 // log: the delta is the log's last segment, new tuples are appended after it.
-// A stop code set by an earlier body makes it return at once.
+// A stop code set by an earlier body makes it return at once.  produced: a
+// word per block.
 template <int B>
 __global__ __launch_bounds__(B) void k_linear_body(const IdxSlot *slots, u64 n_slots,
                                                    const u64 *inner, u64 n_inner, int shift,
                                                    int arity, int s0, int s1, int pop, int plhs,
                                                    int prhs, u64 *hs_slots, u64 hs_mask, u64 *log,
-                                                   LinState *st, u64 *counts) {
-    __shared__ bool s_last;
+                                                   LinState *st, unsigned long long *produced,
+                                                   u64 *counts) {
+    __shared__ u64 s_sum[B / 64];
     if (st->stop != kLinRun) return;  // the same for every block
     const u64 d0 = st->delta_begin, d1 = st->delta_end;
-    join_insert_blocks<B, false>(slots, n_slots, inner, n_inner, shift, log + d0, d1 - d0, arity,
-                                 s0, s1, pop, plhs, prhs, HsSel{hs_slots, hs_mask, nullptr, 0, 0},
-                                 log, st->log_cap, &st->cursor);
-    // join_insert_blocks ends with this block's counter updates acknowledged
-    // (thread 0, before a barrier)
-    if (threadIdx.x == 0) s_last = atomicAdd(&st->blocks_done, 1u) == gridDim.x - 1;
+    u64 nd;
+    if (!join_insert_blocks<B, false, true>(
+            slots, n_slots, inner, n_inner, shift, log + d0, d1 - d0, arity, s0, s1, pop, plhs,
+            prhs, HsSel{hs_slots, hs_mask, nullptr, 0, 0, 0}, log, st->log_cap, &st->cursor, d1,
+            produced, nullptr, &nd))
+        return;
+    // the last block: every other one's count is at the coherence point
+    u64 sum = 0;
+    for (u32 i = threadIdx.x; i < gridDim.x; i += B)
+        sum += __hip_atomic_load(&produced[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
     __syncthreads();
-    if (s_last && threadIdx.x == 0) {
-        __threadfence();  // acquire: every block's counter updates precede its blocks_done add
-        linear_epilogue(st, counts, d1);
+    if (threadIdx.x == 0) {
+        sum = 0;
+        for (int v = 0; v < B / 64; ++v) sum += s_sum[v];
+        linear_epilogue(st, counts, d1, nd, sum);
     }
 }
 
@@ -696,7 +726,7 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage(stage, staged, out, out_cap, &counters[0], lane);
+                flush_stage(stage, staged, out, out_cap, &counters[0], 0, lane);
                 staged = 0;
                 wave_sync_lds();
             }
@@ -704,7 +734,9 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
             staged += cnt;
         }
     }
-    block_final_flush<JB>(s_stage, staged, produced, out, out_cap, counters);
+    u64 unused;
+    block_final_flush<JB, false>(s_stage, staged, produced, out, out_cap, &counters[0], 0,
+                                 &counters[1], &unused);
 }
 
 __global__ void k_set2(u64 *p, u64 a, u64 b) {
@@ -1210,9 +1242,10 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
     const int shift = inner_idx->prefix_cols >= 2 ? 0 : 32;
     const u64 mr = std::max<u64>(inner_idx->max_run, 1);
     Scratch scr(ctx);
-    u64 *st_words, *counts;
+    u64 *st_words, *counts, *produced;
     GDL_TRY(scr.get((sizeof(LinState) + 7) / 8, &st_words));
     GDL_TRY(scr.get(2 * kChunk, &counts));
+    GDL_TRY(scr.get(grid_cap(ctx), &produced));  // a word per block
     LinState *st = (LinState *)st_words;
     u64 d0 = *delta_begin, d1 = *delta_end;
     // TC's map over a bitmap FULL: bodies whose delta is dense run on bit
@@ -1266,7 +1299,7 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         }
         const int k = std::min({ramp, kChunk, max_bodies - done});
         LinState h{};
-        h.cursor = d1;
+        h.cursor = 0;
         h.delta_begin = d0;
         h.delta_end = d1;
         h.size = hs->size;
@@ -1290,7 +1323,8 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
                                (const IdxSlot *)inner_idx->slots, idx_arg(inner_idx), d_inner,
                                n_inner, shift, map.arity, map.src[0],
                                map.arity == 2 ? map.src[1] : 0, pred.op, pred.lhs, pred.rhs,
-                               (u64 *)hs->slots, hs_arg(hs), *d_log, st, counts);
+                               (u64 *)hs->slots, hs_arg(hs), *d_log, st,
+                               (unsigned long long *)produced, counts);
             GDL_TRY(check_launch(ctx, "k_linear_body"));
         }
         LinState r{};
