@@ -354,40 +354,59 @@ __global__ __launch_bounds__(JB) void k_join_materialize(const u64 *inner, const
 constexpr u32 kStage = 256;
 constexpr u64 kHubRun = 32;  // longer inner runs may use the load-balanced variant
 
-// A cursor word counts the new keys (low bits) and, in a linear body, the
-// blocks that are done (from bit kDoneBit on), so that one atomic gives a
-// block its place in the output and tells it whether it is the last.
-constexpr int kDoneBit = 50;
-constexpr u64 kNewMask = (1ull << kDoneBit) - 1;
+// A cursor word counts the new keys in its low bits.  In a linear body it also
+// counts the finished blocks and, with LIN_PACKED, the produced tuples, so that
+// one atomic gives a block its place in the output, hands over its counts and
+// tells it whether it is the last: atomics on one word take 11 ns each, and a
+// body's blocks all end at about the same time.
+enum LinMode {
+    LIN_NONE,    // not a linear body: new keys only
+    LIN_WORDS,   // new keys (50 bits), blocks (14); produced counts in a word per block
+    LIN_PACKED,  // new keys (27 bits), produced tuples (27), blocks (10)
+};
+constexpr u32 kPackedBits = 27, kPackedBlocks = 1023;
+template <int LIN>
+struct LinCursor {
+    static constexpr int kNewBits = LIN == LIN_PACKED ? kPackedBits : 50;
+    static constexpr int kDoneBit = LIN == LIN_PACKED ? 2 * kPackedBits : 50;
+    static constexpr u64 kNewMask = (1ull << kNewBits) - 1;
+};
 
 // Writes stay below out_cap; a cursor past it tells the host the caller's
 // output bound was wrong.
+template <int LIN>
 __device__ __forceinline__ void flush_stage(const u64 *stage, u32 n, u64 *out, u64 out_cap,
                                             unsigned long long *cursor, u64 base, int lane) {
     unsigned long long pos = 0;
-    if (lane == 0) pos = base + (atomicAdd(cursor, (unsigned long long)n) & kNewMask);
+    if (lane == 0)
+        pos = base + (atomicAdd(cursor, (unsigned long long)n) & LinCursor<LIN>::kNewMask);
     pos = __shfl(pos, 0, 64);
     for (u32 x = lane; x < n; x += 64)
         if (pos + x < out_cap) out[pos + x] = stage[x];
 }
 
+// What a linear body's last block learns.
+struct LinCounts {
+    u64 fresh, produced;  // LIN_WORDS: produced is still in the blocks' words
+};
+
 // End of a fused-join block: what the waves still stage goes out with one
-// cursor atomic for the whole block.  The produced count: one more atomic on
-// *produced_to (LIN = false), or a store to the block's own word there
-// (LIN = true, a linear body), which is at the device's coherence point before
-// the cursor says that the block is done: an agent-scope store that has been
-// waited for.  (A fence in its place writes the XCD's whole L2 back, in each of
-// a body's ~190 blocks.)  LIN returns whether this block is the last, and the
-// new keys of all blocks in *total.  Every thread of the block calls it.
-template <int B, bool LIN>
+// cursor atomic for the whole block.  The produced count: with LIN_NONE one
+// more atomic on *produced_to; with LIN_WORDS a store to the block's own word
+// there, which is at the device's coherence point before the cursor says that
+// the block is done (an agent-scope store that has been waited for: a fence in
+// its place writes the XCD's whole L2 back in each of a body's blocks).
+// Returns whether this block is the body's last.  Every thread calls it.
+template <int B, int LIN>
 __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 staged,
                                                   u64 produced, u64 *out, u64 out_cap,
                                                   unsigned long long *cursor, u64 base,
-                                                  unsigned long long *produced_to, u64 *total) {
+                                                  unsigned long long *produced_to,
+                                                  LinCounts *counts) {
+    using C = LinCursor<LIN>;
     __shared__ u32 s_cnt[B / 64];
     __shared__ u64 s_prod[B / 64];
-    __shared__ u64 s_base, s_total;
-    __shared__ bool s_last;
+    __shared__ u64 s_base, s_all;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int d = 32; d >= 1; d >>= 1) produced += __shfl_xor(produced, d, 64);
     if (lane == 0) {
@@ -401,17 +420,21 @@ __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 st
             tot += s_cnt[v];
             prod += s_prod[v];
         }
-        if constexpr (LIN) {
-            __hip_atomic_store(&produced_to[blockIdx.x], (unsigned long long)prod,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            const u64 old = atomicAdd(cursor, (unsigned long long)((1ull << kDoneBit) | tot));
-            s_base = base + (old & kNewMask);
-            s_last = (old >> kDoneBit) == gridDim.x - 1;
-            s_total = (old & kNewMask) + tot;
-        } else {
+        if constexpr (LIN == LIN_NONE) {
             if (prod) atomicAdd(produced_to, (unsigned long long)prod);
             s_base = tot ? base + atomicAdd(cursor, (unsigned long long)tot) : 0;
+        } else {
+            u64 add = (1ull << C::kDoneBit) | tot;
+            if constexpr (LIN == LIN_WORDS) {
+                __hip_atomic_store(&produced_to[blockIdx.x], (unsigned long long)prod,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else {
+                add += prod << kPackedBits;
+            }
+            const u64 old = atomicAdd(cursor, (unsigned long long)add);
+            s_base = base + (old & C::kNewMask);
+            s_all = old + add;
         }
     }
     __syncthreads();
@@ -420,9 +443,11 @@ __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 st
     const u64 *stage = s_stage[w];
     for (u32 x = lane; x < staged; x += 64)
         if (off + x < out_cap) out[off + x] = stage[x];
-    if constexpr (LIN) {
-        *total = s_total;
-        return s_last;
+    if constexpr (LIN != LIN_NONE) {
+        const u64 all = s_all;
+        counts->fresh = all & C::kNewMask;
+        counts->produced = (all >> kPackedBits) & LinCursor<LIN_PACKED>::kNewMask;
+        return (all >> C::kDoneBit) == gridDim.x;
     }
     return false;
 }
@@ -465,16 +490,89 @@ __device__ __forceinline__ void load_segs(const HsSel &h, gdl_hs_seg *s_segs) {
     }
 }
 
+// Inserts the live keys (bit r of `live`: keys[r]) and returns which were new.
+// The home-slot CASes (bitmap: a plain load, since a set bit proves
+// membership, then the ORs) of all of them are in flight together; keys that
+// met another key at home are then probed for one per lane and round, so a
+// wave takes as many probe rounds as its unluckiest lane has collisions, not
+// one for every r that collided somewhere.
+template <int N, bool SEG>
+__device__ __forceinline__ u32 insert_keys(const HsSel &sel, const gdl_hs_seg *s_segs,
+                                           const u64 *keys, u32 live, unsigned long long *outside) {
+    unsigned long long old[N];
+    u32 bm = 0;     // keys that went to a bitmap set (old: the bit before)
+    u32 probe = 0;  // keys that need the full probe
+    u32 fresh = 0;
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        old[r] = 0;
+        if (!((live >> r) & 1u)) continue;
+        const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
+        if (sel.dom_bits && !bm_in_domain(keys[r], sel.dom_bits)) {
+            atomicOr(outside, 1ull);
+            live &= ~(1u << r);
+        } else if (!hs.slots) {
+            live &= ~(1u << r);
+        } else if (hs.mask & kHsBitmap) {
+            const int kb = (int)(hs.mask & 63);
+            if (bm_in_domain(keys[r], kb)) {
+                const u64 b = bm_bit(keys[r], kb);
+                old[r] = ((const u64 *)hs.slots)[b >> 6] & (1ull << (b & 63));
+                bm |= 1u << r;
+            } else {
+                probe |= 1u << r;  // flags the set
+            }
+        } else if (keys[r] != kHsEmpty) {
+            old[r] = atomicCAS((unsigned long long *)((u64 *)hs.slots + (mix64(keys[r]) & hs.mask)),
+                               (unsigned long long)kHsEmpty, (unsigned long long)keys[r]);
+        } else {
+            probe |= 1u << r;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        if (((bm >> r) & 1u) && old[r] == 0) {
+            const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
+            const u64 b = bm_bit(keys[r], (int)(hs.mask & 63));
+            const u64 m = 1ull << (b & 63);
+            old[r] = atomicOr((unsigned long long *)((u64 *)hs.slots + (b >> 6)),
+                              (unsigned long long)m) & m;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        const u32 bit = 1u << r;
+        if (!(live & bit) || (probe & bit)) continue;
+        if (bm & bit) fresh |= old[r] == 0 ? bit : 0u;
+        else if (old[r] == (unsigned long long)kHsEmpty) fresh |= bit;
+        else if (old[r] != (unsigned long long)keys[r]) probe |= bit;
+    }
+    while (probe) {
+        const u32 bit = probe & (0u - probe);
+        u64 k = keys[0];
+#pragma unroll
+        for (int r = 1; r < N; ++r) k = (bit >> r) & 1u ? keys[r] : k;
+        const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, k);
+        const bool is_new =
+            (hs.mask & kHsBitmap) || k == kHsEmpty
+                ? hs_insert_key((u64 *)hs.slots, hs.mask, k)
+                : hs_probe_from((u64 *)hs.slots, hs.mask, k, (mix64(k) + 1) & hs.mask);
+        if (is_new) fresh |= bit;
+        probe &= ~bit;
+    }
+    return fresh;
+}
+
 // One block's share of a fused join + insert (the blocks of the grid stride
 // over the outer tuples): new keys go to out from base + *cursor on.  LIN,
-// produced_to, total and the result as in block_final_flush; counters[2] flags
-// a key outside the id bound.
-template <int B, bool SEG, bool LIN>
+// produced_to, counts and the result as in block_final_flush; *outside flags a
+// key outside the id bound.
+template <int B, bool SEG, int LIN>
 __device__ __forceinline__ bool join_insert_blocks(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
     u64 out_cap, unsigned long long *cursor, u64 out_base, unsigned long long *produced_to,
-    unsigned long long *outside, u64 *total_new) {
+    unsigned long long *outside, LinCounts *counts) {
     __shared__ u64 s_excl[B], s_b[B], s_ok[B];
     __shared__ u64 s_stage[B / 64][kStage];
     __shared__ gdl_hs_seg s_segs[SEG ? kMaxSegs : 1];
@@ -499,10 +597,12 @@ __device__ __forceinline__ bool join_insert_blocks(
         s_b[threadIdx.x] = b;
         s_ok[threadIdx.x] = ok;
         wave_sync_lds();
+        // (two rounds together, to overlap their chains, were slower: 23.8
+        // against 18.0 us for a body of the 200k-node tree)
         for (u64 q = 0; q < total; q += 64) {
             const u64 t = q + lane;
-            bool fresh = false;
             u64 key = 0;
+            u32 live = 0;
             if (t < total) {
                 // the last lane whose run starts at or before t owns position t
                 int lo = 0, hi = 63;
@@ -513,20 +613,15 @@ __device__ __forceinline__ bool join_insert_blocks(
                 }
                 const u64 j = t - wx[lo];
                 key = apply_map(inner[s_b[w * 64 + lo] + j], s_ok[w * 64 + lo], arity, s0, s1);
-                if (eval_pred(key, pop, plhs, prhs)) {
-                    ++produced;
-                    const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, key);
-                    if (sel.dom_bits && !bm_in_domain(key, sel.dom_bits))
-                        atomicOr(outside, 1ull);
-                    else if (hs.slots)
-                        fresh = hs_insert_key((u64 *)hs.slots, hs.mask, key);
-                }
+                live = eval_pred(key, pop, plhs, prhs);
             }
+            produced += live;
+            const bool fresh = insert_keys<1, SEG>(sel, s_segs, &key, live, outside);
             const u64 bal = __ballot(fresh);
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage(stage, staged, out, out_cap, cursor, out_base, lane);
+                flush_stage<LIN>(stage, staged, out, out_cap, cursor, out_base, lane);
                 staged = 0;
                 wave_sync_lds();
             }
@@ -536,7 +631,7 @@ __device__ __forceinline__ bool join_insert_blocks(
         wave_sync_lds();  // s_excl / s_b / s_ok are rewritten next round
     }
     return block_final_flush<B, LIN>(s_stage, staged, produced, out, out_cap, cursor, out_base,
-                                     produced_to, total_new);
+                                     produced_to, counts);
 }
 
 template <int B, bool SEG>
@@ -544,16 +639,15 @@ __global__ __launch_bounds__(B) void k_join_insert(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
     u64 out_cap, unsigned long long *counters) {
-    u64 unused;
-    join_insert_blocks<B, SEG, false>(slots, n_slots, inner, n_inner, shift, outer, n_outer, arity,
-                                      s0, s1, pop, plhs, prhs, sel, out, out_cap, &counters[0], 0,
-                                      &counters[1], &counters[2], &unused);
+    join_insert_blocks<B, SEG, LIN_NONE>(slots, n_slots, inner, n_inner, shift, outer, n_outer,
+                                         arity, s0, s1, pop, plhs, prhs, sel, out, out_cap,
+                                         &counters[0], 0, &counters[1], &counters[2], nullptr);
 }
 
 // State of a stream-ordered linear fixpoint (gdl_fixpoint_linear) in device
 // memory.
 struct LinState {
-    unsigned long long cursor;    // the running body's new keys and finished blocks (kDoneBit)
+    unsigned long long cursor;    // the running body's counts (LinCursor)
     u64 delta_begin, delta_end;   // the body's delta: log[delta_begin, delta_end)
     u64 size;                     // hash set members
     u64 hs_limit;                 // members the set may reach (a fraction of its capacity)
@@ -594,8 +688,8 @@ __device__ void linear_epilogue(LinState *st, u64 *counts, u64 d1, u64 nd, u64 p
 // One body of out := out U map(inner x delta) with FULL = hash set + append
 // log: the delta is the log's last segment, new tuples are appended after it.
 // A stop code set by an earlier body makes it return at once.  produced: a
-// word per block.
-template <int B>
+// word per block (LIN_WORDS).
+template <int B, int LIN>
 __global__ __launch_bounds__(B) void k_linear_body(const IdxSlot *slots, u64 n_slots,
                                                    const u64 *inner, u64 n_inner, int shift,
                                                    int arity, int s0, int s1, int pop, int plhs,
@@ -605,24 +699,24 @@ __global__ __launch_bounds__(B) void k_linear_body(const IdxSlot *slots, u64 n_s
     __shared__ u64 s_sum[B / 64];
     if (st->stop != kLinRun) return;  // the same for every block
     const u64 d0 = st->delta_begin, d1 = st->delta_end;
-    u64 nd;
-    if (!join_insert_blocks<B, false, true>(
+    LinCounts c;
+    if (!join_insert_blocks<B, false, LIN>(
             slots, n_slots, inner, n_inner, shift, log + d0, d1 - d0, arity, s0, s1, pop, plhs,
             prhs, HsSel{hs_slots, hs_mask, nullptr, 0, 0, 0}, log, st->log_cap, &st->cursor, d1,
-            produced, nullptr, &nd))
+            produced, nullptr, &c))
         return;
-    // the last block: every other one's count is at the coherence point
-    u64 sum = 0;
-    for (u32 i = threadIdx.x; i < gridDim.x; i += B)
-        sum += __hip_atomic_load(&produced[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
-    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        sum = 0;
-        for (int v = 0; v < B / 64; ++v) sum += s_sum[v];
-        linear_epilogue(st, counts, d1, nd, sum);
+    // the last block: every other one's counts are at the coherence point
+    if constexpr (LIN == LIN_WORDS) {
+        u64 sum = 0;
+        for (u32 i = threadIdx.x; i < gridDim.x; i += B)
+            sum += __hip_atomic_load(&produced[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+        if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
+        __syncthreads();
+        c.produced = 0;
+        for (int v = 0; v < B / 64; ++v) c.produced += s_sum[v];
     }
+    if (threadIdx.x == 0) linear_epilogue(st, counts, d1, c.fresh, c.produced);
 }
 
 // Load-balanced variant for inner relations with long runs: outputs are
@@ -666,77 +760,24 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
         }
         __syncthreads();  // the next tile overwrites the owners
         produced += __popc(live);
-        // home-slot CAS (bitmap: the OR of the key's bit) of every key first,
-        // independent round trips in flight
-        unsigned long long old[JM_I];
-        u32 bm = 0;  // bit r: key r went to a bitmap set (old[r]: its bit before)
+        const u32 fresh = insert_keys<JM_I, SEG>(sel, s_segs, keys, live, &counters[2]);
 #pragma unroll
         for (int r = 0; r < JM_I; ++r) {
-            old[r] = 0;
-            if ((live >> r) & 1u) {
-                const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
-                if (sel.dom_bits && !bm_in_domain(keys[r], sel.dom_bits)) {
-                    atomicOr(&counters[2], 1ull);
-                    live &= ~(1u << r);
-                } else if (!hs.slots) {
-                    live &= ~(1u << r);
-                } else if (hs.mask & kHsBitmap) {
-                    const int kb = (int)(hs.mask & 63);
-                    if (bm_in_domain(keys[r], kb)) {
-                        // a plain load first: a set bit proves membership
-                        const u64 b = bm_bit(keys[r], kb);
-                        old[r] = ((const u64 *)hs.slots)[b >> 6] & (1ull << (b & 63));
-                        bm |= 1u << r;
-                    }
-                } else if (keys[r] != kHsEmpty) {
-                    old[r] = atomicCAS(
-                        (unsigned long long *)((u64 *)hs.slots + (mix64(keys[r]) & hs.mask)),
-                        (unsigned long long)kHsEmpty, (unsigned long long)keys[r]);
-                }
-            }
-        }
-        // bitmap keys whose bit read clear: the atomic OR decides, all in flight
-#pragma unroll
-        for (int r = 0; r < JM_I; ++r) {
-            if (((bm >> r) & 1u) && old[r] == 0) {
-                const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
-                const u64 b = bm_bit(keys[r], (int)(hs.mask & 63));
-                const u64 m = 1ull << (b & 63);
-                old[r] = atomicOr((unsigned long long *)((u64 *)hs.slots + (b >> 6)),
-                                  (unsigned long long)m) & m;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < JM_I; ++r) {
-            bool fresh = false;
-            if ((bm >> r) & 1u) {
-                fresh = old[r] == 0;
-            } else if ((live >> r) & 1u) {
-                if (keys[r] == kHsEmpty || (old[r] != (unsigned long long)kHsEmpty &&
-                                            old[r] != (unsigned long long)keys[r]) ||
-                    (sel_set<SEG>(sel, s_segs, keys[r]).mask & kHsBitmap)) {
-                    // collision (or the key ~0): the full probe
-                    const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
-                    fresh = hs_insert_key((u64 *)hs.slots, hs.mask, keys[r]);
-                } else {
-                    fresh = old[r] == (unsigned long long)kHsEmpty;
-                }
-            }
-            const u64 bal = __ballot(fresh);
+            const bool f = (fresh >> r) & 1u;
+            const u64 bal = __ballot(f);
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage(stage, staged, out, out_cap, &counters[0], 0, lane);
+                flush_stage<LIN_NONE>(stage, staged, out, out_cap, &counters[0], 0, lane);
                 staged = 0;
                 wave_sync_lds();
             }
-            if (fresh) stage[staged + __popcll(bal & lt)] = keys[r];
+            if (f) stage[staged + __popcll(bal & lt)] = keys[r];
             staged += cnt;
         }
     }
-    u64 unused;
-    block_final_flush<JB, false>(s_stage, staged, produced, out, out_cap, &counters[0], 0,
-                                 &counters[1], &unused);
+    block_final_flush<JB, LIN_NONE>(s_stage, staged, produced, out, out_cap, &counters[0], 0,
+                                    &counters[1], nullptr);
 }
 
 __global__ void k_set2(u64 *p, u64 a, u64 b) {
@@ -1234,11 +1275,14 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
     // 2.5 %; 64 did not; a chunk that stops early leaves no-op launches)
     constexpr int kChunk = 128;
     // a body is bound by the latency of each tuple's chain of dependent
-    // accesses, so every outer tuple gets its own lane (more chains in
-    // flight) in blocks of 512 (fewer blocks: fewer barriers and end-of-block
-    // counter atomics on the shared state); on the 200k-node tree both beat
-    // 256-thread blocks with two tuples per thread
-    constexpr int LB = 512;
+    // accesses (~0.6 us a load) and by the set's atomics (25e9 a second at
+    // random places, whatever their scope: 8 of the 21 us of a body of 190k
+    // outer tuples; its key 5, the end of its blocks 1.4, its launch 4), so every outer tuple gets its own
+    // lane (more chains in flight).  Blocks of 512 (each ends with an atomic on
+    // the shared cursor, 11 ns one after another, but also waits for its
+    // slowest wave): 17.1 us a body on the 200k-node tree, 18.0 with 256 and
+    // 18.4 with 1024; of 256 up to 2^16 outer tuples (50,000 nodes: 9.4
+    // against 10.3 us)
     const int shift = inner_idx->prefix_cols >= 2 ? 0 : 32;
     const u64 mr = std::max<u64>(inner_idx->max_run, 1);
     Scratch scr(ctx);
@@ -1283,12 +1327,21 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         const u64 next = std::max<u64>(nd, 1024) * (u64)std::min(ramp, kChunk);
         GDL_TRY(hashset_reserve2(ctx, hs, next, std::max(worst, next), 0.0,
                                  std::max<u64>(next, 4 * hs->size)));
-        u64 need_log = d1 + std::max<u64>(worst, 4096);
+        // (and, up to twice the log, the rest of the chunk at this delta's
+        // size: a chunk that stops for a full log leaves its remaining launches
+        // to return at once)
+        const int k = std::min({ramp, kChunk, max_bodies - done});
+        const u64 least_log = std::max<u64>(d1 + std::max<u64>(worst, 4096), 2 * *log_cap);
+        u64 need_log = d1 + std::max<u64>(worst, 4096) + std::min<u64>(nd * (u64)(k - 1), d1);
         if (*log_cap < need_log) {
             need_log = std::max<u64>(need_log, 2 * *log_cap);  // geometric
             void *p = nullptr;
             std::string err;
             gdl_status s = ctx->alloc->alloc(need_log * sizeof(u64), &p, &err);
+            if (s == GDL_ERR_OUT_OF_MEMORY && least_log < need_log) {
+                need_log = least_log;
+                s = ctx->alloc->alloc(need_log * sizeof(u64), &p, &err);
+            }
             if (s != GDL_OK) return fail(ctx, s, err);
             if (d1)
                 GDL_HIP(ctx, hipMemcpyAsync(p, *d_log, d1 * sizeof(u64), hipMemcpyDeviceToDevice,
@@ -1297,7 +1350,6 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
             *d_log = (u64 *)p;
             *log_cap = need_log;
         }
-        const int k = std::min({ramp, kChunk, max_bodies - done});
         LinState h{};
         h.cursor = 0;
         h.delta_begin = d0;
@@ -1310,21 +1362,32 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         // a grid for this delta (one outer tuple per thread); a body whose
         // delta outgrows it 8x ends the chunk, so the next chunk is launched
         // wider
+        // the counts of a body packed in one word while they fit it: produced
+        // tuples (and so new ones) below 2^27, at most 1023 blocks
+        const u64 packed_limit = ((1ull << kPackedBits) - 1) / mr;
+        const u64 LB = nd <= std::min<u64>(1u << 16, packed_limit) ? 256 : 512;
         const u64 want = (nd + LB - 1) / LB;
         const unsigned g = (unsigned)std::min<u64>(grid_cap(ctx), std::max<u64>(want, 16));
         h.delta_limit = g >= grid_cap(ctx) ? ~0ull : (u64)g * LB * 8;
         // a delta that turns dense ends the chunk too (bit-matrix bodies next)
         if (dense_at != ~0ull) h.delta_limit = std::min<u64>(h.delta_limit, dense_at - 1);
+        const bool packed = g <= kPackedBlocks && nd <= packed_limit;
+        if (packed) h.delta_limit = std::min<u64>(h.delta_limit, packed_limit);
         Staging stg(ctx);
         GDL_TRY(stg.up(st, &h, sizeof(h)));
-        for (int i = 0; i < k; ++i) {
-            KTimer kt(ctx, K_LINEAR, 0.0);
-            hipLaunchKernelGGL(k_linear_body<LB>, dim3(g), dim3(LB), 0, ctx->stream,
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(g), dim3((unsigned)LB), 0, ctx->stream,
                                (const IdxSlot *)inner_idx->slots, idx_arg(inner_idx), d_inner,
                                n_inner, shift, map.arity, map.src[0],
                                map.arity == 2 ? map.src[1] : 0, pred.op, pred.lhs, pred.rhs,
                                (u64 *)hs->slots, hs_arg(hs), *d_log, st,
                                (unsigned long long *)produced, counts);
+        };
+        for (int i = 0; i < k; ++i) {
+            KTimer kt(ctx, K_LINEAR, 0.0);
+            if (!packed) launch(k_linear_body<512, LIN_WORDS>);
+            else if (LB == 512) launch(k_linear_body<512, LIN_PACKED>);
+            else launch(k_linear_body<256, LIN_PACKED>);
             GDL_TRY(check_launch(ctx, "k_linear_body"));
         }
         LinState r{};

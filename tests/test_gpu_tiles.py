@@ -158,3 +158,20 @@ def test_sort_at_tile_edges(ctx, n, kind):
                 "high_only": gdl.pack(rng.integers(0, 1 << 31, n), np.zeros(n))}[kind]
     assert np.array_equal(ctx.sort(keys, bits, bits), np.sort(keys))
     assert np.array_equal(ctx.sort_unique(keys, -1, -1), np.unique(keys))
+
+
+# a linear body's blocks hand over their counts packed in one word up to 2^27
+# produced tuples and 1023 blocks of 1024 outer tuples, in words of their own
+# above; the ids need a hash set
+@pytest.mark.parametrize("paths", [1, 1023, 1025, 400_000, 1_200_000])
+def test_linear_bodies_of_disjoint_paths(ctx, paths):
+    # node j of path i is i + j * paths + 2^19: three edges a path, in any order
+    i = np.arange(paths, dtype=np.uint64) + np.uint64(1 << 19)
+    node = [i + np.uint64(j * paths) for j in range(4)]
+    edges = np.concatenate([gdl.pack(node[j], node[j + 1]) for j in (1, 0, 2)])
+    got = ctx.run_tc(edges, out_cap=8 * paths)
+    want = np.sort(np.concatenate([gdl.pack(node[a], node[b])
+                                   for a in range(4) for b in range(a + 1, 4)]))
+    assert np.array_equal(got["out"], want)
+    assert [t[3] for t in got["trace"]] == [2 * paths, paths, 0]
+    assert [t[2] for t in got["trace"]] == [2 * paths, paths, 0]
