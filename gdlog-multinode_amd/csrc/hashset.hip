@@ -128,31 +128,57 @@ __global__ __launch_bounds__(HB) void k_hs_rehash(const u64 *old_slots, u64 old_
 }
 
 // Compacts the members of a table (the slots of cap words plus the ~0 flag
-// word after them) into out, one atomic per wave.
+// word after them) into out.  A block takes kXtPer * HB consecutive slots a
+// round and reserves their output with one atomic: one atomic per wave, all on
+// one address at 11 ns each, took 192 us for the 2^20 slots of a batch's set.
+constexpr int kXtPer = 16;
 __global__ __launch_bounds__(HB) void k_hs_extract(const u64 *slots, u64 cap, u64 *out,
                                                    u64 out_cap, unsigned long long *counter) {
-    const u64 lt = lane_mask_lt();
-    for (u64 base = (u64)blockIdx.x * HB; base <= cap; base += (u64)gridDim.x * HB) {
-        const u64 i = base + threadIdx.x;
-        bool keep = false;
-        u64 k = 0;
-        if (i < cap) {
-            k = slots[i];
-            keep = k != kEmpty;
-        } else if (i == cap) {
-            k = kEmpty;
-            keep = slots[cap] != 0ull;
+    __shared__ u32 s_cnt[HB / 64];
+    __shared__ unsigned long long s_base;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const u64 lt = lane_mask_lt(), per_round = (u64)HB * kXtPer;
+    // every thread of a block runs the same rounds (barriers below)
+    for (u64 base = (u64)blockIdx.x * per_round; base <= cap; base += (u64)gridDim.x * per_round) {
+        u64 k[kXtPer];
+        u32 keep = 0, c = 0;
+#pragma unroll
+        for (int j = 0; j < kXtPer; ++j) {
+            const u64 i = base + (u64)j * HB + threadIdx.x;
+            k[j] = i <= cap ? slots[i] : kEmpty;
         }
-        const u64 bal = __ballot(keep);
-        if (bal) {
-            unsigned long long pos = 0;
-            const int leader = __ffsll((unsigned long long)bal) - 1;
-            if ((int)(threadIdx.x & 63) == leader)
-                pos = atomicAdd(counter, (unsigned long long)__popcll(bal));
-            pos = __shfl(pos, leader, 64);
-            const u64 at = pos + __popcll(bal & lt);
-            if (keep && at < out_cap) out[at] = k;
+#pragma unroll
+        for (int j = 0; j < kXtPer; ++j) {
+            const u64 i = base + (u64)j * HB + threadIdx.x;
+            bool f = i < cap && k[j] != kEmpty;
+            if (i == cap) {  // the flag word: the key ~0 is a member
+                f = k[j] != 0;
+                k[j] = kEmpty;
+            }
+            keep |= (u32)f << j;
+            c += (u32)__popcll(__ballot(f));
         }
+        if (lane == 0) s_cnt[wv] = c;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            u32 t = 0;
+            for (int w = 0; w < HB / 64; ++w) {
+                const u32 x = s_cnt[w];
+                s_cnt[w] = t;
+                t += x;
+            }
+            s_base = t ? atomicAdd(counter, (unsigned long long)t) : 0ull;
+        }
+        __syncthreads();
+        u64 pos = s_base + s_cnt[wv];
+#pragma unroll
+        for (int j = 0; j < kXtPer; ++j) {
+            const bool f = (keep >> j) & 1u;
+            const u64 bal = __ballot(f), at = pos + __popcll(bal & lt);
+            if (f && at < out_cap) out[at] = k[j];
+            pos += (u64)__popcll(bal);
+        }
+        __syncthreads();  // s_cnt and s_base are rewritten next round
     }
 }
 
@@ -390,7 +416,7 @@ gdl_status gdl_hashset_extract(gdl_ctx *ctx, const gdl_hashset *hs, uint64_t *d_
         GDL_TRY(check_launch(ctx, "k_bm_extract"));
     } else {
         KTimer kt(ctx, K_HS_EXTRACT, 8.0 * hs->capacity + 8.0 * hs->size);
-        hipLaunchKernelGGL(k_hs_extract, dim3(hs_grid(ctx, hs->capacity + 1)), dim3(HB), 0,
+        hipLaunchKernelGGL(k_hs_extract, dim3(hs_grid(ctx, hs->capacity / kXtPer + 1)), dim3(HB), 0,
                            ctx->stream, (const u64 *)hs->slots, hs->capacity, d_out, out_cap,
                            (unsigned long long *)counter);
         GDL_TRY(check_launch(ctx, "k_hs_extract"));
