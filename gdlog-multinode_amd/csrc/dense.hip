@@ -69,16 +69,24 @@ __device__ __forceinline__ int select_bit(u64 w, int j) {
 // column with kb-bit columns) to out[base ..), in bit order.  Each lane puts
 // the round-local numbers of its bits in the wave's LDS list (buf, 4096
 // entries) from its exclusive count on; the wave then stores the keys with
-// consecutive lanes on consecutive positions.  Returns the round's total
-// (the same in every lane).
+// consecutive lanes on consecutive positions, past the caches with NT (nothing
+// reads them soon).  Returns the round's total (the same in every lane).
+// (Words of more than 8 bits put in the list by the whole wave, a bit per
+// lane: 0.40 against 0.32 ms for 68M keys of 2^30 bits.)
+template <bool NT>
 __device__ __forceinline__ u64 stage_write(u64 wd, u64 bitbase, int kb, u64 *out, u64 base,
                                            u64 out_cap, uint16_t *buf) {
     const int lane = threadIdx.x & 63;
-    const u64 c = (u64)__popcll(wd);
-    const u64 incl = wave_inclusive_scan(c);
-    const u64 total = __shfl(incl, 63, 64);
+    const u32 c = (u32)__popcll(wd);
+    u32 incl = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const u32 v = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += v;
+    }
+    const u32 total = __builtin_amdgcn_readlane(incl, 63);
     if (total == 0) return 0;
-    u32 at = (u32)(incl - c);
+    u32 at = incl - c;
     const u32 l64 = (u32)lane << 6;
     while (wd) {
         buf[at++] = (uint16_t)(l64 | (u32)(__ffsll((unsigned long long)wd) - 1));
@@ -86,9 +94,13 @@ __device__ __forceinline__ u64 stage_write(u64 wd, u64 bitbase, int kb, u64 *out
     }
     wave_sync_lds();
     const u64 lo_mask = (1ull << kb) - 1;
-    for (u64 t = lane; t < total; t += 64) {
+    for (u32 t = lane; t < total; t += 64) {
         const u64 bit = bitbase + buf[t];
-        if (base + t < out_cap) out[base + t] = ((bit >> kb) << 32) | (bit & lo_mask);
+        const u64 key = ((bit >> kb) << 32) | (bit & lo_mask);
+        if (base + t < out_cap) {
+            if constexpr (NT) __builtin_nontemporal_store(key, &out[base + t]);
+            else out[base + t] = key;
+        }
     }
     wave_sync_lds();  // the list is rewritten by the next round
     return total;
@@ -122,7 +134,7 @@ __device__ __forceinline__ u64 xt_word(const u64 *words, const u64 *minus, const
 template <int R>
 __global__ __launch_bounds__(DB) void k_xt_count(const u64 *words, u64 n_words, u64 n_tiles,
                                                  const u64 *minus, const u32 *minus_pop, int rs,
-                                                 u64 *tile_counts) {
+                                                 u32 *tile_counts) {
     const u64 tile = (u64)blockIdx.x * DWV + (threadIdx.x >> 6);
     if (tile >= n_tiles) return;  // the same for the whole wave
     const int lane = threadIdx.x & 63;
@@ -137,7 +149,7 @@ __global__ __launch_bounds__(DB) void k_xt_count(const u64 *words, u64 n_words, 
 #pragma unroll
     for (int r = 0; r < R; ++r) c += (u64)__popcll(w[r]);
     c = wave_sum(c);
-    if (lane == 0) tile_counts[tile] = c;
+    if (lane == 0) tile_counts[tile] = (u32)c;
 }
 
 template <int R>
@@ -159,13 +171,13 @@ __global__ __launch_bounds__(DB) void k_xt_write(const u64 *words, u64 n_words, 
     u64 base = tile_offsets[tile];
 #pragma unroll
     for (int r = 0; r < R; ++r)
-        base += stage_write(w[r], (t0 + (u64)r * 64) * 64, kb, out, base, out_cap,
+        base += stage_write<true>(w[r], (t0 + (u64)r * 64) * 64, kb, out, base, out_cap,
                             s_buf[threadIdx.x >> 6]);
 }
 
 // Pass 1 and pass 2 of the extraction over `tiles` tiles of 64 * rounds words.
 static gdl_status launch_xt_count(gdl_ctx *ctx, int rounds, const u64 *words, u64 nw, u64 tiles,
-                                  const u64 *minus, const u32 *minus_pop, int rs, u64 *tc) {
+                                  const u64 *minus, const u32 *minus_pop, int rs, u32 *tc) {
     const unsigned blocks = (unsigned)((tiles + DWV - 1) / DWV);
 #define GDL_XT_COUNT(R)                                                                        \
     hipLaunchKernelGGL(k_xt_count<R>, dim3(blocks), dim3(DB), 0, ctx->stream, words, nw, tiles, \
@@ -211,15 +223,16 @@ static gdl_status bitmap_extract_sorted(gdl_ctx *ctx, const u64 *words, int kb, 
     const u64 tiles = (nw + 64ull * rounds - 1) / (64ull * rounds);
     const int rs = kb >= 6 ? kb - 6 : 0;
     Scratch scr(ctx);
+    u32 *counts;
     u64 *tc;
+    GDL_TRY(scr.get(tiles, &counts));
     GDL_TRY(scr.get(tiles + 1, &tc));
     {
         KTimer kt(ctx, K_BM_EXTRACT, 8.0 * nw);
-        GDL_TRY(launch_xt_count(ctx, rounds, words, nw, tiles, minus, minus_pop, rs, tc));
+        GDL_TRY(launch_xt_count(ctx, rounds, words, nw, tiles, minus, minus_pop, rs, counts));
     }
-    GDL_TRY(scan_inplace(ctx, tc, tiles));
     u64 total = 0;
-    GDL_TRY(read_u64(ctx, tc + tiles, &total));
+    GDL_TRY(exclusive_scan_u32_to_u64(ctx, counts, tiles, tc, &total));
     *n_out = total;
     if (total > out_cap)
         return fail(ctx, GDL_ERR_OVERFLOW, "bitmap extract: " + std::to_string(total) +
@@ -233,23 +246,39 @@ static gdl_status bitmap_extract_sorted(gdl_ctx *ctx, const u64 *words, int kb, 
 // ---------------------------------------------------------------------------
 // Bodies on bit matrices.
 
-// Device state of a run of dense bodies.  The counters come first.
+// The counters of the running body, one set per group of blocks (blockIdx mod
+// kGroups), each on a line of its own: atomics on one line take 11 ns one after
+// another, and with a single set the counters of a body's 2048 combine, 2048
+// row-OR and 4096 transpose blocks took 50-110 us of its time.
+constexpr u32 kGroups = 32;
+enum DenseCounter {
+    DC_NEW,       // new tuples
+    DC_RAW,       // produced tuples
+    DC_ROWS_IO,   // the combine's row reads + writes
+    DC_ROWS_NEW,  // rows that got new tuples
+    DC_COMBINE,   // (the combine's counters end here)
+    DC_EXP_IO = DC_COMBINE,  // SG: the expansion's row reads + writes
+    DC_TR_IO,     // column expansion: 64-byte segments the transposes moved
+    DC_OR_IO,     // and the row reads + writes of its row OR
+    DC_NUM
+};
+struct alignas(128) DenseGroup {
+    unsigned long long c[DC_NUM];
+    u32 done;         // the group's combine blocks that finished
+    u32 append_done;  // and its append blocks
+};
+
+// Device state of a run of dense bodies.
 struct DenseState {
+    DenseGroup group[kGroups];
     unsigned long long cursor;   // log end
-    unsigned long long n_new;    // the running body's new tuples
-    unsigned long long raw;      // its produced tuples
-    unsigned long long rows_io;   // the combine's row reads + writes of the running body
-    unsigned long long exp_io;    // the expansion's row reads + writes
-    unsigned long long rows_new;  // rows that got new tuples
-    unsigned long long tr_io;     // SG column expansion: 64-byte segments the transposes moved
-    unsigned long long or_io;     // and the row reads + writes of its row OR
     u64 col_above;     // SG: a body whose delta has at least this many tuples expands by columns
     u64 log_cap;
     u64 sparse_below;  // a body with fewer new tuples ends the run
     u64 append_base;   // the log end before the last body's append
-    u32 stop, body, blocks_done, max_bodies;
+    u32 stop, body, groups_done, max_bodies;
     u32 appended;       // bodies whose new tuples are in the log
-    u32 append_blocks;  // blocks of the running append that finished
+    u32 append_groups;  // groups of the running append that finished
     u32 bad;            // a delta key outside the domain
     u32 col;            // SG: the running body expands by columns
     u32 asym;           // set-up: FULL or the first delta differs from its transpose
@@ -257,9 +286,7 @@ struct DenseState {
     u32 d0_loose;       // set-up: its keys are not strictly increasing
 };
 enum : u32 { kDnRun = 0, kDnFixpoint = 1, kDnGrow = 2, kDnLimit = 3, kDnSparse = 4 };
-// per body: new tuples, produced tuples, combine rows, expansion rows, rows
-// with new tuples, column expansion: transposed segments, OR rows
-constexpr int kCounts = 7;
+constexpr int kCounts = DC_NUM;  // per body
 
 // The rule's static relations as row lists.  pred: r1 grouped by its second
 // column (for row x, the y with r1(y, x)); act: the rows with a non-empty
@@ -299,34 +326,46 @@ struct DenseArgs {
     u64 *log;
 };
 
-// End of a body (thread 0 of the last block): record its counts and decide
-// whether the next enqueued body runs.
-__device__ void dense_epilogue(DenseState *st, u64 *counts) {
-    const u64 nn = atomicAdd(&st->n_new, 0ull);
-    const u64 raw = atomicAdd(&st->raw, 0ull);
-    const u64 io = atomicAdd(&st->rows_io, 0ull);
-    const u64 eio = atomicAdd(&st->exp_io, 0ull);
-    const u64 rn = atomicAdd(&st->rows_new, 0ull);
-    const u64 tio = atomicAdd(&st->tr_io, 0ull);
-    const u64 oio = atomicAdd(&st->or_io, 0ull);
+// Every memory operation of this thread before it is done (an atomic: at the
+// device's coherence point) before any after it starts.  What follows reads
+// with agent-scope loads, so no cache has to be written back or invalidated,
+// as a fence would do (the XCD's whole L2, once per block or slice).
+__device__ __forceinline__ void order_memory() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+__device__ __forceinline__ void group_add(DenseState *st, DenseCounter c, u64 v) {
+    if (v)
+        atomicAdd(&st->group[blockIdx.x % kGroups].c[c], (unsigned long long)v);
+}
+
+// Counts this block as finished in its group and the group, when it is its
+// last block, among the groups (one thread of each block); true for the last
+// block of all.  *mine is back at 0 after the last block of its group.  A grid
+// of up to kOneGroup blocks is one group: one atomic less in a row.
+constexpr u32 kOneGroup = 64;
+__device__ __forceinline__ bool last_of_groups(DenseState *st, u32 DenseGroup::*done,
+                                               u32 *groups) {
+    order_memory();
+    const bool one = gridDim.x <= kOneGroup;
+    const u32 r = one ? 0 : blockIdx.x % kGroups;
+    const u32 members = one ? gridDim.x : (gridDim.x - r + kGroups - 1) / kGroups;
+    u32 *mine = &(st->group[r].*done);
+    if (atomicAdd(mine, 1u) != members - 1) return false;
+    atomicExch(mine, 0u);
+    return one || atomicAdd(groups, 1u) == kGroups - 1;
+}
+
+// End of a body: record its counts v and decide whether the next enqueued
+// body runs (one thread).
+__device__ void dense_epilogue(DenseState *st, u64 *counts, const u64 *v) {
     const u32 b = st->body;
     u64 *c = counts + kCounts * b;
-    c[0] = nn;
-    c[1] = raw;
-    c[2] = io;
-    c[3] = eio;
-    c[4] = rn;
-    c[5] = tio;
-    c[6] = oio;
-    st->n_new = 0;
-    st->raw = 0;
-    st->rows_io = 0;
-    st->exp_io = 0;
-    st->rows_new = 0;
-    st->tr_io = 0;
-    st->or_io = 0;
+#pragma unroll
+    for (int j = 0; j < DC_NUM; ++j) c[j] = v[j];
+    const u64 nn = v[DC_NEW];
     st->col = nn >= st->col_above ? 1u : 0u;  // how the next body expands
-    st->blocks_done = 0;
+    st->groups_done = 0;
     st->append_base = st->cursor;
     u32 stop = kDnRun;
     if (nn == 0) stop = kDnFixpoint;
@@ -336,35 +375,54 @@ __device__ void dense_epilogue(DenseState *st, u64 *counts) {
     st->body = b + 1;  // last: the append launched next reads it
 }
 
-// Block totals -> state; the last block runs the epilogue.
+// Block totals -> the group's counters; the last block runs the epilogue, over
+// the first group's combine counters alone when there is one group (the
+// expansions' counters are SG's, and in all groups).
+template <bool SG>
 __device__ __forceinline__ void dense_block_end(DenseState *st, u64 *counts, u64 nn, u64 raw,
                                                 u64 io, u64 rn) {
-    __shared__ u64 s_v[DWV][4];
+    __shared__ u64 s_v[DWV][DC_COMBINE];
+    __shared__ u64 s_sum[DC_NUM];
     __shared__ bool s_last;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool one = gridDim.x <= kOneGroup;
     if (lane == 0) {
-        s_v[wv][0] = nn;
-        s_v[wv][1] = raw;
-        s_v[wv][2] = io;
-        s_v[wv][3] = rn;
+        s_v[wv][DC_NEW] = nn;
+        s_v[wv][DC_RAW] = raw;
+        s_v[wv][DC_ROWS_IO] = io;
+        s_v[wv][DC_ROWS_NEW] = rn;
     }
+    if (threadIdx.x < DC_NUM) s_sum[threadIdx.x] = 0;
     __syncthreads();
     if (threadIdx.x == 0) {
-        u64 t[4] = {0, 0, 0, 0};
-        for (int v = 0; v < DWV; ++v)
-            for (int j = 0; j < 4; ++j) t[j] += s_v[v][j];
-        if (t[0]) atomicAdd(&st->n_new, (unsigned long long)t[0]);
-        if (t[1]) atomicAdd(&st->raw, (unsigned long long)t[1]);
-        if (t[2]) atomicAdd(&st->rows_io, (unsigned long long)t[2]);
-        if (t[3]) atomicAdd(&st->rows_new, (unsigned long long)t[3]);
-        __threadfence();  // release the counter updates before counting this block finished
-        s_last = atomicAdd(&st->blocks_done, 1u) == gridDim.x - 1;
+        unsigned long long *c = st->group[one ? 0 : blockIdx.x % kGroups].c;
+#pragma unroll
+        for (int j = 0; j < DC_COMBINE; ++j) {
+            u64 t = 0;
+            for (int v = 0; v < DWV; ++v) t += s_v[v][j];
+            if (t) atomicAdd(&c[j], (unsigned long long)t);
+        }
+        s_last = last_of_groups(st, &DenseGroup::done, &st->groups_done);
     }
     __syncthreads();
-    if (s_last && threadIdx.x == 0) {
-        __threadfence();  // acquire: every block's updates precede its blocks_done add
-        dense_epilogue(st, counts);
+    if (!s_last) return;
+    auto take = [&](int g, int j) {  // a counter's value; 0 is left there
+        unsigned long long *p = &st->group[g].c[j];
+        const u64 v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return v;
+    };
+    if (!SG && one) {
+        if (threadIdx.x < DC_COMBINE) s_sum[threadIdx.x] = take(0, threadIdx.x);
+    } else if (threadIdx.x < kGroups * 4) {
+        // thread t: group t / 4, counters t % 4 and t % 4 + 4
+        for (int j = threadIdx.x & 3; j < (SG ? DC_NUM : DC_COMBINE); j += 4) {
+            const u64 v = take(threadIdx.x >> 2, j);
+            if (v) atomicAdd((unsigned long long *)&s_sum[j], (unsigned long long)v);
+        }
     }
+    __syncthreads();
+    if (threadIdx.x == 0) dense_epilogue(st, counts, s_sum);
 }
 
 // ORs rows src[y] (rw words) into acc over the entries y of flag mask m of
@@ -633,7 +691,7 @@ __global__ __launch_bounds__(DB) void k_dense_expand(DenseArgs a, const u32 *pop
         if (threadIdx.x == 0) upop[r] = (u32)tot;
         io += 2;
     }
-    if (threadIdx.x == 0 && io) atomicAdd(&st->exp_io, (unsigned long long)io);
+    if (threadIdx.x == 0) group_add(st, DC_EXP_IO, io);
 }
 
 // One body's output rows, a wave per work item (row x, a slice of its pred
@@ -717,12 +775,12 @@ __global__ __launch_bounds__(DB) void k_dense_combine(DenseArgs a, const u32 *po
             w_io += flagged;
         }
         if (!SG) w_raw += raw;
-        __threadfence();  // release this slice's ORs before counting it finished
+        order_memory();  // this slice's ORs before counting it finished
         u32 old = 0;
         if (lane == 0) old = atomicAdd(&a.slice_done[g], 1u);
         old = (u32)__shfl((int)old, 0, 64);
         if (old + 1 != a.n_slices[g]) continue;  // the same for the whole wave
-        __threadfence();  // acquire: every slice's ORs precede its count
+        order_memory();  // every slice's ORs precede its count
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const u64 w = (u64)lane + 64u * k;
@@ -751,7 +809,7 @@ __global__ __launch_bounds__(DB) void k_dense_combine(DenseArgs a, const u32 *po
         w_rn += total ? 1 : 0;
         w_io += 2;
     }
-    dense_block_end(st, counts, w_new, wave_sum(w_raw), w_io, w_rn);
+    dense_block_end<SG>(st, counts, w_new, wave_sum(w_raw), w_io, w_rn);
 }
 
 // Appends the last body's new tuples (the D rows with a non-zero pop) to the
@@ -768,7 +826,6 @@ __global__ __launch_bounds__(DB) void k_dense_append(DenseArgs a, const u32 *pop
                                                      DenseState *st, const u64 *counts) {
     __shared__ u64 s_w[DWV + 1];
     __shared__ unsigned long long s_base;
-    __shared__ bool s_last;
     __shared__ uint16_t s_buf[DWV][4096];
     const u32 body = st->body;
     if (st->appended >= body) return;
@@ -807,17 +864,11 @@ __global__ __launch_bounds__(DB) void k_dense_append(DenseArgs a, const u32 *pop
         if (pop[x] == 0) continue;
         const u64 w0 = (i % cpr) * 64, w = w0 + lane;
         const u64 v = w < a.rw ? D[(u64)x * a.rw + w] : 0ull;
-        at += stage_write(v, ((u64)x << kb) + w0 * 64, kb, a.log, at, ~0ull, s_buf[wv]);
+        at += stage_write<false>(v, ((u64)x << kb) + w0 * 64, kb, a.log, at, ~0ull, s_buf[wv]);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(&st->append_blocks, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (s_last && threadIdx.x == 0) {
-        __threadfence();
-        st->append_blocks = 0;
+    if (threadIdx.x == 0 && last_of_groups(st, &DenseGroup::append_done, &st->append_groups)) {
+        st->append_groups = 0;
         st->appended = body;
     }
 }
@@ -916,7 +967,7 @@ __global__ __launch_bounds__(TB) void k_bt_transpose(const u64 *src, const u32 *
     if (st && threadIdx.x == 0) {
         u64 segs = TB;  // the stored ones
         for (int w = 0; w < TB / 64; ++w) segs += s_live[w];
-        atomicAdd(&st->tr_io, (unsigned long long)segs);
+        group_add(st, DC_TR_IO, segs);
     }
 }
 
@@ -1027,12 +1078,12 @@ __global__ __launch_bounds__(DB) void k_dense_or_rows(OrRows o, u64 rw, const u3
                         atomicOr((unsigned long long *)&gr[w], (unsigned long long)acc[k]);
                 }
             }
-            __threadfence();  // release this slice's ORs before counting it finished
+            order_memory();  // this slice's ORs before counting it finished
             u32 old = 0;
             if (lane == 0) old = atomicAdd(&o.slice_done[g], 1u);
             old = (u32)__shfl((int)old, 0, 64);
             if (old + 1 != o.n_slices[g]) continue;  // the same for the whole wave
-            __threadfence();  // acquire: every slice's ORs precede its count
+            order_memory();  // every slice's ORs precede its count
             any = false;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -1067,7 +1118,7 @@ __global__ __launch_bounds__(DB) void k_dense_or_rows(OrRows o, u64 rw, const u3
     if (threadIdx.x == 0) {
         u64 t = 0;
         for (int w = 0; w < DWV; ++w) t += s_io[w];
-        if (t) atomicAdd(&st->or_io, (unsigned long long)t);
+        group_add(st, DC_OR_IO, t);
     }
 }
 
@@ -1086,20 +1137,14 @@ __global__ __launch_bounds__(DB) void k_dense_count_col(const u64 *keys, u64 n, 
 }
 
 __global__ __launch_bounds__(DB) void k_dense_fill_col(const u64 *keys, u64 n, int col, int kb,
-                                                       u64 *cursor, u32 *idx) {
+                                                       const u64 *off, u32 *left, u32 *idx) {
     for (u64 i = (u64)blockIdx.x * DB + threadIdx.x; i < n; i += (u64)gridDim.x * DB) {
         const u64 k = keys[i];
         const u64 c0 = k >> 32, c1 = k & 0xffffffffull;
         if ((c0 >> kb) || (c1 >> kb)) continue;
         const u64 row = col ? c1 : c0;
-        const u64 at = atomicAdd((unsigned long long *)&cursor[row], 1ull);
-        idx[at] = (u32)(col ? c0 : c1);
+        idx[off[row] + atomicSub(&left[row], 1u) - 1] = (u32)(col ? c0 : c1);
     }
-}
-
-__global__ __launch_bounds__(DB) void k_u32_to_u64(const u32 *in, u64 n, u64 *out) {
-    for (u64 i = (u64)blockIdx.x * DB + threadIdx.x; i < n; i += (u64)gridDim.x * DB)
-        out[i] = in[i];
 }
 
 __global__ __launch_bounds__(DB) void k_dense_act(const u64 *off, u64 rows, u32 *act,
@@ -1132,34 +1177,47 @@ __global__ __launch_bounds__(DB) void k_dense_planes(const u64 *off, u64 rw, int
     }
 }
 
-// Delta keys -> per-row counts (duplicates counted).
-__global__ __launch_bounds__(DB) void k_dense_mark(const u64 *keys, u64 n, int kb, u32 *pop,
-                                                   DenseState *st) {
-    // one add per run of equal rows within a wave's 64 keys (delta keys
-    // usually come sorted: a row's keys would all add to one counter)
-    const int lane = threadIdx.x & 63;
-    const u64 wave = (u64)blockIdx.x * DWV + (threadIdx.x >> 6);
-    const u64 n_waves = (u64)gridDim.x * DWV;
-    for (u64 base = wave * 64; base < n; base += n_waves * 64) {
-        const u64 i = base + lane;
-        bool valid = false;
-        u64 row = ~0ull - (u64)lane;  // distinct per lane when not a key
-        if (i < n) {
+// pop[row] += the keys of each row; *bad when a key lies outside the domain.
+// A block counts `per` * DB keys in an LDS table of rows (per at most kMarkPer)
+// and adds each row once (a row that finds no place adds directly): a hub row's
+// keys all add to one word, 11 ns each, which took 0.25-0.37 ms for the first
+// delta of SG on an R-MAT graph of 40,000 edges.
+constexpr int kMarkPer = 16;
+constexpr u32 kMarkSlots = 4096, kNoRow = ~0u;
+__global__ __launch_bounds__(DB) void k_dense_mark(const u64 *keys, u64 n, int per, u32 slot_mask,
+                                                   int kb, u32 *pop, DenseState *st) {
+    __shared__ u32 s_row[kMarkSlots], s_cnt[kMarkSlots];
+    const u64 per_round = (u64)DB * per;
+    for (u64 base = (u64)blockIdx.x * per_round; base < n; base += (u64)gridDim.x * per_round) {
+        for (u32 x = threadIdx.x; x <= slot_mask; x += DB) {
+            s_row[x] = kNoRow;
+            s_cnt[x] = 0;
+        }
+        __syncthreads();
+        for (int j = 0; j < per; ++j) {
+            const u64 i = base + (u64)j * DB + threadIdx.x;
+            if (i >= n) break;
             const u64 k = keys[i];
             const u64 c0 = k >> 32, c1 = k & 0xffffffffull;
             if ((c0 >> kb) || (c1 >> kb)) {
                 atomicOr(&st->bad, 1u);
-            } else {
-                valid = true;
-                row = c0;
+                continue;
             }
+            const u32 row = (u32)c0;
+            u32 slot = ((row * 2654435761u) >> 16) & slot_mask;
+            int tries = 8;
+            for (; tries; --tries) {
+                const u32 old = atomicCAS(&s_row[slot], kNoRow, row);
+                if (old == kNoRow || old == row) break;
+                slot = (slot + 1) & slot_mask;
+            }
+            if (tries) atomicAdd(&s_cnt[slot], 1u);
+            else atomicAdd(&pop[row], 1u);
         }
-        const u64 prev = __shfl_up(row, 1, 64);
-        const bool head = lane == 0 || row != prev;
-        const u64 heads = __ballot(head);
-        const u64 above = lane == 63 ? 0ull : (heads & (~0ull << (lane + 1)));
-        const int next = above ? __ffsll((unsigned long long)above) - 1 : 64;
-        if (head && valid) atomicAdd(&pop[row], (u32)(next - lane));
+        __syncthreads();
+        for (u32 x = threadIdx.x; x <= slot_mask; x += DB)
+            if (s_cnt[x]) atomicAdd(&pop[s_row[x]], s_cnt[x]);
+        __syncthreads();
     }
 }
 
@@ -1494,16 +1552,17 @@ bool dense_join_insert(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner, const u64 
         // NEW's keys, in key order, after the keys already in *d_new
         const int rounds = xt_rounds(words);
         const u64 tiles = (words + 64ull * rounds - 1) / (64ull * rounds);
+        u32 *tile_counts;
         u64 *tc;
+        GDL_TRY(scr.get(tiles, &tile_counts));
         GDL_TRY(scr.get(tiles + 1, &tc));
         {
             KTimer kt(ctx, K_BM_EXTRACT, 8.0 * words);
             GDL_TRY(launch_xt_count(ctx, rounds, (const u64 *)R, words, tiles, nullptr, nullptr, 0,
-                                    tc));
+                                    tile_counts));
         }
-        GDL_TRY(scan_inplace(ctx, tc, tiles));
         u64 total = 0;
-        GDL_TRY(read_u64(ctx, tc + tiles, &total));
+        GDL_TRY(exclusive_scan_u32_to_u64(ctx, tile_counts, tiles, tc, &total));
         if (*n_new + total > *new_cap || !*d_new) {
             const u64 cap = *n_new + total + (*n_new + total) / 4 + 1024;
             void *p = nullptr;
@@ -1567,18 +1626,10 @@ static gdl_status group_by_col(gdl_ctx *ctx, DevBufs &mem, const u64 *keys, u64 
                            n, col, kb, cnt_scratch, bad);
         GDL_TRY(check_launch(ctx, "k_dense_count_col"));
     }
-    hipLaunchKernelGGL(k_u32_to_u64, dim3(dgrid(ctx, rows)), dim3(DB), 0, ctx->stream,
-                       cnt_scratch, rows, *off);
-    GDL_TRY(check_launch(ctx, "k_u32_to_u64"));
-    GDL_TRY(scan_inplace(ctx, *off, rows));
+    GDL_TRY(exclusive_scan_u32_to_u64(ctx, cnt_scratch, rows, *off, nullptr));
     if (n) {
-        Scratch scr(ctx);
-        u64 *cursor;
-        GDL_TRY(scr.get(rows, &cursor));
-        GDL_HIP(ctx, hipMemcpyAsync(cursor, *off, rows * sizeof(u64), hipMemcpyDeviceToDevice,
-                                    ctx->stream));
         hipLaunchKernelGGL(k_dense_fill_col, dim3(dgrid(ctx, n)), dim3(DB), 0, ctx->stream, keys,
-                           n, col, kb, cursor, *idx);
+                           n, col, kb, *off, cnt_scratch, *idx);
         GDL_TRY(check_launch(ctx, "k_dense_fill_col"));
     }
     return GDL_OK;
@@ -1948,8 +1999,12 @@ gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
     const bool sym_cand = col_above != ~0ull && rule->r1 == rule->r2 && rule->n1 == rule->n2;
     {
         KTimer kt(ctx, K_DENSE_SETUP, 24.0 * n_delta + 8.0 * rows * rw);
-        hipLaunchKernelGGL(k_dense_mark, dim3(dgrid(ctx, n_delta)), dim3(DB), 0, ctx->stream,
-                           d_delta, n_delta, kb, pop[0], st);
+        // two blocks per CU before a block takes more than DB keys
+        const int per = (int)std::max<u64>(1, std::min<u64>(kMarkPer, n_delta / (512 * DB)));
+        u32 slots = 2 * DB;
+        while (slots < 2u * DB * per && slots < kMarkSlots) slots *= 2;
+        hipLaunchKernelGGL(k_dense_mark, dim3(dgrid(ctx, (n_delta + per - 1) / per)), dim3(DB), 0,
+                           ctx->stream, d_delta, n_delta, per, slots - 1, kb, pop[0], st);
         GDL_TRY(check_launch(ctx, "k_dense_mark"));
         hipLaunchKernelGGL(k_dense_zero_rows, dim3(dgrid(ctx, rows * rw)), dim3(DB), 0,
                            ctx->stream, pop[0], rows, rw, D[0]);
@@ -2177,25 +2232,25 @@ gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
         GDL_TRY(device_error_status(ctx, dev_err));
         for (u32 b = 0; b < r.body; ++b, ++done) {
             const u64 *cb = c + kCounts * b;
-            h_new[done] = cb[0];
-            h_raw[done] = cb[1];
+            h_new[done] = cb[DC_NEW];
+            h_raw[done] = cb[DC_RAW];
             const double row = 8.0 * (double)rw;
             // combine: the pred rows read (D, and SG's U), FULL's row read,
             // the new delta row written, new words set in FULL
-            ctx->stats[K_DENSE_COMBINE].alg_bytes += row * (double)cb[2] + 8.0 * (double)cb[0];
+            ctx->stats[K_DENSE_COMBINE].alg_bytes += row * (double)cb[DC_ROWS_IO] + 8.0 * (double)cb[0];
             // expansion bit by bit: the delta row read, U's row written, one
             // 16-byte entry per delta bit; by columns: the 64-byte segments
             // the transposes read and wrote, the OR's row reads and writes
-            if (cb[5] == 0)
+            if (cb[DC_TR_IO] == 0)
                 ctx->stats[K_DENSE_EXPAND].alg_bytes +=
-                    row * (double)cb[3] + 16.0 * (double)in_delta;
-            ctx->stats[K_DENSE_TRANSPOSE].alg_bytes += 64.0 * (double)cb[5];
-            ctx->stats[K_DENSE_ORROWS].alg_bytes += row * (double)cb[6];
+                    row * (double)cb[DC_EXP_IO] + 16.0 * (double)in_delta;
+            ctx->stats[K_DENSE_TRANSPOSE].alg_bytes += 64.0 * (double)cb[DC_TR_IO];
+            ctx->stats[K_DENSE_ORROWS].alg_bytes += row * (double)cb[DC_OR_IO];
             // append: the rows with new tuples read, their keys written
             if (!log_last)
-                ctx->stats[K_DENSE_APPEND].alg_bytes += row * (double)cb[4] + 8.0 * (double)cb[0];
+                ctx->stats[K_DENSE_APPEND].alg_bytes += row * (double)cb[DC_ROWS_NEW] + 8.0 * (double)cb[0];
             in_delta = cb[0];
-            last_rows = cb[4];
+            last_rows = cb[DC_ROWS_NEW];
             hs->size += cb[0];
         }
         if (!log_last && r.appended < r.body) {
