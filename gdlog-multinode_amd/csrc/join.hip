@@ -51,8 +51,8 @@ __device__ __forceinline__ u64 wave_run_end(const u64 *keys, u64 n, u64 from, u6
 // the next set bit, and only the span's last run looks past the span.  (A
 // galloping search from every run start, a serial chain of dependent loads
 // for a few lanes of each wave, took 1.76 ms to count 41M keys in 262k runs
-// and 0.58 ms to build the direct-mapped index; this takes 0.14 and 0.13 ms,
-// 2.3 and 2.6 TB/s.)
+// and 0.58 ms to build the direct-mapped index; this takes 0.12 and 0.08 ms,
+// 2.7 and 4.0 TB/s.)
 template <int R, typename F>
 __device__ __forceinline__ u32 span_runs(const u64 *keys, u64 n, int shift, u64 base, F emit) {
     const int lane = threadIdx.x & 63;
@@ -62,18 +62,17 @@ __device__ __forceinline__ u32 span_runs(const u64 *keys, u64 n, int shift, u64 
         const u64 i = base + (u64)r * 64 + lane;
         p[r] = i < n ? keys[i] >> shift : 0;
     }
-    u64 before = lane == 0 && base > 0 ? keys[base - 1] >> shift : 0;
+    u64 before = base > 0 ? keys[base - 1] >> shift : 0;
     u32 count = 0;
     u64 last = 0;  // prefix of the span's last key
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const u64 i = base + (u64)r * 64 + lane;
-        const u64 up = __shfl_up(p[r], 1, 64);
-        const bool head = i < n && (i == 0 || (lane ? up : before) != p[r]);
+        const u64 up = wave_shift_up(p[r], before);  // in every lane
+        const bool head = i < n && (i == 0 || up != p[r]);
         heads[r] = __ballot(head);
         count += (u32)__popcll(heads[r]);
-        last = __shfl(p[r], 63, 64);
-        before = last;
+        last = before = wave_last(p[r]);
     }
     if (count == 0) return 0;
     const u64 end = base + 64ull * R;

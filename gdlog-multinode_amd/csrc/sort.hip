@@ -123,12 +123,12 @@ struct DigitState {
                            __HIP_MEMORY_SCOPE_AGENT);
     }
     // Keys of this digit in the tiles before `tile` (> 0); row: the digit's
-    // word of tile 0, rows R words apart.  Reads 8 predecessors at a time, and
+    // word of tile 0, rows R words apart.  Reads 4 predecessors at a time, and
     // waits only for tiles whose block runs and publishes its own count
     // without waiting (tiles are handed out in the order blocks start).
     template <int R>
     static __device__ __forceinline__ u64 before(const S *row, u32 tile) {
-        constexpr int W = 8;
+        constexpr int W = 4;
         u64 sum = 0;
         for (long long j = (long long)tile - 1; j >= 0;) {
             S w[W];
@@ -208,9 +208,9 @@ __global__ __launch_bounds__(RH_B) void k_rs_hist(const u64 *in, u64 n, int lo_b
 // counts, places the keys in digit order in LDS, learns the counts of the
 // tiles before (DigitState::before), and stores the keys run by run, so
 // consecutive lanes store consecutive addresses.  The keys are read and
-// written once.  41M keys: 0.206 ms a pass, 3.2 TB/s (a count launch, a scan
+// written once.  41M keys: 0.198 ms a pass, 3.3 TB/s (a count launch, a scan
 // over tiles and a scatter launch took 0.120 + 0.022 + 0.250); 100,000 keys:
-// 8.6 us (7.4 + 3.4 + 11).  x_flags: 1 compress on reading, 2 expand on writing.
+// 7.9 us (7.4 + 3.4 + 11).  x_flags: 1 compress on reading, 2 expand on writing.
 template <int RB, int B, int I, typename S>
 __global__ __launch_bounds__(B) void k_rs_pass(const u64 *in, u64 *out, u64 n, int pass,
                                                int lo_bits, int x_flags, const u32 *hist, S *state,
@@ -475,16 +475,19 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
 template <int RB>
 static gdl_status tile_passes(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bits, bool xf,
                               int dbits, int passes, u64 *d_out) {
-    // Tiles: 2048 keys up to 2^18 (more CUs at work), 4096 up to 2^22, 8192
-    // above (longer runs per digit in the stores, fewer tickets); a digit's
-    // running count fits 30 bits below 2^30 keys.
+    // Tiles: 2048 keys up to 2^18 (more CUs at work), 4096 up to 2^20, 8192
+    // above (longer runs per digit in the stores, fewer tickets); few keys a
+    // thread, so a wave's serial ranking is short.  Measured, us for 4 passes:
+    // 100,000 keys 40 (256 threads x 8: 43), 1M 70 (512 x 8: 72), 2.5M 101 (4096
+    // keys a tile: 117), 41M 895 (512 x 16: 928).  A digit's running count fits
+    // 30 bits below 2^30 keys.
     if (n <= 1ull << 18)
-        return tile_passes_of<RB, 256, 8, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
-    if (n <= 1ull << 22)
-        return tile_passes_of<RB, 512, 8, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+        return tile_passes_of<RB, 512, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+    if (n <= 1ull << 20)
+        return tile_passes_of<RB, 1024, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
     if (n < 1ull << 30)
-        return tile_passes_of<RB, 512, 16, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
-    return tile_passes_of<RB, 512, 16, u64>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+        return tile_passes_of<RB, 1024, 8, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+    return tile_passes_of<RB, 1024, 8, u64>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
 }
 
 // Shared driver of sort and sort+unique.  For n <= 4096 with `unique`,

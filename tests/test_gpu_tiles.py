@@ -138,9 +138,9 @@ def test_join_offsets_at_tile_edges(ctx, n):
     d.free(); o.free()
 
 
-# tiles of 2048 keys up to 2^18 keys, of 4096 up to 2^22, of 8192 above
-@pytest.mark.parametrize("n", [4097, 6144, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 1_000_001,
-                               1 << 22, (1 << 22) + 1, (1 << 22) + 8192])
+# tiles of 2048 keys up to 2^18 keys, of 4096 up to 2^20, of 8192 above
+@pytest.mark.parametrize("n", [4097, 6144, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 1 << 20, (1 << 20) + 1,
+                               1_100_003, 1 << 22, (1 << 22) + 8193])
 @pytest.mark.parametrize("kind", ["random36", "random32", "sorted", "reversed", "one_odd",
                                   "few", "high_only"])
 def test_sort_at_tile_edges(ctx, n, kind):
