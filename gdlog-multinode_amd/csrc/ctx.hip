@@ -137,9 +137,9 @@ gdl_status read_u64(gdl_ctx *ctx, const u64 *d, u64 *h, int count) {
     return GDL_OK;
 }
 
-gdl_status read_result(gdl_ctx *ctx, u64 *h) {
+gdl_status read_result(gdl_ctx *ctx, u64 *h, int count) {
     GDL_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *h = *(volatile u64 *)result_word(ctx);
+    for (int i = 0; i < count; ++i) h[i] = ((volatile u64 *)result_words(ctx))[i];
     return GDL_OK;
 }
 
@@ -366,7 +366,9 @@ gdl_status gdl_ctx_create(const gdl_config *cfg_in, gdl_ctx **out) {
         hipHostMalloc((void **)&ctx->h_pinned, 64 * sizeof(uint64_t), hipHostMallocDefault) !=
             hipSuccess ||
         hipMalloc((void **)&ctx->d_err, 256) != hipSuccess ||
-        hipMemset(ctx->d_err, 0, 256) != hipSuccess) {
+        hipMemset(ctx->d_err, 0, 256) != hipSuccess ||
+        hipMalloc((void **)&ctx->words, sizeof(CtxWords)) != hipSuccess ||
+        hipMemsetAsync(ctx->words, 0, sizeof(CtxWords), ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         gdl_ctx_destroy(ctx);
         return GDL_ERR_HIP;
@@ -392,6 +394,7 @@ gdl_status gdl_ctx_destroy(gdl_ctx *ctx) {
     delete ctx->alloc;
     if (ctx->d_err) (void)hipFree(ctx->d_err);
     if (ctx->d_tiles) (void)hipFree(ctx->d_tiles);
+    if (ctx->words) (void)hipFree(ctx->words);
     if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
     if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

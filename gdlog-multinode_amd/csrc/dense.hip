@@ -326,14 +326,6 @@ struct DenseArgs {
     u64 *log;
 };
 
-// Every memory operation of this thread before it is done (an atomic: at the
-// device's coherence point) before any after it starts.  What follows reads
-// with agent-scope loads, so no cache has to be written back or invalidated,
-// as a fence would do (the XCD's whole L2, once per block or slice).
-__device__ __forceinline__ void order_memory() {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
 __device__ __forceinline__ void group_add(DenseState *st, DenseCounter c, u64 v) {
     if (v)
         atomicAdd(&st->group[blockIdx.x % kGroups].c[c], (unsigned long long)v);

@@ -89,6 +89,21 @@ enum KernelId {
 };
 extern const char *kKernelNames[K_NUM];
 
+// Device words of a context that kernels leave at zero for the next one (or
+// need no initial value), so that no call clears its counters first; the calls
+// of a context follow each other on its stream.
+constexpr u32 kSortCounts = 4096;              // digit counts of all passes
+constexpr u32 kSortWords = kSortCounts + 16;   // and a ticket counter per pass
+constexpr u32 kMaxEndBlocks = 8192;            // blocks of a kernel that ends in CtxWords
+struct CtxWords {
+    alignas(128) unsigned long long idx[3];    // distinct prefixes, longest run, blocks done
+    alignas(128) unsigned long long bits[3];   // OR of each column, blocks done
+    alignas(128) unsigned long long cursor;    // new keys, and blocks done from bit 50 on
+    unsigned long long outside;                // a key was outside the id bound
+    alignas(128) u32 sort[2][kSortWords];      // a sort uses one and clears the other
+    alignas(128) unsigned long long produced[kMaxEndBlocks];  // a word per block, set before read
+};
+
 struct PendingTiming {
     int kid;
     hipEvent_t start, stop;
@@ -114,6 +129,9 @@ struct gdl_ctx {
     uint64_t *d_tiles = nullptr;   // running sums of single-pass kernels (gdl::TileLook)
     uint64_t tile_cap = 0;         // tiles d_tiles has room for
     uint32_t tile_epoch = 0;       // the last call's tag, 0..255
+    gdl::CtxWords *words = nullptr;  // device
+    uint32_t sort_set = 0;         // the set of digit counts the next sort uses
+    bool sort_dirty = false;       // a sort did not get to clear the other set
     int cu_count = 0;
     gdl_tuning tune{GDL_DEFAULT_LOAD_FACTOR, 8, 8, 256};  // load_factor mirrors cfg.load_factor
     std::string last_error;
@@ -267,10 +285,11 @@ struct TileLook {
 constexpr u64 kTileWordsAt = 16;  // the words' place in d_tiles, after the ticket's line
 constexpr u64 kTilesMin = 16384;
 gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out);
-// A pinned word that a kernel of the context's stream can write its result to
-// (no copy back to the host), and its value once the stream has been waited for.
-inline u64 *result_word(gdl_ctx *ctx) { return ctx->h_pinned + 63; }
-gdl_status read_result(gdl_ctx *ctx, u64 *h);
+// Pinned words that a kernel of the context's stream can write its results to
+// (no copy back to the host), and their values once the stream has been waited
+// for.
+inline u64 *result_words(gdl_ctx *ctx) { return ctx->h_pinned + 56; }
+gdl_status read_result(gdl_ctx *ctx, u64 *h, int count = 1);
 
 // ---- internal entry points shared between translation units
 gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *d_out,
@@ -295,6 +314,13 @@ gdl_status hashset_reserve2(gdl_ctx *ctx, gdl_hashset *hs, u64 expected, u64 wor
 gdl_status index_build(gdl_ctx *ctx, const u64 *keys, u64 n, int prefix_cols, gdl_index *out);
 gdl_status join_count(gdl_ctx *ctx, const u64 *inner, u64 n_inner, const gdl_index *idx,
                       const u64 *outer, u64 n_outer, u32 *counts, u64 *begins);
+// The outer tuples' run starts and the exclusive scan of the run lengths
+// (n_outer + 1 offsets): join_count and the scan.
+gdl_status join_offsets(gdl_ctx *ctx, const u64 *inner, u64 n_inner, const gdl_index *idx,
+                        const u64 *outer, u64 n_outer, u64 *begins, u64 *offsets, u64 *total);
+// Arrays of up to this many u32 values are scanned in one launch: their sum is
+// below the 2^54 that a tile's word holds, whatever they are.
+constexpr u64 kScanOnePass = 1ull << 22;
 // Per-instance hash sets of a segmented fused join (one per batch slot).
 constexpr u32 kMaxSegs = 256;
 // Bodies on bit matrices (dense.hip): the smallest delta for which the
@@ -390,10 +416,33 @@ __device__ __forceinline__ u64 block_exclusive_scan(u64 v, u64 *s_wave, u64 *tot
     return res;
 }
 
+// Every memory operation of this thread before it is done (an atomic: at the
+// device's coherence point) before any after it starts.  What follows reads
+// with agent-scope loads or atomics, so no cache has to be written back or
+// invalidated, as a fence would do (the XCD's whole L2, once per block).
+__device__ __forceinline__ void order_memory() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// A cursor word counts new keys in its low bits and finished blocks from
+// kDoneBit on.
+constexpr int kDoneBit = 50;
+constexpr u64 kNewMask = (1ull << kDoneBit) - 1;
+
+// Counts this block as done (thread 0, after its own updates); true for the
+// last, which sees every other block's.
+__device__ __forceinline__ bool last_block(unsigned long long *done) {
+    order_memory();
+    return atomicAdd(done, 1ull) == gridDim.x - 1;
+}
+
 // A block's tile, in the order in which blocks start: every tile before it
 // belongs to a block that is running or done.  `s_tile` is a shared word.
 __device__ __forceinline__ u32 tile_ticket(const TileLook &look, u32 *s_tile) {
-    if (gridDim.x == 1) return 0;
+    if (gridDim.x == 1) {
+        *s_tile = 0;  // every thread reads its own store
+        return 0;
+    }
     if (threadIdx.x == 0) {
         const u32 t = atomicAdd(look.ticket, 1u);
         // the last ticket is out: back to 0 for the next kernel
@@ -452,6 +501,62 @@ __device__ __forceinline__ u64 tile_before(const TileLook &look, u32 tile, u64 a
     put(2, before + aggregate);
     return before;
 }
+
+// A tile of 8 B values of an exclusive scan, 8 consecutive ones a thread,
+// through LDS: the caller fills `in` (at pad(x) for the tile's value x; zeros
+// past the end) and has a barrier; out[base ..) gets the scan, the last tile
+// out[n] and *total.
+template <int B>
+struct ScanTile {
+    static constexpr int kPer = 8, kTile = B * kPer;
+    u32 in[kTile + kTile / 32];
+    u64 out[kTile + kTile / 32];
+    u64 wave[B / 64];
+    u64 before;
+    u32 tile;
+    // 8-value strides over all banks
+    static __device__ __forceinline__ u32 pad(u32 x) { return x + x / 32; }
+
+    __device__ __forceinline__ void scan(const TileLook &look, u64 base, u64 n, u64 *out_to,
+                                         u64 *total) {
+        const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+        u32 v[kPer];
+        u64 sum = 0;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            v[j] = in[pad(t * kPer + j)];
+            sum += v[j];
+        }
+        const u64 inc = wave_inclusive_scan(sum);
+        if (lane == 63) wave[w] = inc;
+        __syncthreads();
+        if (t < 64) {
+            u64 all = 0;
+            for (int k = 0; k < B / 64; ++k) all += wave[k];
+            const u64 b = tile_before(look, tile, all);
+            if (t == 0) {
+                before = b;
+                if (tile == gridDim.x - 1) {
+                    out_to[n] = b + all;
+                    if (total) *total = b + all;
+                }
+            }
+        }
+        u64 at = inc - sum;
+        for (int k = 0; k < w; ++k) at += wave[k];
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            out[pad(t * kPer + j)] = at;
+            at += v[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kPer; ++r) {
+            const u32 x = r * B + t;
+            if (base + x < n) out_to[base + x] = before + out[pad(x)];
+        }
+    }
+};
 
 __device__ __forceinline__ u32 key_col(u64 k, int c) {
     return c ? (u32)(k & 0xffffffffull) : (u32)(k >> 32);

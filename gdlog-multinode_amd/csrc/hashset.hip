@@ -70,7 +70,7 @@ __device__ __forceinline__ bool bm_insert_wave(u64 *words, int kb, bool valid, u
 // all on one address, serialised at a few ns each.
 constexpr int kHsPer = 4;
 __global__ __launch_bounds__(HB) void k_hs_insert_new(u64 *slots, u64 mask, const u64 *keys, u64 n,
-                                                      u64 *out, unsigned long long *counter) {
+                                                      u64 *out, CtxWords *words, u64 *result) {
     __shared__ u32 s_cnt[HB / 64 + 1];
     __shared__ unsigned long long s_base;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(HB) void k_hs_insert_new(u64 *slots, u64 mask, cons
                 s_cnt[w] = t;
                 t += x;
             }
-            s_base = t ? atomicAdd(counter, (unsigned long long)t) : 0ull;
+            s_base = t ? atomicAdd(&words->cursor, (unsigned long long)t) & kNewMask : 0ull;
         }
         __syncthreads();
         u64 pos = s_base + s_cnt[wv];
@@ -116,6 +116,12 @@ __global__ __launch_bounds__(HB) void k_hs_insert_new(u64 *slots, u64 mask, cons
         }
         __syncthreads();  // s_cnt and s_base are rewritten next round
     }
+    if (threadIdx.x) return;
+    // the last block has every block's count in the same word
+    const u64 old = atomicAdd(&words->cursor, 1ull << kDoneBit);
+    if ((old >> kDoneBit) != gridDim.x - 1) return;
+    *result = old & kNewMask;
+    atomicExch(&words->cursor, 0ull);
 }
 
 // Re-inserts every member of an old table into a new one.
@@ -297,19 +303,14 @@ gdl_status hashset_insert_new(gdl_ctx *ctx, gdl_hashset *hs, const u64 *keys, u6
     *n_new = 0;
     if (n == 0) return GDL_OK;
     GDL_TRY(hashset_reserve(ctx, hs, n));
-    Scratch scr(ctx);
-    u64 *counter;
-    GDL_TRY(scr.get(1, &counter));
-    GDL_HIP(ctx, hipMemsetAsync(counter, 0, sizeof(u64), ctx->stream));
     {
         KTimer kt(ctx, K_HS_INSERT, 24.0 * n);
-        hipLaunchKernelGGL(k_hs_insert_new, dim3(hs_grid(ctx, (n + kHsPer - 1) / kHsPer)),
-                           dim3(HB), 0, ctx->stream,
-                           (u64 *)hs->slots, hs_arg(hs), keys, n, d_new,
-                           (unsigned long long *)counter);
+        const unsigned g = std::min(hs_grid(ctx, (n + kHsPer - 1) / kHsPer), kMaxEndBlocks);
+        hipLaunchKernelGGL(k_hs_insert_new, dim3(g), dim3(HB), 0, ctx->stream, (u64 *)hs->slots,
+                           hs_arg(hs), keys, n, d_new, ctx->words, result_words(ctx));
         GDL_TRY(check_launch(ctx, "k_hs_insert_new"));
     }
-    GDL_TRY(read_u64(ctx, counter, n_new));
+    GDL_TRY(read_result(ctx, n_new));
     hs->size += *n_new;
     return GDL_OK;
 }

@@ -95,15 +95,15 @@ __device__ __forceinline__ u32 span_runs(const u64 *keys, u64 n, int shift, u64 
 // grows with the span (1M keys in 400k runs: 37 us with 64 or 256).
 constexpr u64 kLongSpan = 1ull << 22;
 
-// out[0] += distinct prefixes, out[1] = max(longest run); one atomic pair per
-// block; out[2] = the largest prefix (the last key's: keys are sorted).  One
+// result[0] = distinct prefixes, result[1] = the longest run, result[2] = the
+// largest prefix (the last key's: keys are sorted), by the last block.  One
 // block of 16 waves per CU: the atomics all go to the same two words, ~12 ns
 // each (1024 blocks of 4 waves spent 25 us on them).
 constexpr int IC_B = 1024;
 template <int R>
-__global__ __launch_bounds__(IC_B) void k_idx_count(const u64 *keys, u64 n, int shift, u64 *out) {
+__global__ __launch_bounds__(IC_B) void k_idx_count(const u64 *keys, u64 n, int shift,
+                                                    CtxWords *words, u64 *result) {
     __shared__ u64 s_sum[IC_B / 64], s_max[IC_B / 64];
-    if (blockIdx.x == 0 && threadIdx.x == 0) out[2] = keys[n - 1] >> shift;
     u64 acc = 0, mx = 0;
     const u64 span = 64ull * R;
     for (u64 b = ((u64)blockIdx.x * (IC_B / 64) + (threadIdx.x >> 6)) * span; b < n;
@@ -126,8 +126,14 @@ __global__ __launch_bounds__(IC_B) void k_idx_count(const u64 *keys, u64 n, int 
             a += s_sum[w];
             m = s_max[w] > m ? s_max[w] : m;
         }
-        if (a) atomicAdd((unsigned long long *)&out[0], (unsigned long long)a);
-        if (m) atomicMax((unsigned long long *)&out[1], (unsigned long long)m);
+        if (a) atomicAdd(&words->idx[0], (unsigned long long)a);
+        if (m) atomicMax(&words->idx[1], (unsigned long long)m);
+        if (last_block(&words->idx[2])) {
+            result[0] = atomicExch(&words->idx[0], 0ull);
+            result[1] = atomicExch(&words->idx[1], 0ull);
+            result[2] = keys[n - 1] >> shift;
+            atomicExch(&words->idx[2], 0ull);
+        }
     }
 }
 
@@ -207,6 +213,33 @@ __global__ __launch_bounds__(JB) void k_join_count(const IdxSlot *slots, u64 n_s
         counts[i] = (u32)c;
         begins[i] = b;
     }
+}
+
+// The outer tuples' run starts and the exclusive scan of their run lengths in
+// one launch (a count launch and a scan are 3.2 + 5.7 us for CSPA's joins, most
+// of them below 4096 outer tuples).
+template <int B>
+__global__ __launch_bounds__(B) void k_join_offsets(const IdxSlot *slots, u64 n_slots,
+                                                    const u64 *inner, u64 n_inner, int shift,
+                                                    const u64 *outer, u64 n_outer, TileLook look,
+                                                    u64 *begins, u64 *offsets, u64 *total) {
+    using Tile = ScanTile<B>;
+    __shared__ Tile s;
+    const u64 base = (u64)tile_ticket(look, &s.tile) * Tile::kTile;
+#pragma unroll
+    for (int r = 0; r < Tile::kPer; ++r) {
+        const u32 x = r * B + threadIdx.x;
+        const u64 i = base + x;
+        u64 b = 0, c = 0;
+        if (i < n_outer) {
+            if (!lookup_run(slots, n_slots, inner, n_inner, shift, outer[i] >> shift, &b, &c))
+                b = c = 0;
+            begins[i] = b;
+        }
+        s.in[Tile::pad(x)] = (u32)c;
+    }
+    __syncthreads();
+    s.scan(look, base, n_outer, offsets, total);
 }
 
 // ---- outputs numbered by the exclusive scan of the run lengths -------------
@@ -349,60 +382,56 @@ __global__ __launch_bounds__(JB) void k_join_materialize(const u64 *inner, const
 // pairs with a wave prefix sum, so every lane handles one produced tuple per
 // round whatever the run lengths (a hub run is spread over the wave).  New
 // keys are staged per wave in LDS and flushed with one atomic per kStage keys
-// (counters[0] is the output cursor); counters[1] counts produced tuples.
+// (the cursor).
 constexpr u32 kStage = 256;
 constexpr u64 kHubRun = 32;  // longer inner runs may use the load-balanced variant
 
-// A cursor word counts the new keys in its low bits.  In a linear body it also
-// counts the finished blocks and, with LIN_PACKED, the produced tuples, so that
-// one atomic gives a block its place in the output, hands over its counts and
-// tells it whether it is the last: atomics on one word take 11 ns each, and a
-// body's blocks all end at about the same time.
-enum LinMode {
-    LIN_NONE,    // not a linear body: new keys only
-    LIN_WORDS,   // new keys (50 bits), blocks (14); produced counts in a word per block
-    LIN_PACKED,  // new keys (27 bits), produced tuples (27), blocks (10)
+// How a fused join's blocks hand over their counts: one atomic on the cursor
+// word gives a block its place in the output and tells it whether it is the
+// last (atomics on one word take 11 ns each, and the blocks all end at about
+// the same time), which then has all of them.
+enum EndMode {
+    END_WORDS,   // cursor: new keys (50 bits), blocks (14); produced counts in a word per block
+    END_PACKED,  // cursor: new keys (27 bits), produced tuples (27), blocks (10)
 };
 constexpr u32 kPackedBits = 27, kPackedBlocks = 1023;
-template <int LIN>
-struct LinCursor {
-    static constexpr int kNewBits = LIN == LIN_PACKED ? kPackedBits : 50;
-    static constexpr int kDoneBit = LIN == LIN_PACKED ? 2 * kPackedBits : 50;
-    static constexpr u64 kNewMask = (1ull << kNewBits) - 1;
+template <int END>
+struct EndCursor {
+    static constexpr int kNewBits = END == END_PACKED ? kPackedBits : kDoneBit;
+    static constexpr int kBlocksAt = END == END_PACKED ? 2 * kPackedBits : kDoneBit;
+    static constexpr u64 kNew = (1ull << kNewBits) - 1;
 };
 
 // Writes stay below out_cap; a cursor past it tells the host the caller's
 // output bound was wrong.
-template <int LIN>
+template <int END>
 __device__ __forceinline__ void flush_stage(const u64 *stage, u32 n, u64 *out, u64 out_cap,
                                             unsigned long long *cursor, u64 base, int lane) {
     unsigned long long pos = 0;
     if (lane == 0)
-        pos = base + (atomicAdd(cursor, (unsigned long long)n) & LinCursor<LIN>::kNewMask);
+        pos = base + (atomicAdd(cursor, (unsigned long long)n) & EndCursor<END>::kNew);
     pos = __shfl(pos, 0, 64);
     for (u32 x = lane; x < n; x += 64)
         if (pos + x < out_cap) out[pos + x] = stage[x];
 }
 
-// What a linear body's last block learns.
-struct LinCounts {
-    u64 fresh, produced;  // LIN_WORDS: produced is still in the blocks' words
+// What the last block learns.
+struct EndCounts {
+    u64 fresh, produced;  // END_WORDS: produced is still in the blocks' words
 };
 
-// End of a fused-join block: what the waves still stage goes out with one
-// cursor atomic for the whole block.  The produced count: with LIN_NONE one
-// more atomic on *produced_to; with LIN_WORDS a store to the block's own word
-// there, which is at the device's coherence point before the cursor says that
-// the block is done (an agent-scope store that has been waited for: a fence in
-// its place writes the XCD's whole L2 back in each of a body's blocks).
-// Returns whether this block is the body's last.  Every thread calls it.
-template <int B, int LIN>
+// End of a fused-join block: what the waves still stage goes out at the place
+// that the cursor gives, and the block's counts are handed over (EndMode).
+// END_WORDS: the produced count is at the device's coherence point before the
+// cursor says that the block is done (an agent-scope store that has been waited
+// for).  Returns whether this block is the last.  Every thread calls it.
+template <int B, int END>
 __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 staged,
                                                   u64 produced, u64 *out, u64 out_cap,
                                                   unsigned long long *cursor, u64 base,
                                                   unsigned long long *produced_to,
-                                                  LinCounts *counts) {
-    using C = LinCursor<LIN>;
+                                                  EndCounts *counts) {
+    using C = EndCursor<END>;
     __shared__ u32 s_cnt[B / 64];
     __shared__ u64 s_prod[B / 64];
     __shared__ u64 s_base, s_all;
@@ -419,22 +448,17 @@ __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 st
             tot += s_cnt[v];
             prod += s_prod[v];
         }
-        if constexpr (LIN == LIN_NONE) {
-            if (prod) atomicAdd(produced_to, (unsigned long long)prod);
-            s_base = tot ? base + atomicAdd(cursor, (unsigned long long)tot) : 0;
+        u64 add = (1ull << C::kBlocksAt) | tot;
+        if constexpr (END == END_WORDS) {
+            __hip_atomic_store(&produced_to[blockIdx.x], (unsigned long long)prod,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            order_memory();
         } else {
-            u64 add = (1ull << C::kDoneBit) | tot;
-            if constexpr (LIN == LIN_WORDS) {
-                __hip_atomic_store(&produced_to[blockIdx.x], (unsigned long long)prod,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            } else {
-                add += prod << kPackedBits;
-            }
-            const u64 old = atomicAdd(cursor, (unsigned long long)add);
-            s_base = base + (old & C::kNewMask);
-            s_all = old + add;
+            add += prod << kPackedBits;
         }
+        const u64 old = atomicAdd(cursor, (unsigned long long)add);
+        s_base = base + (old & C::kNew);
+        s_all = old + add;
     }
     __syncthreads();
     u64 off = s_base;
@@ -442,13 +466,37 @@ __device__ __forceinline__ bool block_final_flush(u64 (*s_stage)[kStage], u32 st
     const u64 *stage = s_stage[w];
     for (u32 x = lane; x < staged; x += 64)
         if (off + x < out_cap) out[off + x] = stage[x];
-    if constexpr (LIN != LIN_NONE) {
-        const u64 all = s_all;
-        counts->fresh = all & C::kNewMask;
-        counts->produced = (all >> kPackedBits) & LinCursor<LIN_PACKED>::kNewMask;
-        return (all >> C::kDoneBit) == gridDim.x;
-    }
-    return false;
+    const u64 all = s_all;
+    counts->fresh = all & C::kNew;
+    counts->produced = (all >> kPackedBits) & EndCursor<END_PACKED>::kNew;
+    return (all >> C::kBlocksAt) == gridDim.x;
+}
+
+// The sum of the blocks' produced words (END_WORDS), by the last block.
+template <int B>
+__device__ __forceinline__ u64 sum_produced(const unsigned long long *produced) {
+    __shared__ u64 s_sum[B / 64];
+    u64 sum = 0;
+    for (u32 i = threadIdx.x; i < gridDim.x; i += B)
+        sum += __hip_atomic_load(&produced[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    sum = 0;
+    for (int v = 0; v < B / 64; ++v) sum += s_sum[v];
+    return sum;
+}
+
+// The last block of a fused join: new keys, produced tuples and whether a key
+// was outside the id bound to the host; the context's words back to zero.
+template <int B>
+__device__ __forceinline__ void publish_join(CtxWords *words, u64 fresh, u64 *result) {
+    const u64 produced = sum_produced<B>(words->produced);
+    if (threadIdx.x) return;
+    result[0] = fresh;
+    result[1] = produced;
+    result[2] = atomicExch(&words->outside, 0ull);
+    atomicExch(&words->cursor, 0ull);
 }
 
 // Target of a fused join's inserts: one hash set, or one set per fixpoint
@@ -461,7 +509,7 @@ struct HsSel {
     int seg_shift;
     // > 0: the caller sized the set and the output by this id bound; a
     // produced key with an id at or above 2^dom_bits is not inserted and
-    // sets counters[2]
+    // sets *outside
     int dom_bits;
 };
 
@@ -509,6 +557,7 @@ __device__ __forceinline__ u32 insert_keys(const HsSel &sel, const gdl_hs_seg *s
         const gdl_hs_seg hs = sel_set<SEG>(sel, s_segs, keys[r]);
         if (sel.dom_bits && !bm_in_domain(keys[r], sel.dom_bits)) {
             atomicOr(outside, 1ull);
+            order_memory();  // before this block is done
             live &= ~(1u << r);
         } else if (!hs.slots) {
             live &= ~(1u << r);
@@ -563,15 +612,15 @@ __device__ __forceinline__ u32 insert_keys(const HsSel &sel, const gdl_hs_seg *s
 }
 
 // One block's share of a fused join + insert (the blocks of the grid stride
-// over the outer tuples): new keys go to out from base + *cursor on.  LIN,
+// over the outer tuples): new keys go to out from base + *cursor on.  END,
 // produced_to, counts and the result as in block_final_flush; *outside flags a
 // key outside the id bound.
-template <int B, bool SEG, int LIN>
+template <int B, bool SEG, int END>
 __device__ __forceinline__ bool join_insert_blocks(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
     u64 out_cap, unsigned long long *cursor, u64 out_base, unsigned long long *produced_to,
-    unsigned long long *outside, LinCounts *counts) {
+    unsigned long long *outside, EndCounts *counts) {
     __shared__ u64 s_excl[B], s_b[B], s_ok[B];
     __shared__ u64 s_stage[B / 64][kStage];
     __shared__ gdl_hs_seg s_segs[SEG ? kMaxSegs : 1];
@@ -620,7 +669,7 @@ __device__ __forceinline__ bool join_insert_blocks(
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage<LIN>(stage, staged, out, out_cap, cursor, out_base, lane);
+                flush_stage<END>(stage, staged, out, out_cap, cursor, out_base, lane);
                 staged = 0;
                 wave_sync_lds();
             }
@@ -629,7 +678,7 @@ __device__ __forceinline__ bool join_insert_blocks(
         }
         wave_sync_lds();  // s_excl / s_b / s_ok are rewritten next round
     }
-    return block_final_flush<B, LIN>(s_stage, staged, produced, out, out_cap, cursor, out_base,
+    return block_final_flush<B, END>(s_stage, staged, produced, out, out_cap, cursor, out_base,
                                      produced_to, counts);
 }
 
@@ -637,16 +686,19 @@ template <int B, bool SEG>
 __global__ __launch_bounds__(B) void k_join_insert(
     const IdxSlot *slots, u64 n_slots, const u64 *inner, u64 n_inner, int shift, const u64 *outer,
     u64 n_outer, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel, u64 *out,
-    u64 out_cap, unsigned long long *counters) {
-    join_insert_blocks<B, SEG, LIN_NONE>(slots, n_slots, inner, n_inner, shift, outer, n_outer,
-                                         arity, s0, s1, pop, plhs, prhs, sel, out, out_cap,
-                                         &counters[0], 0, &counters[1], &counters[2], nullptr);
+    u64 out_cap, u64 out_base, CtxWords *words, u64 *result) {
+    EndCounts c;
+    if (join_insert_blocks<B, SEG, END_WORDS>(slots, n_slots, inner, n_inner, shift, outer,
+                                              n_outer, arity, s0, s1, pop, plhs, prhs, sel, out,
+                                              out_cap, &words->cursor, out_base, words->produced,
+                                              &words->outside, &c))
+        publish_join<B>(words, c.fresh, result);
 }
 
 // State of a stream-ordered linear fixpoint (gdl_fixpoint_linear) in device
 // memory.
 struct LinState {
-    unsigned long long cursor;    // the running body's counts (LinCursor)
+    unsigned long long cursor;    // the running body's counts (EndMode)
     u64 delta_begin, delta_end;   // the body's delta: log[delta_begin, delta_end)
     u64 size;                     // hash set members
     u64 hs_limit;                 // members the set may reach (a fraction of its capacity)
@@ -687,34 +739,24 @@ __device__ void linear_epilogue(LinState *st, u64 *counts, u64 d1, u64 nd, u64 p
 // One body of out := out U map(inner x delta) with FULL = hash set + append
 // log: the delta is the log's last segment, new tuples are appended after it.
 // A stop code set by an earlier body makes it return at once.  produced: a
-// word per block (LIN_WORDS).
-template <int B, int LIN>
+// word per block (END_WORDS).
+template <int B, int END>
 __global__ __launch_bounds__(B) void k_linear_body(const IdxSlot *slots, u64 n_slots,
                                                    const u64 *inner, u64 n_inner, int shift,
                                                    int arity, int s0, int s1, int pop, int plhs,
                                                    int prhs, u64 *hs_slots, u64 hs_mask, u64 *log,
                                                    LinState *st, unsigned long long *produced,
                                                    u64 *counts) {
-    __shared__ u64 s_sum[B / 64];
     if (st->stop != kLinRun) return;  // the same for every block
     const u64 d0 = st->delta_begin, d1 = st->delta_end;
-    LinCounts c;
-    if (!join_insert_blocks<B, false, LIN>(
+    EndCounts c;
+    if (!join_insert_blocks<B, false, END>(
             slots, n_slots, inner, n_inner, shift, log + d0, d1 - d0, arity, s0, s1, pop, plhs,
             prhs, HsSel{hs_slots, hs_mask, nullptr, 0, 0, 0}, log, st->log_cap, &st->cursor, d1,
             produced, nullptr, &c))
         return;
     // the last block: every other one's counts are at the coherence point
-    if constexpr (LIN == LIN_WORDS) {
-        u64 sum = 0;
-        for (u32 i = threadIdx.x; i < gridDim.x; i += B)
-            sum += __hip_atomic_load(&produced[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
-        if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
-        __syncthreads();
-        c.produced = 0;
-        for (int v = 0; v < B / 64; ++v) c.produced += s_sum[v];
-    }
+    if constexpr (END == END_WORDS) c.produced = sum_produced<B>(produced);
     if (threadIdx.x == 0) linear_epilogue(st, counts, d1, c.fresh, c.produced);
 }
 
@@ -729,7 +771,7 @@ template <bool SEG>
 __global__ __launch_bounds__(JB) void k_join_insert_lb(
     const u64 *inner, const u64 *outer, u64 n_outer, const u64 *offsets, const u64 *begins,
     u64 total, u32 per, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel,
-    u64 *out, u64 out_cap, unsigned long long *counters) {
+    u64 *out, u64 out_cap, u64 out_base, CtxWords *words, u64 *result) {
     __shared__ JoinTile jt;
     __shared__ u64 s_stage[JB / 64][kStage];
     __shared__ gdl_hs_seg s_segs[SEG ? kMaxSegs : 1];
@@ -759,7 +801,7 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
         }
         __syncthreads();  // the next tile overwrites the owners
         produced += __popc(live);
-        const u32 fresh = insert_keys<JM_I, SEG>(sel, s_segs, keys, live, &counters[2]);
+        const u32 fresh = insert_keys<JM_I, SEG>(sel, s_segs, keys, live, &words->outside);
 #pragma unroll
         for (int r = 0; r < JM_I; ++r) {
             const bool f = (fresh >> r) & 1u;
@@ -767,7 +809,7 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
             const u32 cnt = (u32)__popcll(bal);
             if (staged + cnt > kStage) {
                 wave_sync_lds();
-                flush_stage<LIN_NONE>(stage, staged, out, out_cap, &counters[0], 0, lane);
+                flush_stage<END_WORDS>(stage, staged, out, out_cap, &words->cursor, out_base, lane);
                 staged = 0;
                 wave_sync_lds();
             }
@@ -775,19 +817,10 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
             staged += cnt;
         }
     }
-    block_final_flush<JB, LIN_NONE>(s_stage, staged, produced, out, out_cap, &counters[0], 0,
-                                    &counters[1], nullptr);
-}
-
-__global__ void k_set2(u64 *p, u64 a, u64 b) {
-    p[0] = a;
-    p[1] = b;
-}
-
-__global__ void k_set3(u64 *p, u64 a, u64 b, u64 c) {
-    p[0] = a;
-    p[1] = b;
-    p[2] = c;
+    EndCounts c;
+    if (block_final_flush<JB, END_WORDS>(s_stage, staged, produced, out, out_cap, &words->cursor,
+                                         out_base, words->produced, &c))
+        publish_join<JB>(words, c.fresh, result);
 }
 
 __global__ __launch_bounds__(JB) void k_project(const u64 *in, u64 n, int arity, int s0, int s1,
@@ -832,21 +865,19 @@ gdl_status index_build(gdl_ctx *ctx, const u64 *keys, u64 n, int prefix_cols, gd
     const int shift = prefix_cols >= 2 ? 0 : 32;
     u64 distinct = 0, max_run = 0, max_prefix = 0;
     {
-        Scratch scr(ctx);
-        u64 *cnt;
-        GDL_TRY(scr.get(3, &cnt));
-        GDL_HIP(ctx, hipMemsetAsync(cnt, 0, 3 * sizeof(u64), ctx->stream));
         KTimer kt(ctx, K_IDX_COUNT, 8.0 * n);
         const u64 cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
         if (n >= kLongSpan)
             hipLaunchKernelGGL(k_idx_count<16>, dim3(std::min<u64>(grid_for(n, IC_B * 16), cus)),
-                               dim3(IC_B), 0, ctx->stream, keys, n, shift, cnt);
+                               dim3(IC_B), 0, ctx->stream, keys, n, shift, ctx->words,
+                               result_words(ctx));
         else
             hipLaunchKernelGGL(k_idx_count<4>, dim3(std::min<u64>(grid_for(n, IC_B * 4), cus)),
-                               dim3(IC_B), 0, ctx->stream, keys, n, shift, cnt);
+                               dim3(IC_B), 0, ctx->stream, keys, n, shift, ctx->words,
+                               result_words(ctx));
         GDL_TRY(check_launch(ctx, "k_idx_count"));
         u64 h[3];
-        GDL_TRY(read_u64(ctx, cnt, h, 3));
+        GDL_TRY(read_result(ctx, h, 3));
         distinct = h[0];
         max_run = h[1];
         max_prefix = h[2];
@@ -915,6 +946,35 @@ gdl_status join_count(gdl_ctx *ctx, const u64 *inner, u64 n_inner, const gdl_ind
                        (const IdxSlot *)idx->slots, idx_arg(idx), inner, n_inner, shift, outer,
                        n_outer, counts, begins);
     return check_launch(ctx, "k_join_count");
+}
+
+gdl_status join_offsets(gdl_ctx *ctx, const u64 *inner, u64 n_inner, const gdl_index *idx,
+                        const u64 *outer, u64 n_outer, u64 *begins, u64 *offsets, u64 *total) {
+    if (n_outer == 0 || n_inner == 0 || idx->n_slots == 0 || n_outer > kScanOnePass) {
+        Scratch scr(ctx);
+        u32 *counts;
+        GDL_TRY(scr.get(n_outer, &counts));
+        GDL_TRY(join_count(ctx, inner, n_inner, idx, outer, n_outer, counts, begins));
+        return exclusive_scan_u32_to_u64(ctx, counts, n_outer, offsets, total);
+    }
+    // tiles of 8192 outer tuples from 2^18 on (fewer tickets), of 2048 below
+    const int shift = idx->prefix_cols >= 2 ? 0 : 32;
+    const bool big = n_outer >= 1ull << 18;
+    const u64 tile = (big ? 1024 : JB) * 8, nt = (n_outer + tile - 1) / tile;
+    TileLook look;
+    GDL_TRY(tile_look(ctx, nt, &look));
+    {
+        KTimer kt(ctx, K_JOIN_COUNT, 8.0 * n_outer + 16.0 * n_outer + 16.0 * n_outer);
+        auto launch = [&](auto kern, int block) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream,
+                               (const IdxSlot *)idx->slots, idx_arg(idx), inner, n_inner, shift,
+                               outer, n_outer, look, begins, offsets, result_words(ctx));
+        };
+        if (big) launch(k_join_offsets<1024>, 1024);
+        else launch(k_join_offsets<JB>, JB);
+        GDL_TRY(check_launch(ctx, "k_join_offsets"));
+    }
+    return read_result(ctx, total);
 }
 
 gdl_status join_materialize(gdl_ctx *ctx, const u64 *inner, const u64 *outer, u64 n_outer,
@@ -1007,14 +1067,12 @@ gdl_status gdl_join(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n_inner,
     *n_out = 0;
     if (n_outer == 0 || n_inner == 0) return GDL_OK;
     Scratch scr(ctx);
-    u32 *counts;
     u64 *begins, *offsets;
-    GDL_TRY(scr.get(n_outer, &counts));
     GDL_TRY(scr.get(n_outer, &begins));
     GDL_TRY(scr.get(n_outer + 1, &offsets));
-    GDL_TRY(join_count(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, counts, begins));
     u64 total = 0;
-    GDL_TRY(exclusive_scan_u32_to_u64(ctx, counts, n_outer, offsets, &total));
+    GDL_TRY(join_offsets(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, begins, offsets,
+                         &total));
     if (total == 0) return GDL_OK;
     void *buf = nullptr;
     std::string err;
@@ -1068,7 +1126,7 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
     const u64 mr = inner_idx->max_run ? inner_idx->max_run : n_inner;
     u64 bound = (n_outer > ~0ull / mr) ? ~0ull : n_outer * mr;
     const u64 loose_limit = std::max<u64>(1ull << 24, 4 * n_outer);
-    const u64 cap_blocks = grid_cap(ctx);
+    const u64 cap_blocks = std::min<u64>(grid_cap(ctx), kMaxEndBlocks);
     const int fb = (int)ctx->tune.join_block;  // block of the flattened kernel
     // the count sizes the output set and buffer; with per-instance sets (SEG)
     // the caller has sized both already (the output capacity is checked after
@@ -1080,14 +1138,12 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
         counted = counted || dense_join_pays(ctx, hs, map, pred, inner_idx->prefix_cols, n_inner,
                                              n_outer, bound);
     Scratch lb(ctx);
-    u32 *counts = nullptr;
     u64 *begins = nullptr, *offsets = nullptr;
     if (counted) {
-        GDL_TRY(lb.get(n_outer, &counts));
         GDL_TRY(lb.get(n_outer, &begins));
         GDL_TRY(lb.get(n_outer + 1, &offsets));
-        GDL_TRY(join_count(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, counts, begins));
-        GDL_TRY(exclusive_scan_u32_to_u64(ctx, counts, n_outer, offsets, &bound));
+        GDL_TRY(join_offsets(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, begins, offsets,
+                             &bound));
     }
     if (bound == 0) return GDL_OK;
     if constexpr (!SEG) {
@@ -1118,11 +1174,10 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
                 hs && hs->key_bits ? "bitmap " : "hash ", hs ? (int)hs->key_bits : 0,
                 balanced ? "balanced" : "wave-flattened");
     if (balanced && !counted) {
-        GDL_TRY(lb.get(n_outer, &counts));
         GDL_TRY(lb.get(n_outer, &begins));
         GDL_TRY(lb.get(n_outer + 1, &offsets));
-        GDL_TRY(join_count(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, counts, begins));
-        GDL_TRY(exclusive_scan_u32_to_u64(ctx, counts, n_outer, offsets, &bound));
+        GDL_TRY(join_offsets(ctx, d_inner, n_inner, inner_idx, d_outer, n_outer, begins, offsets,
+                             &bound));
         if (bound == 0) return GDL_OK;
     }
     if constexpr (!SEG) {
@@ -1157,12 +1212,6 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
             *new_cap = cap;
         }
     }
-    Scratch scr(ctx);
-    u64 *counters;
-    GDL_TRY(scr.get(3, &counters));
-    hipLaunchKernelGGL(k_set3, dim3(1), dim3(1), 0, ctx->stream, counters, (u64)*n_new, (u64)0,
-                       (u64)0);
-    GDL_TRY(check_launch(ctx, "k_set3"));
     if (balanced) {
         KTimer kt(ctx, K_JOIN_INSERT, 24.0 * n_outer);
         const u64 nt = (bound + JM_TILE - 1) / JM_TILE;
@@ -1171,7 +1220,7 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
                            ctx->stream, d_inner, d_outer, n_outer, offsets, begins, bound, per,
                            map.arity, map.src[0],
                            map.arity == 2 ? map.src[1] : 0, pred.op, pred.lhs, pred.rhs, sel,
-                           *d_new, *new_cap, (unsigned long long *)counters);
+                           *d_new, *new_cap, (u64)*n_new, ctx->words, result_words(ctx));
         GDL_TRY(check_launch(ctx, "k_join_insert_lb"));
     } else {
         KTimer kt(ctx, K_JOIN_INSERT, 8.0 * n_outer + 64.0 * n_outer);
@@ -1182,7 +1231,7 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
                                (const IdxSlot *)inner_idx->slots, idx_arg(inner_idx), d_inner,
                                n_inner, shift, d_outer, n_outer, map.arity, map.src[0],
                                map.arity == 2 ? map.src[1] : 0, pred.op, pred.lhs, pred.rhs, sel,
-                               *d_new, *new_cap, (unsigned long long *)counters);
+                               *d_new, *new_cap, (u64)*n_new, ctx->words, result_words(ctx));
         };
         switch (fb) {
             case 64: launch(k_join_insert<64, SEG>, 64); break;
@@ -1193,7 +1242,8 @@ static gdl_status join_insert_impl(gdl_ctx *ctx, const u64 *d_inner, u64 n_inner
         GDL_TRY(check_launch(ctx, "k_join_insert"));
     }
     u64 h[3];
-    GDL_TRY(read_u64(ctx, counters, h, 3));
+    GDL_TRY(read_result(ctx, h, 3));
+    h[0] += *n_new;  // the output's end
     if (h[2])
         return fail(ctx, GDL_ERR_OVERFLOW,
                     "fused join: a produced key has an id at or above 2^" +
@@ -1384,9 +1434,9 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         };
         for (int i = 0; i < k; ++i) {
             KTimer kt(ctx, K_LINEAR, 0.0);
-            if (!packed) launch(k_linear_body<512, LIN_WORDS>);
-            else if (LB == 512) launch(k_linear_body<512, LIN_PACKED>);
-            else launch(k_linear_body<256, LIN_PACKED>);
+            if (!packed) launch(k_linear_body<512, END_WORDS>);
+            else if (LB == 512) launch(k_linear_body<512, END_PACKED>);
+            else launch(k_linear_body<256, END_PACKED>);
             GDL_TRY(check_launch(ctx, "k_linear_body"));
         }
         LinState r{};

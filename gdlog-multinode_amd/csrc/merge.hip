@@ -188,7 +188,7 @@ static gdl_status merge_impl(gdl_ctx *ctx, const u64 *A, u64 na, const u64 *B, u
         KTimer kt(ctx, K_MERGE, 8.0 * tot);
         auto launch = [&](auto kern, int block) {
             hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream, A, na, B, nb,
-                               U, D, look, result_word(ctx), ctx->d_err);
+                               U, D, look, result_words(ctx), ctx->d_err);
         };
         if (big) launch(k_merge<1024>, 1024);
         else launch(k_merge<256>, 256);

@@ -218,64 +218,20 @@ __global__ __launch_bounds__(B) void k_compact(const u64 *in, u64 n, F flag, Til
     }
 }
 
-// Exclusive scan of u32 values to u64 in one launch: a tile of 2048 through
-// LDS (8 consecutive values a thread), its offset from tile_before.
-constexpr int SO_I = 8;
-constexpr int SO_TILE = TB * SO_I;
-constexpr u64 kScanOnePass = 1ull << 22;
-__global__ __launch_bounds__(TB) void k_scan_one(const u32 *in, u64 n, TileLook look, u64 *out,
-                                                 u64 *total) {
-    __shared__ u32 s_in[SO_TILE + SO_TILE / 32];
-    __shared__ u64 s_out[SO_TILE + SO_TILE / 32];
-    __shared__ u64 s_w[TB / 64];
-    __shared__ u64 s_before;
-    __shared__ u32 s_tile;
-    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const u32 tile = tile_ticket(look, &s_tile);
-    const u64 base = (u64)tile * SO_TILE;
-    auto pad = [](u32 x) { return x + x / 32; };  // 8-value strides over all banks
+// Exclusive scan of u32 values to u64 in one launch (ScanTile).
+template <int B>
+__global__ __launch_bounds__(B) void k_scan_one(const u32 *in, u64 n, TileLook look, u64 *out,
+                                                u64 *total) {
+    using Tile = ScanTile<B>;
+    __shared__ Tile s;
+    const u64 base = (u64)tile_ticket(look, &s.tile) * Tile::kTile;
 #pragma unroll
-    for (int r = 0; r < SO_I; ++r) {
-        const u32 x = r * TB + t;
-        s_in[pad(x)] = base + x < n ? in[base + x] : 0;
+    for (int r = 0; r < Tile::kPer; ++r) {
+        const u32 x = r * B + threadIdx.x;
+        s.in[Tile::pad(x)] = base + x < n ? in[base + x] : 0;
     }
     __syncthreads();
-    u32 v[SO_I];
-    u64 sum = 0;
-#pragma unroll
-    for (int j = 0; j < SO_I; ++j) {
-        v[j] = s_in[pad(t * SO_I + j)];
-        sum += v[j];
-    }
-    const u64 inc = wave_inclusive_scan(sum);
-    if (lane == 63) s_w[w] = inc;
-    __syncthreads();
-    if (t < 64) {
-        u64 all = 0;
-        for (int k = 0; k < TB / 64; ++k) all += s_w[k];
-        const u64 before = tile_before(look, tile, all);
-        if (t == 0) {
-            s_before = before;
-            if (tile == gridDim.x - 1) {
-                out[n] = before + all;
-                if (total) *total = before + all;
-            }
-        }
-    }
-    u64 at = inc - sum;
-    for (int k = 0; k < w; ++k) at += s_w[k];
-#pragma unroll
-    for (int j = 0; j < SO_I; ++j) {
-        s_out[pad(t * SO_I + j)] = at;
-        at += v[j];
-    }
-    __syncthreads();
-    const u64 before = s_before;
-#pragma unroll
-    for (int r = 0; r < SO_I; ++r) {
-        const u32 x = r * TB + t;
-        if (base + x < n) out[base + x] = before + s_out[pad(x)];
-    }
+    s.scan(look, base, n, out, total);
 }
 
 // ----------------------------------------------------------------- host side
@@ -321,18 +277,24 @@ static gdl_status exclusive_scan_impl(gdl_ctx *ctx, const T *d_in, u64 n, u64 *d
 
 gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *d_out,
                                      u64 *total_host) {
-    // One launch up to 2^22 values: their sum is below the 2^54 that a tile's
-    // word holds whatever they are, and the scans of a program's joins (most of
-    // them below 4096 values) are bound by launches: CSPA's 102 at 500 ids take
-    // 6.4 us each, three launches took 6.0 + 3.0 + 7.8.
+    // One launch where that is exact: the scans of a program's joins (most of
+    // them below 4096 values) are bound by launches, and CSPA's 102 at 500 ids
+    // take 6.4 us each, where three launches took 6.0 + 3.0 + 7.8.
     if (n == 0 || n > kScanOnePass) return exclusive_scan_impl<u32>(ctx, d_in, n, d_out, total_host);
-    const u64 nt = (n + SO_TILE - 1) / SO_TILE;
+    // (tiles of 8192 values from 2^18 on, a quarter of the tickets: 2M values
+    // 12 us, in tiles of 2048 24 us)
+    const bool big = n >= 1ull << 18;
+    const u64 tile = (big ? 1024 : TB) * 8, nt = (n + tile - 1) / tile;
     TileLook look;
     GDL_TRY(tile_look(ctx, nt, &look));
     {
         KTimer kt(ctx, K_SCAN_ONE, 12.0 * n);
-        hipLaunchKernelGGL(k_scan_one, dim3((unsigned)nt), dim3(TB), 0, ctx->stream, d_in, n, look,
-                           d_out, total_host ? result_word(ctx) : nullptr);
+        auto launch = [&](auto kern, int block) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream, d_in, n,
+                               look, d_out, total_host ? result_words(ctx) : nullptr);
+        };
+        if (big) launch(k_scan_one<1024>, 1024);
+        else launch(k_scan_one<TB>, TB);
         GDL_TRY(check_launch(ctx, "k_scan_one"));
     }
     return total_host ? read_result(ctx, total_host) : GDL_OK;
@@ -372,7 +334,7 @@ static gdl_status compact_impl(gdl_ctx *ctx, const u64 *d_in, u64 n, F flag, u64
         KTimer kt(ctx, K_COMPACT, 16.0 * n);
         auto launch = [&](auto kern, int block) {
             hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream, d_in, n,
-                               flag, look, d_out, result_word(ctx));
+                               flag, look, d_out, result_words(ctx));
         };
         if (big) launch(k_compact<1024, F>, 1024);
         else launch(k_compact<TB, F>, TB);

@@ -158,7 +158,7 @@ struct DigitState {
 };
 
 // Digit counts of every pass in one read of the keys: hist[p << RB | digit]
-// (zeroed before), LDS counters per block, two copies by wave parity.  A wave
+// (zero before), LDS counters per block, two copies by wave parity.  A wave
 // whose keys all have one digit (the high digits of sorted or clustered keys)
 // adds it once.  Also clears the passes' first array of digit states.  Four
 // 9-bit digits of 41M keys: 0.100 ms, 3.3 TB/s.
@@ -167,7 +167,7 @@ template <int RB>
 __global__ __launch_bounds__(RH_B) void k_rs_hist(const u64 *in, u64 n, int lo_bits, int xf,
                                                   int dbits, int passes, u32 *hist, u32 *state,
                                                   u64 state_words) {
-    constexpr int BINS = 4096;  // passes << RB is at most this
+    constexpr int BINS = kSortCounts;  // passes << RB is at most this
     __shared__ u32 s_h[2][BINS];
     const int t = threadIdx.x, copy = (t >> 6) & 1;
     const u64 g = (u64)blockIdx.x * RH_B + t, stride = (u64)gridDim.x * RH_B;
@@ -208,13 +208,15 @@ __global__ __launch_bounds__(RH_B) void k_rs_hist(const u64 *in, u64 n, int lo_b
 // counts, places the keys in digit order in LDS, learns the counts of the
 // tiles before (DigitState::before), and stores the keys run by run, so
 // consecutive lanes store consecutive addresses.  The keys are read and
-// written once.  41M keys: 0.198 ms a pass, 3.3 TB/s (a count launch, a scan
+// written once.  The first pass clears the counts of the sort before (`clear`)
+// for the next.  41M keys: 0.198 ms a pass, 3.3 TB/s (a count launch, a scan
 // over tiles and a scatter launch took 0.120 + 0.022 + 0.250); 100,000 keys:
 // 7.9 us (7.4 + 3.4 + 11).  x_flags: 1 compress on reading, 2 expand on writing.
 template <int RB, int B, int I, typename S>
 __global__ __launch_bounds__(B) void k_rs_pass(const u64 *in, u64 *out, u64 n, int pass,
                                                int lo_bits, int x_flags, const u32 *hist, S *state,
-                                               S *state_next, u32 *ticket, u32 *err) {
+                                               S *state_next, u32 *ticket, u32 *clear,
+                                               u32 *err) {
     constexpr int R = 1 << RB, NW = B / 64, TILE = B * I;
     constexpr int DPT = R > B ? R / B : 1;  // digits a thread owns (threads past R / DPT: none)
     constexpr int WORDS = TILE > NW * R / 2 ? TILE : NW * R / 2;
@@ -239,6 +241,8 @@ __global__ __launch_bounds__(B) void k_rs_pass(const u64 *in, u64 *out, u64 n, i
         keys[r] = x < tile_n ? in[base + x] : 0;
     }
     for (int d = t; d < R; d += B) state_next[(u64)tile * R + d] = 0;
+    if (clear && tile == 0)
+        for (u32 x = t; x < kSortWords; x += B) clear[x] = 0;
     u32 *wh = s_hist + w * R;
 #pragma unroll
     for (int r = 0; r < I; ++r) {
@@ -395,39 +399,40 @@ __global__ __launch_bounds__(RS_B) void k_rs_oneblock(const u64 *in, u64 *out, u
     if (t == RS_B - 1) *n_out = off;  // wave 3's running offset ends at the total
 }
 
-// Bit lengths of the two 32-bit halves: out[0] |= c0 of every key, out[1] |= c1.
-__global__ __launch_bounds__(256) void k_key_bits(const u64 *in, u64 n, u64 *out) {
-    u64 hi = 0, lo = 0;
-    for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < n; i += (u64)gridDim.x * 256) {
-        const u64 k = in[i];
-        hi |= k >> 32;
-        lo |= k & 0xffffffffull;
-    }
-    for (int d = 32; d >= 1; d >>= 1) {
-        hi |= __shfl_xor(hi, d, 64);
-        lo |= __shfl_xor(lo, d, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        atomicOr((unsigned long long *)&out[0], (unsigned long long)hi);
-        atomicOr((unsigned long long *)&out[1], (unsigned long long)lo);
-    }
+// The OR of each column over all keys (their bit lengths), to result[0] and
+// result[1] by the last block.
+__global__ __launch_bounds__(256) void k_key_bits(const u64 *in, u64 n, CtxWords *words,
+                                                  u64 *result) {
+    __shared__ u64 s_or[4];
+    u64 both = 0;
+    for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < n; i += (u64)gridDim.x * 256)
+        both |= in[i];
+    for (int d = 32; d >= 1; d >>= 1) both |= __shfl_xor(both, d, 64);
+    if ((threadIdx.x & 63) == 0) s_or[threadIdx.x >> 6] = both;
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int w = 1; w < 4; ++w) both |= s_or[w];
+    atomicOr(&words->bits[0], (unsigned long long)(both >> 32));
+    atomicOr(&words->bits[1], (unsigned long long)(both & 0xffffffffull));
+    if (!last_block(&words->bits[2])) return;
+    result[0] = atomicExch(&words->bits[0], 0ull);
+    result[1] = atomicExch(&words->bits[1], 0ull);
+    atomicExch(&words->bits[2], 0ull);
 }
 
 static int bit_length(u64 v) { return v ? 64 - __builtin_clzll(v) : 0; }
 
 static gdl_status measure_bits(gdl_ctx *ctx, const u64 *d_in, u64 n, int *hi_bits, int *lo_bits) {
-    Scratch scr(ctx);
-    u64 *acc;
-    GDL_TRY(scr.get(2, &acc));
-    GDL_HIP(ctx, hipMemsetAsync(acc, 0, 2 * sizeof(u64), ctx->stream));
-    unsigned grid = (unsigned)std::min<u64>(grid_for(n, 256 * 8), 2048);
+    // (two blocks a CU for large arrays: three atomics each, on one line)
+    const unsigned grid = (unsigned)std::min<u64>(grid_for(n, 256 * 8), 512);
     {
         KTimer kt(ctx, K_KEY_BITS, 8.0 * n);
-        hipLaunchKernelGGL(k_key_bits, dim3(grid), dim3(256), 0, ctx->stream, d_in, n, acc);
+        hipLaunchKernelGGL(k_key_bits, dim3(grid), dim3(256), 0, ctx->stream, d_in, n, ctx->words,
+                           result_words(ctx));
         GDL_TRY(check_launch(ctx, "k_key_bits"));
     }
     u64 h[2];
-    GDL_TRY(read_u64(ctx, acc, h, 2));
+    GDL_TRY(read_result(ctx, h, 2));
     *hi_bits = bit_length(h[0]);
     *lo_bits = bit_length(h[1]);
     return GDL_OK;
@@ -441,14 +446,14 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
     constexpr int R = 1 << RB;
     const u32 nb = (u32)((n + B * I - 1) / (B * I));
     Scratch scr(ctx);
-    u32 *hist;  // passes x R counts, then a ticket counter per pass
     S *state;
     u64 *tmp = nullptr;
-    const size_t hist_words = (size_t)passes * (R + 1);
-    GDL_TRY(scr.get(hist_words, &hist));
     GDL_TRY(scr.get(2 * (u64)R * nb, &state));
     if (passes > 1) GDL_TRY(scr.get(n, &tmp));
-    GDL_HIP(ctx, hipMemsetAsync(hist, 0, hist_words * sizeof(u32), ctx->stream));
+    if (ctx->sort_dirty)
+        GDL_HIP(ctx, hipMemsetAsync(ctx->words->sort, 0, sizeof(ctx->words->sort), ctx->stream));
+    ctx->sort_dirty = true;  // until every launch has been made
+    u32 *hist = ctx->words->sort[ctx->sort_set], *other = ctx->words->sort[ctx->sort_set ^ 1];
     {
         KTimer kt(ctx, K_RS_HIST, 8.0 * n);
         const u64 cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -465,10 +470,12 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
         hipLaunchKernelGGL((k_rs_pass<RB, B, I, S>), dim3(nb), dim3(B), 0, ctx->stream, src, dst,
                            n, pass_code(p * dbits, dbits), lo_bits, x_flags, hist + (size_t)p * R,
                            state + (u64)(p & 1) * R * nb, state + (u64)(~p & 1) * R * nb,
-                           hist + (size_t)passes * R + p, ctx->d_err);
+                           hist + kSortCounts + p, p ? nullptr : other, ctx->d_err);
         GDL_TRY(check_launch(ctx, "k_rs_pass"));
         src = dst;
     }
+    ctx->sort_set ^= 1;
+    ctx->sort_dirty = false;
     return GDL_OK;
 }
 
