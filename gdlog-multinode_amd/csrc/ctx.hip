@@ -170,6 +170,7 @@ Staging::~Staging() {
 }
 
 gdl_status Staging::sync() {
+    GDL_TRY(send());
     GDL_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
     land_pending();
     used_ = 0;
@@ -179,14 +180,53 @@ gdl_status Staging::sync() {
 void Staging::land_pending() {
     for (const Pending &p : pending_) memcpy(p.h_dst, ctx_->h_stage + p.at, p.n);
     pending_.clear();
+    sent_ = 0;
 }
 
 gdl_status Staging::later(void *h_dst, const void *d_src, size_t n) {
     if (!n) return GDL_OK;
     char *at;
     GDL_TRY(room(n, &at));
-    GDL_HIP(ctx_, hipMemcpyAsync(at, d_src, n, hipMemcpyDeviceToHost, ctx_->stream));
-    pending_.push_back({h_dst, (size_t)(at - ctx_->h_stage), n});
+    pending_.push_back({h_dst, d_src, (size_t)(at - ctx_->h_stage), n});
+    return GDL_OK;
+}
+
+// Up to kGather device ranges, in 4-byte words, into the pinned buffer.
+constexpr int kGather = 8;
+struct GatherArgs {
+    const u32 *src[kGather];
+    u64 at[kGather], words[kGather];
+    int count;
+};
+__global__ __launch_bounds__(256) void k_gather(GatherArgs a, u32 *dst) {
+    const u64 stride = (u64)gridDim.x * 256;
+    for (int k = 0; k < a.count; ++k)
+        for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < a.words[k]; i += stride)
+            dst[a.at[k] + i] = a.src[k][i];
+}
+
+gdl_status Staging::send() {
+    while (sent_ < pending_.size()) {
+        GatherArgs a{};
+        u64 words = 0;
+        for (; sent_ < pending_.size() && a.count < kGather; ++sent_) {
+            const Pending &p = pending_[sent_];
+            // (places in the buffer are 256-byte aligned)
+            if (p.n % 4 || p.n > (1u << 20)) {
+                GDL_HIP(ctx_, hipMemcpyAsync(ctx_->h_stage + p.at, p.d_src, p.n,
+                                             hipMemcpyDeviceToHost, ctx_->stream));
+                continue;
+            }
+            a.src[a.count] = (const u32 *)p.d_src;
+            a.at[a.count] = p.at / 4;
+            a.words[a.count++] = p.n / 4;
+            words += p.n / 4;
+        }
+        if (!a.count) continue;
+        hipLaunchKernelGGL(k_gather, dim3(std::min(grid_for(words, 256 * 4), 256u)), dim3(256), 0,
+                           ctx_->stream, a, (u32 *)ctx_->h_stage);
+        GDL_TRY(check_launch(ctx_, "k_gather"));
+    }
     return GDL_OK;
 }
 

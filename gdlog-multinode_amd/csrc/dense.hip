@@ -1965,6 +1965,7 @@ gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
     }
     HostEvent grouped;
     GDL_HIP(ctx, hipEventCreateWithFlags(&grouped.e, hipEventDisableTiming));
+    GDL_TRY(stg.send());
     GDL_HIP(ctx, hipEventRecord(grouped.e, ctx->stream));
 
     // the delta as bit rows (buffer 0)

@@ -253,17 +253,21 @@ class Staging {
     gdl_status up(void *d_dst, const void *h_src, size_t n);
     gdl_status down(void *h_dst, const void *d_src, size_t n);
     gdl_status sync();
-    // A copy to the host that lands in h_dst at the next land(), land_at()
-    // or sync(): several reads for one wait.
+    // A copy to the host that lands in h_dst at the next land() or land_at():
+    // several reads for one wait, and one launch (send(), or land() itself)
+    // that gathers them into the buffer: a copy command each costs the host
+    // ~3 us and the stream ~2.6.
     gdl_status later(void *h_dst, const void *d_src, size_t n);
+    gdl_status send();
     gdl_status land();
-    // Waits for `ev` only (recorded after the later() copies): the stream
-    // keeps running the work enqueued after it.
+    // Waits for `ev` only (recorded after send()): the stream keeps running the
+    // work enqueued after it.
     gdl_status land_at(hipEvent_t ev);
 
   private:
     struct Pending {
         void *h_dst;
+        const void *d_src;
         size_t at, n;
     };
     gdl_status room(size_t n, char **at);
@@ -271,6 +275,7 @@ class Staging {
     gdl_ctx *ctx_;
     size_t used_ = 0;
     std::vector<Pending> pending_;
+    size_t sent_ = 0;  // the first of them that no launch has gathered yet
 };
 
 // Running sums over the tiles of one kernel (tile_before below): a ticket
