@@ -186,9 +186,11 @@ void cspa_program(const EdgeInput &assign, const EdgeInput &dereference, int gri
     out->sizes[3] = value_flow_2__2_1->full->tuple_counts;
     out->checksum = relation_checksum(value_alias_2__1_2->full);
     if (out->want_keys) {
-        out->main_keys = relation_keys(value_alias_2__1_2->full);
-        out->extra_keys[0] = relation_keys(value_flow_2__1_2->full);
-        out->extra_keys[1] = relation_keys(memory_alias_2__1_2->full);
+        take_keys(value_alias_2__1_2->full, out->main_dst, out->main_cap, &out->main_keys);
+        take_keys(value_flow_2__1_2->full, out->extra_dst[0], out->extra_cap[0],
+                  &out->extra_keys[0]);
+        take_keys(memory_alias_2__1_2->full, out->extra_dst[1], out->extra_cap[1],
+                  &out->extra_keys[1]);
     }
     for (Relation *r : {assign_2__2_1, dereference_2__1_2, dereference_2__2_1, value_flow_2__1_2,
                         value_flow_2__2_1, memory_alias_2__1_2, memory_alias_2__2_1,

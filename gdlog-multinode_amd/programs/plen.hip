@@ -82,8 +82,10 @@ void path_length_program(const EdgeInput &graph, int grid_size, int block_size,
                 check(st, "gdl_segment_labels_sorted");
             }
             if (lens) {
-                host_lens.resize(n);
-                check(gdl_memcpy_d2h(ctx, host_lens.data(), sorted_labels, n * sizeof(uint32_t)),
+                const bool direct = out->lens_dst && n <= out->main_cap;
+                if (!direct) host_lens.resize(n);
+                check(gdl_memcpy_d2h(ctx, direct ? out->lens_dst : host_lens.data(),
+                                     sorted_labels, n * sizeof(uint32_t)),
                       "lens D2H");
             }
             container_take(full, sorted, n, n, true);
@@ -109,7 +111,7 @@ void path_length_program(const EdgeInput &graph, int grid_size, int block_size,
     out->n_main = n;
     out->checksum = relation_checksum(full);
     out->sizes[0] = bounds.size() - 1;  // distinct hop counts: the longest is this many
-    if (out->want_keys) out->main_keys = relation_keys(full);
+    if (out->want_keys) take_keys(full, out->main_dst, out->main_cap, &out->main_keys);
     if (lens) *lens = std::move(host_lens);
     free_relation(edge_2__2_1);
     free_relation(path_2__1_2);

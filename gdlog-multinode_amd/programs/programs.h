@@ -55,10 +55,19 @@ struct ProgramOutput {
     uint64_t checksum = 0;  // relation_checksum of the main output
     std::vector<uint64_t> main_keys;
     std::vector<uint64_t> extra_keys[2];
+    // where the caller wants them: a result that fits its destination goes
+    // there from the device, and its vector stays empty
+    uint64_t *main_dst = nullptr, *extra_dst[2] = {nullptr, nullptr};
+    uint64_t main_cap = 0, extra_cap[2] = {0, 0};
+    uint32_t *lens_dst = nullptr;  // path_length's hop counts, main_cap of them
     uint64_t sizes[4] = {0, 0, 0, 0};
 };
 
 double now_ms();  // device-synchronised wall clock
+// The container's keys in order, into dst when they fit its cap, else into *keys.
+// By way of the vector, 25 MB of closure were zeroed and copied twice on the
+// host: the whole of that call took 3.75 ms, straight to dst 2.69 ms.
+void take_keys(GHashRelContainer *c, uint64_t *dst, uint64_t cap, std::vector<uint64_t> *keys);
 uint64_t sum_delta(const std::vector<IterationRecord> &t);
 
 void tc_program(const EdgeInput &graph, int max_iteration, int grid_size, int block_size,

@@ -23,6 +23,15 @@ uint64_t sum_delta(const std::vector<IterationRecord> &t) {
     return s;
 }
 
+void take_keys(GHashRelContainer *c, uint64_t *dst, uint64_t cap, std::vector<uint64_t> *keys) {
+    const uint64_t n = c->tuple_counts;
+    if (!dst || n > cap || !c->sorted) {
+        *keys = relation_keys(c);
+        return;
+    }
+    if (n) check(gdl_memcpy_d2h(context(), dst, c->keys, n * sizeof(uint64_t)), "result D2H");
+}
+
 void EdgeInput::load(Relation *r, const std::string &name, bool reversed, int grid_size,
                      int block_size, bool tmp_flag) const {
     if (dev) {
@@ -104,6 +113,14 @@ gdl_status run_program(gdl_ctx *ctx, gdl_prog_result *res, const gdl_prog_buffer
     reset_checkpoint_sequence();
     ProgramOutput out;
     out.want_keys = bufs && (bufs->out || bufs->extra0 || bufs->extra1);
+    if (bufs) {
+        out.main_dst = bufs->out;
+        out.main_cap = bufs->out_cap;
+        out.extra_dst[0] = bufs->extra0;
+        out.extra_cap[0] = bufs->extra0_cap;
+        out.extra_dst[1] = bufs->extra1;
+        out.extra_cap[1] = bufs->extra1_cap;
+    }
     gdl_status st = GDL_OK;
     try {
         body(&out);
@@ -231,6 +248,9 @@ gdl_status gdl_prog_path_length(gdl_ctx *ctx, const uint64_t *edges, uint64_t n,
     std::vector<uint64_t> k;
     gdl_status st = run_program(ctx, res, nullptr, [&](ProgramOutput *out) {
         out->want_keys = keys != nullptr;
+        out->main_dst = keys;
+        out->main_cap = cap;
+        out->lens_dst = lens;
         path_length_program(in, grid_for_ctx(ctx), kBlock, out, lens ? &l : nullptr);
         k = std::move(out->main_keys);
     });

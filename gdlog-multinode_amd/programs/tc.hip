@@ -42,7 +42,7 @@ void tc_program(const EdgeInput &graph, int max_iteration, int grid_size, int bl
     out->derived = sum_delta(tc_scc.trace);
     out->n_main = path_2__1_2->full->tuple_counts;
     out->checksum = relation_checksum(path_2__1_2->full);
-    if (out->want_keys) out->main_keys = relation_keys(path_2__1_2->full);
+    if (out->want_keys) take_keys(path_2__1_2->full, out->main_dst, out->main_cap, &out->main_keys);
     free_relation(edge_2__2_1);
     free_relation(path_2__1_2);
     delete edge_2__2_1;

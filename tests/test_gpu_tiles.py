@@ -139,8 +139,8 @@ def test_join_offsets_at_tile_edges(ctx, n):
 
 
 # tiles of 2048 keys up to 2^18 keys, of 4096 up to 2^20, of 8192 above
-@pytest.mark.parametrize("n", [4097, 6144, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 1 << 20, (1 << 20) + 1,
-                               1_100_003, 1 << 22, (1 << 22) + 8193])
+@pytest.mark.parametrize("n", [4097, 6144, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 1 << 20,
+                               (1 << 20) + 1, 1_100_003, 1 << 22, (1 << 22) + 8193])
 @pytest.mark.parametrize("kind", ["random36", "random32", "sorted", "reversed", "one_odd",
                                   "few", "high_only"])
 def test_sort_at_tile_edges(ctx, n, kind):
@@ -175,3 +175,34 @@ def test_linear_bodies_of_disjoint_paths(ctx, paths):
     assert np.array_equal(got["out"], want)
     assert [t[3] for t in got["trace"]] == [2 * paths, paths, 0]
     assert [t[2] for t in got["trace"]] == [2 * paths, paths, 0]
+
+
+# a result of n keys goes straight into a buffer that holds it; a smaller one
+# is refused and left as it was
+@pytest.mark.parametrize("prog", ["tc", "sg", "path_length"])
+@pytest.mark.parametrize("short", [0, 1])
+def test_program_results_into_the_callers_buffer(ctx, prog, short):
+    import ctypes
+    e = gdl.gen_er(7, 300, 900)
+    fn = {"tc": ctx.run_tc, "sg": ctx.run_sg, "path_length": ctx.run_path_length}[prog]
+    want = fn(e)
+    n = want["n_out"]
+    p64, p32 = ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint32)
+    out = np.full(n + 8, 5, dtype=np.uint64)
+    lens = np.full(n + 8, 5, dtype=np.uint32)
+    res = gdl.ProgResult()
+    src = e.ctypes.data_as(ctypes.c_void_p)
+    if prog == "path_length":
+        st = ctx.prog.gdl_prog_path_length(ctx.h, src, e.size, 0, ctypes.byref(res),
+                                           out.ctypes.data_as(p64), lens.ctypes.data_as(p32),
+                                           n - short)
+    else:
+        b = gdl.ProgBuffers()
+        b.out, b.out_cap = out.ctypes.data_as(p64), n - short
+        args = (ctx.h, src, e.size, 0) + ((-1,) if prog == "tc" else ())
+        st = getattr(ctx.prog, "gdl_prog_" + prog)(*args, ctypes.byref(res), ctypes.byref(b))
+    assert st == (5 if short else 0) and res.n_out == n
+    k = 0 if short else n
+    assert np.array_equal(out[:k], want["out"][:k]) and np.all(out[k:] == 5)
+    if prog == "path_length":
+        assert np.array_equal(lens[:k], want["lens"][:k]) and np.all(lens[k:] == 5)
