@@ -42,28 +42,6 @@ __device__ __forceinline__ u64 wave_sum(u64 v) {
     return v;
 }
 
-// Position of the j-th set bit (0-based) of w (j < popcount(w)).
-__device__ __forceinline__ int select_bit(u64 w, int j) {
-    int pos = 0;
-    u32 x = (u32)w;
-    int c = __popc(x);
-    if (j >= c) {
-        j -= c;
-        pos = 32;
-        x = (u32)(w >> 32);
-    }
-    c = __popc(x & 0xffffu);
-    if (j >= c) { j -= c; pos += 16; x >>= 16; }
-    c = __popc(x & 0xffu);
-    if (j >= c) { j -= c; pos += 8; x >>= 8; }
-    c = __popc(x & 0xfu);
-    if (j >= c) { j -= c; pos += 4; x >>= 4; }
-    c = __popc(x & 0x3u);
-    if (j >= c) { j -= c; pos += 2; x >>= 2; }
-    if (j >= (int)(x & 1u)) pos += 1;
-    return pos;
-}
-
 // Writes the keys of one round of 64 consecutive words, one per lane (lane
 // l: word wd, bit i -> key of bit number bitbase + 64 l + i, (row << 32) |
 // column with kb-bit columns) to out[base ..), in bit order.  Each lane puts

@@ -299,9 +299,6 @@ gdl_status read_result(gdl_ctx *ctx, u64 *h, int count = 1);
 // ---- internal entry points shared between translation units
 gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *d_out,
                                      u64 *total_host /* may be null: no sync */);
-gdl_status exclusive_scan_u64(gdl_ctx *ctx, const u64 *d_in, u64 n, u64 *d_out);
-// In-place exclusive scan of v[0..n); v[n] receives the total (v holds n + 1).
-gdl_status scan_inplace(gdl_ctx *ctx, u64 *v, u64 n);
 gdl_status sort_keys(gdl_ctx *ctx, const u64 *d_in, u64 n, int hi_bits, int lo_bits, u64 *d_out);
 gdl_status unique_keys(gdl_ctx *ctx, const u64 *d_in, u64 n, u64 *d_out, u64 *n_out);
 gdl_status sort_unique_keys(gdl_ctx *ctx, const u64 *d_in, u64 n, int hi_bits, int lo_bits,

@@ -5,7 +5,7 @@
 // of a sorted key array; each slot maps a prefix to its run [begin,
 // begin + count).  Slot = 16 bytes, probed with one 128-bit load.  The run
 // length is stored saturated at 2^24 - 1 and recomputed by galloping search
-// when saturated.
+// in a probe that finds it so.
 //
 // Materialize is load-balanced: blocks take tiles of 2048 consecutive outputs
 // and find the outer tuples that own them in LDS (JoinTile).
@@ -16,8 +16,6 @@ namespace gdl {
 constexpr int JB = 256;
 constexpr int JM_I = 8;
 constexpr int JM_TILE = JB * JM_I;
-
-__device__ __forceinline__ int prefix_shift(int prefix_cols) { return prefix_cols >= 2 ? 0 : 32; }
 
 // First index >= from whose prefix differs from p (keys sorted, keys[from - 1]
 // has prefix p; n when the run lasts to the end), found by the whole wave: the

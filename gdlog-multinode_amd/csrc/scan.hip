@@ -18,8 +18,7 @@ __device__ __forceinline__ u64 tile_item(u64 base, int w, int r, int lane) {
 __device__ __forceinline__ u64 wave_bcast_last(u64 v) { return __shfl(v, 63, 64); }
 
 // Sum of a tile -> block_sums[blockIdx.x]
-template <typename T>
-__global__ __launch_bounds__(TB) void k_scan_reduce(const T *in, u64 n, u64 *block_sums) {
+__global__ __launch_bounds__(TB) void k_scan_reduce(const u32 *in, u64 n, u64 *block_sums) {
     __shared__ u64 s_w[TB / 64 + 1];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
     const u64 base = (u64)blockIdx.x * TILE;
@@ -34,13 +33,11 @@ __global__ __launch_bounds__(TB) void k_scan_reduce(const T *in, u64 n, u64 *blo
     if (t == 0) block_sums[blockIdx.x] = tot;
 }
 
-// Exclusive scan in place by one block per array (block 0: v0, block 1: v1);
-// v[n] = total, and block 0 also stores it to *total_out.  Each thread scans
-// 4 consecutive elements per round of 4 * BLOCK.
+// Exclusive scan in place by one block; v[n] = total, also stored to
+// *total_out.  Each thread scans 4 consecutive elements per round of 4 * BLOCK.
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_scan_top(u64 *v0, u64 *v1, u64 n, u64 *total_out) {
+__global__ __launch_bounds__(BLOCK) void k_scan_top(u64 *v, u64 n, u64 *total_out) {
     __shared__ u64 s_w[BLOCK / 64 + 1];
-    u64 *v = blockIdx.x ? v1 : v0;
     const int t = threadIdx.x;
     u64 carry = 0;
     for (u64 b = 0; b < n; b += 4 * BLOCK) {
@@ -63,13 +60,12 @@ __global__ __launch_bounds__(BLOCK) void k_scan_top(u64 *v0, u64 *v1, u64 n, u64
     }
     if (t == 0) {
         v[n] = carry;
-        if (total_out) total_out[blockIdx.x] = carry;
+        *total_out = carry;
     }
 }
 
 // Exclusive scan of a tile with the block offset from block_sums.
-template <typename T>
-__global__ __launch_bounds__(TB) void k_scan_down(const T *in, u64 n, const u64 *block_sums,
+__global__ __launch_bounds__(TB) void k_scan_down(const u32 *in, u64 n, const u64 *block_sums,
                                                   u64 *out) {
     __shared__ u64 s_w[TB / 64 + 1];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
@@ -236,16 +232,7 @@ __global__ __launch_bounds__(B) void k_scan_one(const u32 *in, u64 n, TileLook l
 
 // ----------------------------------------------------------------- host side
 
-static gdl_status scan_top(gdl_ctx *ctx, u64 *v, u64 n, u64 *total_dev) {
-    KTimer kt(ctx, K_SCAN_TOP, 16.0 * n);
-    hipLaunchKernelGGL(k_scan_top<1024>, dim3(1), dim3(1024), 0, ctx->stream, v, v, n,
-                       total_dev);
-    return check_launch(ctx, "k_scan_top");
-}
-
-template <typename T>
-static gdl_status exclusive_scan_impl(gdl_ctx *ctx, const T *d_in, u64 n, u64 *d_out,
-                                      u64 *total_host) {
+static gdl_status scan_three(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *d_out, u64 *total_host) {
     if (n == 0) {
         GDL_HIP(ctx, hipMemsetAsync(d_out, 0, sizeof(u64), ctx->stream));
         if (total_host) {
@@ -259,16 +246,21 @@ static gdl_status exclusive_scan_impl(gdl_ctx *ctx, const T *d_in, u64 n, u64 *d
     u64 *bs;
     GDL_TRY(scr.get(nb + 1, &bs));
     {
-        KTimer kt(ctx, K_SCAN_REDUCE, (double)sizeof(T) * n);
-        hipLaunchKernelGGL(k_scan_reduce<T>, dim3((unsigned)nb), dim3(TB), 0, ctx->stream, d_in,
-                           n, bs);
+        KTimer kt(ctx, K_SCAN_REDUCE, 4.0 * n);
+        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(TB), 0, ctx->stream, d_in, n,
+                           bs);
         GDL_TRY(check_launch(ctx, "k_scan_reduce"));
     }
-    GDL_TRY(scan_top(ctx, bs, nb, d_out + n));
     {
-        KTimer kt(ctx, K_SCAN_DOWN, (double)(sizeof(T) + 8) * n);
-        hipLaunchKernelGGL(k_scan_down<T>, dim3((unsigned)nb), dim3(TB), 0, ctx->stream, d_in, n,
-                           bs, d_out);
+        KTimer kt(ctx, K_SCAN_TOP, 16.0 * nb);
+        hipLaunchKernelGGL(k_scan_top<1024>, dim3(1), dim3(1024), 0, ctx->stream, bs, nb,
+                           d_out + n);
+        GDL_TRY(check_launch(ctx, "k_scan_top"));
+    }
+    {
+        KTimer kt(ctx, K_SCAN_DOWN, 12.0 * n);
+        hipLaunchKernelGGL(k_scan_down, dim3((unsigned)nb), dim3(TB), 0, ctx->stream, d_in, n, bs,
+                           d_out);
         GDL_TRY(check_launch(ctx, "k_scan_down"));
     }
     if (total_host) GDL_TRY(read_u64(ctx, d_out + n, total_host));
@@ -280,7 +272,7 @@ gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *
     // One launch where that is exact: the scans of a program's joins (most of
     // them below 4096 values) are bound by launches, and CSPA's 102 at 500 ids
     // take 6.4 us each, where three launches took 6.0 + 3.0 + 7.8.
-    if (n == 0 || n > kScanOnePass) return exclusive_scan_impl<u32>(ctx, d_in, n, d_out, total_host);
+    if (n == 0 || n > kScanOnePass) return scan_three(ctx, d_in, n, d_out, total_host);
     // (tiles of 8192 values from 2^18 on, a quarter of the tickets: 2M values
     // 12 us, in tiles of 2048 24 us)
     const bool big = n >= 1ull << 18;
@@ -298,23 +290,6 @@ gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *
         GDL_TRY(check_launch(ctx, "k_scan_one"));
     }
     return total_host ? read_result(ctx, total_host) : GDL_OK;
-}
-
-gdl_status exclusive_scan_u64(gdl_ctx *ctx, const u64 *d_in, u64 n, u64 *d_out) {
-    return exclusive_scan_impl<u64>(ctx, d_in, n, d_out, nullptr);
-}
-
-gdl_status scan_inplace(gdl_ctx *ctx, u64 *v, u64 n) {
-    // one block up to 2^15 entries (a few microseconds); a 1024-thread block
-    // over 2^18 of them takes ~150 us, the three-pass scan a few launches
-    if (n <= 32768) return scan_top(ctx, v, n, nullptr);
-    Scratch scr(ctx);
-    u64 *tmp;
-    GDL_TRY(scr.get(n + 1, &tmp));
-    GDL_TRY(exclusive_scan_impl<u64>(ctx, v, n, tmp, nullptr));
-    GDL_HIP(ctx, hipMemcpyAsync(v, tmp, (n + 1) * sizeof(u64), hipMemcpyDeviceToDevice,
-                                ctx->stream));
-    return GDL_OK;
 }
 
 template <typename F>
