@@ -143,7 +143,20 @@ gdl_status read_result(gdl_ctx *ctx, u64 *h, int count) {
     return GDL_OK;
 }
 
+bool records_graph(gdl_ctx *ctx) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return ctx->capturing ||
+           (hipStreamIsCapturing(ctx->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone);
+}
+
 gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out) {
+    // Every caller waits for its counts, which no capture allows: the wait
+    // comes first there, so that nothing is recorded and the capture ends in
+    // the error it always ended in.
+    if (records_graph(ctx)) {
+        GDL_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        return fail(ctx, GDL_ERR_UNSUPPORTED, "a call that waits, in a graph capture");
+    }
     if (tiles > ctx->tile_cap) {
         // outside the caching allocator: it lives as long as the context
         const u64 cap = std::max<u64>({tiles, 2 * ctx->tile_cap, kTilesMin});

@@ -290,6 +290,11 @@ struct TileLook {
 constexpr u64 kTileWordsAt = 16;  // the words' place in d_tiles, after the ticket's line
 constexpr u64 kTilesMin = 16384;
 gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out);
+// The stream records a graph (gdl_graph_begin, or a capture of the caller's):
+// what a launch takes from the host is then the same at every replay, so no
+// recorded kernel may use tile words (their epoch) or a context counter that
+// only the next call clears.
+bool records_graph(gdl_ctx *ctx);
 // Pinned words that a kernel of the context's stream can write its results to
 // (no copy back to the host), and their values once the stream has been waited
 // for.

@@ -1,8 +1,8 @@
 // Allocation-free sort + unique for callers that cannot allocate device
 // memory (code under HIP-graph capture, tight serving loops, harnesses that
 // forbid hipMalloc).  Its scratch -- the radix sort's ping-pong buffer and
-// digit counts and the sorted copy ahead of the unique pass -- lives in one file-scope device array of fixed
-// size instead of the context allocator.
+// digit states and the sorted copy ahead of the unique pass -- lives in one
+// file-scope device array of fixed size instead of the context allocator.
 //
 // Each GPU that loads this library holds the array until the process ends.
 // Its device address is looked up once per device, with that device current,

@@ -272,7 +272,9 @@ gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *
     // One launch where that is exact: the scans of a program's joins (most of
     // them below 4096 values) are bound by launches, and CSPA's 102 at 500 ids
     // take 6.4 us each, where three launches took 6.0 + 3.0 + 7.8.
-    if (n == 0 || n > kScanOnePass) return scan_three(ctx, d_in, n, d_out, total_host);
+    // (A recorded graph takes the three: they keep nothing in the context.)
+    if (n == 0 || n > kScanOnePass || records_graph(ctx))
+        return scan_three(ctx, d_in, n, d_out, total_host);
     // (tiles of 8192 values from 2^18 on, a quarter of the tickets: 2M values
     // 12 us, in tiles of 2048 24 us)
     const bool big = n >= 1ull << 18;

@@ -157,6 +157,12 @@ struct DigitState {
     }
 };
 
+// The counts of a sort in a recorded graph (a kernel, not a memset node).
+__global__ __launch_bounds__(256) void k_rs_clear(u32 *hist) {
+    const u32 i = blockIdx.x * 256 + threadIdx.x;
+    if (i < kSortWords) hist[i] = 0;
+}
+
 // Digit counts of every pass in one read of the keys: hist[p << RB | digit]
 // (zero before), LDS counters per block, two copies by wave parity.  A wave
 // whose keys all have one digit (the high digits of sorted or clustered keys)
@@ -448,12 +454,26 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
     Scratch scr(ctx);
     S *state;
     u64 *tmp = nullptr;
-    GDL_TRY(scr.get(2 * (u64)R * nb, &state));
+    const u64 states = 2 * (u64)R * nb;
+    GDL_TRY(scr.get(states + kSortWords, &state));
     if (passes > 1) GDL_TRY(scr.get(n, &tmp));
-    if (ctx->sort_dirty)
-        GDL_HIP(ctx, hipMemsetAsync(ctx->words->sort, 0, sizeof(ctx->words->sort), ctx->stream));
-    ctx->sort_dirty = true;  // until every launch has been made
-    u32 *hist = ctx->words->sort[ctx->sort_set], *other = ctx->words->sort[ctx->sort_set ^ 1];
+    // A recorded sort replays with the set it was recorded with, whatever sorts
+    // ran in between: it has counts of its own (behind the states, so that it
+    // allocates no more than an eager one) and clears them itself.
+    const bool recorded = records_graph(ctx);
+    u32 *hist = (u32 *)(state + states), *other = nullptr;
+    if (recorded) {
+        hipLaunchKernelGGL(k_rs_clear, dim3((kSortWords + 255) / 256), dim3(256), 0, ctx->stream,
+                           hist);
+        GDL_TRY(check_launch(ctx, "k_rs_clear"));
+    } else {
+        if (ctx->sort_dirty)
+            GDL_HIP(ctx,
+                    hipMemsetAsync(ctx->words->sort, 0, sizeof(ctx->words->sort), ctx->stream));
+        ctx->sort_dirty = true;  // until every launch has been made
+        hist = ctx->words->sort[ctx->sort_set];
+        other = ctx->words->sort[ctx->sort_set ^ 1];
+    }
     {
         KTimer kt(ctx, K_RS_HIST, 8.0 * n);
         const u64 cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -474,6 +494,7 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
         GDL_TRY(check_launch(ctx, "k_rs_pass"));
         src = dst;
     }
+    if (recorded) return GDL_OK;
     ctx->sort_set ^= 1;
     ctx->sort_dirty = false;
     return GDL_OK;

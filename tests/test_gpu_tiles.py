@@ -206,3 +206,29 @@ def test_program_results_into_the_callers_buffer(ctx, prog, short):
     assert np.array_equal(out[:k], want["out"][:k]) and np.all(out[k:] == 5)
     if prog == "path_length":
         assert np.array_equal(lens[:k], want["lens"][:k]) and np.all(lens[k:] == 5)
+
+
+# a recorded sort replays with other keys and after other sorts
+@pytest.mark.parametrize("n", [4097, 300_000, 1_100_003])
+def test_sort_in_a_graph(ctx, n):
+    ctx.stats_enable(False)
+    rng = np.random.default_rng(n)
+    sets = [gdl.pack(rng.integers(0, 1 << 18, n), rng.integers(0, 1 << 18, n)) for _ in range(4)]
+    d, o = ctx.to_device(sets[0]), ctx.alloc(n)
+
+    def sort():
+        ctx._check(ctx.eng.gdl_sort_u64(ctx.h, d.ptr, n, 18, 18, o.ptr), "sort")
+
+    sort()  # the scratch is in the context's pool from here on
+    ctx.sync()
+    ctx.graph_begin()
+    sort()
+    g = ctx.graph_end()
+    for k in sets + sets[:1]:
+        assert np.array_equal(ctx.sort(k[: n // 2 + 4096]), np.sort(k[: n // 2 + 4096]))
+        ctx._check(ctx.eng.gdl_memcpy_h2d(ctx.h, d.ptr, k.ctypes.data, k.nbytes), "h2d")
+        ctx.graph_launch(g)
+        ctx.sync()
+        assert np.array_equal(o.numpy(), np.sort(k))
+    ctx.graph_destroy(g)
+    d.free(); o.free()
