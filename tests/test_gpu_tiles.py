@@ -232,3 +232,17 @@ def test_sort_in_a_graph(ctx, n):
         assert np.array_equal(o.numpy(), np.sort(k))
     ctx.graph_destroy(g)
     d.free(); o.free()
+
+
+# a block takes 4096 slots a round, the last round holds the word of the key ~0
+@pytest.mark.parametrize("n", [0, 1, 700, 5000, 300_000])
+@pytest.mark.parametrize("top", [False, True])
+def test_set_extraction_by_blocks(ctx, n, top):
+    keys = np.unique(np.random.default_rng(n).integers(0, 1 << 63, n, dtype=np.uint64))
+    if top:
+        keys = np.append(keys, np.uint64(0xffffffffffffffff))
+    hs = ctx.hashset_create(0)
+    if keys.size:
+        assert ctx.hashset_insert_new(hs, keys).size == keys.size
+    assert np.array_equal(np.sort(ctx.hashset_extract(hs)), keys)
+    ctx.hashset_free(hs)
