@@ -1333,10 +1333,9 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
     const int shift = inner_idx->prefix_cols >= 2 ? 0 : 32;
     const u64 mr = std::max<u64>(inner_idx->max_run, 1);
     Scratch scr(ctx);
-    u64 *st_words, *counts, *produced;
+    u64 *st_words, *counts;
     GDL_TRY(scr.get((sizeof(LinState) + 7) / 8, &st_words));
     GDL_TRY(scr.get(2 * kChunk, &counts));
-    GDL_TRY(scr.get(grid_cap(ctx), &produced));  // a word per block
     LinState *st = (LinState *)st_words;
     u64 d0 = *delta_begin, d1 = *delta_end;
     // TC's map over a bitmap FULL: bodies whose delta is dense run on bit
@@ -1374,21 +1373,12 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         const u64 next = std::max<u64>(nd, 1024) * (u64)std::min(ramp, kChunk);
         GDL_TRY(hashset_reserve2(ctx, hs, next, std::max(worst, next), 0.0,
                                  std::max<u64>(next, 4 * hs->size)));
-        // (and, up to twice the log, the rest of the chunk at this delta's
-        // size: a chunk that stops for a full log leaves its remaining launches
-        // to return at once)
-        const int k = std::min({ramp, kChunk, max_bodies - done});
-        const u64 least_log = std::max<u64>(d1 + std::max<u64>(worst, 4096), 2 * *log_cap);
-        u64 need_log = d1 + std::max<u64>(worst, 4096) + std::min<u64>(nd * (u64)(k - 1), d1);
+        u64 need_log = d1 + std::max<u64>(worst, 4096);
         if (*log_cap < need_log) {
             need_log = std::max<u64>(need_log, 2 * *log_cap);  // geometric
             void *p = nullptr;
             std::string err;
             gdl_status s = ctx->alloc->alloc(need_log * sizeof(u64), &p, &err);
-            if (s == GDL_ERR_OUT_OF_MEMORY && least_log < need_log) {
-                need_log = least_log;
-                s = ctx->alloc->alloc(need_log * sizeof(u64), &p, &err);
-            }
             if (s != GDL_OK) return fail(ctx, s, err);
             if (d1)
                 GDL_HIP(ctx, hipMemcpyAsync(p, *d_log, d1 * sizeof(u64), hipMemcpyDeviceToDevice,
@@ -1397,6 +1387,13 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
             *d_log = (u64 *)p;
             *log_cap = need_log;
         }
+        // as many bodies of this delta's size as the log holds: a body that
+        // finds it full stops the chunk, and the launches after it return at
+        // once but still cost a launch each (50,000-node tree: 4.07 ms so,
+        // 4.34 ms without).  The log is not grown for them: a run that fits
+        // its memory needs no room beyond the next body's.
+        const u64 fit = (*log_cap - d1 - worst) / nd + 1;
+        const int k = (int)std::min<u64>(fit, (u64)std::min({ramp, kChunk, max_bodies - done}));
         LinState h{};
         h.cursor = 0;
         h.delta_begin = d0;
@@ -1414,8 +1411,9 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
         const u64 packed_limit = ((1ull << kPackedBits) - 1) / mr;
         const u64 LB = nd <= std::min<u64>(1u << 16, packed_limit) ? 256 : 512;
         const u64 want = (nd + LB - 1) / LB;
-        const unsigned g = (unsigned)std::min<u64>(grid_cap(ctx), std::max<u64>(want, 16));
-        h.delta_limit = g >= grid_cap(ctx) ? ~0ull : (u64)g * LB * 8;
+        const u64 most = std::min<u64>(grid_cap(ctx), kMaxEndBlocks);
+        const unsigned g = (unsigned)std::min<u64>(most, std::max<u64>(want, 16));
+        h.delta_limit = g >= most ? ~0ull : (u64)g * LB * 8;
         // a delta that turns dense ends the chunk too (bit-matrix bodies next)
         if (dense_at != ~0ull) h.delta_limit = std::min<u64>(h.delta_limit, dense_at - 1);
         const bool packed = g <= kPackedBlocks && nd <= packed_limit;
@@ -1427,8 +1425,8 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
                                (const IdxSlot *)inner_idx->slots, idx_arg(inner_idx), d_inner,
                                n_inner, shift, map.arity, map.src[0],
                                map.arity == 2 ? map.src[1] : 0, pred.op, pred.lhs, pred.rhs,
-                               (u64 *)hs->slots, hs_arg(hs), *d_log, st,
-                               (unsigned long long *)produced, counts);
+                               (u64 *)hs->slots, hs_arg(hs), *d_log, st, ctx->words->produced,
+                               counts);
         };
         for (int i = 0; i < k; ++i) {
             KTimer kt(ctx, K_LINEAR, 0.0);
