@@ -149,7 +149,7 @@ bool records_graph(gdl_ctx *ctx) {
            (hipStreamIsCapturing(ctx->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone);
 }
 
-gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out) {
+gdl_status tile_look(gdl_ctx *ctx, u64 tiles, Scratch *scr, TileLook *out) {
     // Every caller waits for its counts, which no capture allows: the wait
     // comes first there, so that nothing is recorded and the capture ends in
     // the error it always ended in.
@@ -157,24 +157,22 @@ gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out) {
         GDL_HIP(ctx, hipStreamSynchronize(ctx->stream));
         return fail(ctx, GDL_ERR_UNSUPPORTED, "a call that waits, in a graph capture");
     }
-    if (tiles > ctx->tile_cap) {
-        // outside the caching allocator: it lives as long as the context
-        const u64 cap = std::max<u64>({tiles, 2 * ctx->tile_cap, kTilesMin});
-        uint64_t *p = nullptr;
-        GDL_HIP(ctx, hipMalloc((void **)&p, (kTileWordsAt + cap) * sizeof(u64)));
-        if (ctx->d_tiles) (void)hipFree(ctx->d_tiles);  // waits for the device
-        ctx->d_tiles = p;
-        ctx->tile_cap = cap;
-        ctx->tile_epoch = 255;
+    u64 *words = ctx->d_tiles;
+    if (tiles > kTilesKept) {
+        // from the pool, like any scratch: the byte cap counts them, and cached
+        // blocks make room for them
+        GDL_TRY(scr->get(kTileWordsAt + tiles, &words));
+        GDL_HIP(ctx, hipMemsetAsync(words, 0, (kTileWordsAt + tiles) * sizeof(u64), ctx->stream));
+        out->epoch = 1;
+    } else {
+        if (ctx->tile_epoch >= 255) {
+            GDL_HIP(ctx, hipMemsetAsync(words, 0, kTileBytes, ctx->stream));
+            ctx->tile_epoch = 0;
+        }
+        out->epoch = ++ctx->tile_epoch;
     }
-    if (ctx->tile_epoch >= 255) {
-        GDL_HIP(ctx, hipMemsetAsync(ctx->d_tiles, 0, (kTileWordsAt + ctx->tile_cap) * sizeof(u64),
-                                    ctx->stream));
-        ctx->tile_epoch = 0;
-    }
-    out->ticket = (unsigned int *)ctx->d_tiles;
-    out->words = (unsigned long long *)ctx->d_tiles + kTileWordsAt;
-    out->epoch = ++ctx->tile_epoch;
+    out->ticket = (unsigned int *)words;
+    out->words = (unsigned long long *)words + kTileWordsAt;
     return GDL_OK;
 }
 
@@ -421,13 +419,14 @@ gdl_status gdl_ctx_create(const gdl_config *cfg_in, gdl_ctx **out) {
         hipMalloc((void **)&ctx->d_err, 256) != hipSuccess ||
         hipMemset(ctx->d_err, 0, 256) != hipSuccess ||
         hipMalloc((void **)&ctx->words, sizeof(CtxWords)) != hipSuccess ||
-        hipMemsetAsync(ctx->words, 0, sizeof(CtxWords), ctx->stream) != hipSuccess) {
+        hipMemsetAsync(ctx->words, 0, sizeof(CtxWords), ctx->stream) != hipSuccess ||
+        hipMalloc((void **)&ctx->d_tiles, kTileBytes) != hipSuccess ||
+        hipMemsetAsync(ctx->d_tiles, 0, kTileBytes, ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         gdl_ctx_destroy(ctx);
         return GDL_ERR_HIP;
     }
-    TileLook look;  // its memory comes with the context
-    if (tile_look(ctx, kTilesMin, &look) != GDL_OK || noalloc_setup(ctx) != GDL_OK) {
+    if (noalloc_setup(ctx) != GDL_OK) {
         gdl_ctx_destroy(ctx);
         return GDL_ERR_HIP;
     }

@@ -127,7 +127,6 @@ struct gdl_ctx {
     size_t h_stage_cap = 0;
     uint32_t *d_err = nullptr;     // kernel-side error word
     uint64_t *d_tiles = nullptr;   // running sums of single-pass kernels (gdl::TileLook)
-    uint64_t tile_cap = 0;         // tiles d_tiles has room for
     uint32_t tile_epoch = 0;       // the last call's tag, 0..255
     gdl::CtxWords *words = nullptr;  // device
     uint32_t sort_set = 0;         // the set of digit counts the next sort uses
@@ -279,17 +278,19 @@ class Staging {
 };
 
 // Running sums over the tiles of one kernel (tile_before below): a ticket
-// counter and a word per tile, kept with the context.  Every call tags its
-// words with an epoch of its own, so they are cleared once in 255 calls and
-// not before each; the calls of a context follow each other on its stream.
+// counter and a word per tile, kept with the context up to kTilesKept tiles.
+// Every call tags its words with an epoch of its own, so they are cleared once
+// in 255 calls and not before each; the calls of a context follow each other
+// on its stream.  More tiles take their words from the call's scratch.
 struct TileLook {
     unsigned long long *words;
     unsigned int *ticket;
     u32 epoch;
 };
 constexpr u64 kTileWordsAt = 16;  // the words' place in d_tiles, after the ticket's line
-constexpr u64 kTilesMin = 16384;
-gdl_status tile_look(gdl_ctx *ctx, u64 tiles, TileLook *out);
+constexpr u64 kTilesKept = 16384;  // 134M keys of a merge, 268M of a compaction
+constexpr size_t kTileBytes = (kTileWordsAt + kTilesKept) * sizeof(u64);
+gdl_status tile_look(gdl_ctx *ctx, u64 tiles, Scratch *scr, TileLook *out);
 // The stream records a graph (gdl_graph_begin, or a capture of the caller's):
 // what a launch takes from the host is then the same at every replay, so no
 // recorded kernel may use tile words (their epoch) or a context counter that

@@ -959,8 +959,9 @@ gdl_status join_offsets(gdl_ctx *ctx, const u64 *inner, u64 n_inner, const gdl_i
     const int shift = idx->prefix_cols >= 2 ? 0 : 32;
     const bool big = n_outer >= 1ull << 18;
     const u64 tile = (big ? 1024 : JB) * 8, nt = (n_outer + tile - 1) / tile;
+    Scratch scr(ctx);
     TileLook look;
-    GDL_TRY(tile_look(ctx, nt, &look));
+    GDL_TRY(tile_look(ctx, nt, &scr, &look));
     {
         KTimer kt(ctx, K_JOIN_COUNT, 8.0 * n_outer + 16.0 * n_outer + 16.0 * n_outer);
         auto launch = [&](auto kern, int block) {

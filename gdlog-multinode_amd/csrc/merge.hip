@@ -180,8 +180,9 @@ static gdl_status merge_impl(gdl_ctx *ctx, const u64 *A, u64 na, const u64 *B, u
     const bool big = tot >= 1ull << 19;
     const u64 tile = (big ? 1024 : 256) * MG_I, nt = (tot + tile - 1) / tile;
     if (nt > 0x7fffffffull) return fail(ctx, GDL_ERR_OVERFLOW, "merge: too many tiles");
+    Scratch scr(ctx);
     TileLook look;
-    GDL_TRY(tile_look(ctx, nt, &look));
+    GDL_TRY(tile_look(ctx, nt, &scr, &look));
     {
         // algorithmic bytes: read A and B here; the U / D writes are added
         // below once their sizes are known

@@ -279,8 +279,9 @@ gdl_status exclusive_scan_u32_to_u64(gdl_ctx *ctx, const u32 *d_in, u64 n, u64 *
     // 12 us, in tiles of 2048 24 us)
     const bool big = n >= 1ull << 18;
     const u64 tile = (big ? 1024 : TB) * 8, nt = (n + tile - 1) / tile;
+    Scratch scr(ctx);
     TileLook look;
-    GDL_TRY(tile_look(ctx, nt, &look));
+    GDL_TRY(tile_look(ctx, nt, &scr, &look));
     {
         KTimer kt(ctx, K_SCAN_ONE, 12.0 * n);
         auto launch = [&](auto kern, int block) {
@@ -305,8 +306,9 @@ static gdl_status compact_impl(gdl_ctx *ctx, const u64 *d_in, u64 n, F flag, u64
     // in tiles of 4096 are 10,000 of them; smaller tiles below, for more CUs
     const bool big = n >= 1ull << 20;
     const u64 tile = (big ? 1024 : TB) * TI, nt = (n + tile - 1) / tile;
+    Scratch scr(ctx);
     TileLook look;
-    GDL_TRY(tile_look(ctx, nt, &look));
+    GDL_TRY(tile_look(ctx, nt, &scr, &look));
     {
         KTimer kt(ctx, K_COMPACT, 16.0 * n);
         auto launch = [&](auto kern, int block) {

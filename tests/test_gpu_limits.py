@@ -59,3 +59,30 @@ def test_linear_fixpoint_in_the_log_it_has(ctx, n):
     ctx.hashset_free(hs)
     for x in (inner, log, fresh):
         x.free()
+
+
+# More than 16384 tiles of a merge take their running sums' words from the
+# pool: the byte cap counts them, and a call that they fit gives the same result.
+def test_tile_words_of_a_large_merge_are_counted(ctx):
+    n = (1 << 27) + 1000
+    full = np.arange(n, dtype=np.uint64) * np.uint64(2)
+    newt = np.concatenate([full[:: n // 7], full[:: n // 5] + np.uint64(1), full[-1:]])
+    newt = np.unique(newt)
+    f, t, d = ctx.to_device(full), ctx.to_device(newt), ctx.alloc(newt.size)
+    m = u64()
+
+    def diff(room):
+        ctx.set_mem_cap(ctx.mem_info()["in_use"] + room)
+        try:
+            return ctx.eng.gdl_set_difference_u64(ctx.h, t.ptr, newt.size, f.ptr, n, d.ptr,
+                                                  ctypes.byref(m))
+        finally:
+            ctx.set_mem_cap(0)
+
+    want = newt[newt % np.uint64(2) == 1]
+    assert diff(1 << 16) == 2  # the words of 16385 tiles are 131 kB
+    for _ in range(3):
+        m.value = 0
+        assert diff(1 << 20) == 0 and np.array_equal(d.numpy(m.value), want)
+    for x in (f, t, d):
+        x.free()
