@@ -15,7 +15,7 @@ namespace gdl {
 
 constexpr int JB = 256;
 constexpr int JM_I = 8;
-constexpr int JM_TILE = JB * JM_I;
+constexpr int JM_TILE = JB * JM_I;  // outputs of a block's tile
 
 // First index >= from whose prefix differs from p (keys sorted, keys[from - 1]
 // has prefix p; n when the run lasts to the end), found by the whole wave: the
@@ -241,25 +241,27 @@ __global__ __launch_bounds__(B) void k_join_offsets(const IdxSlot *slots, u64 n_
 }
 
 // ---- outputs numbered by the exclusive scan of the run lengths -------------
-// A block takes tiles of JM_TILE consecutive outputs.  The outer tuples whose
+// A block takes tiles of JB * I consecutive outputs.  The outer tuples whose
 // runs meet the tile are compacted in LDS and their first outputs marked in a
 // bit array, so the owner of output w is a population count away, and
 // consecutive lanes take consecutive outputs: inner reads and stores are
 // coalesced whatever the run lengths.  (Each thread used to find its 8
 // consecutive outputs' owner by a binary search over all offsets, ~21
 // dependent loads at 2M outer tuples, and stored through LDS.)
-constexpr int JM_W = JM_TILE / 64;
+template <int I>
 struct JoinTile {
-    u64 src[JM_TILE];  // owner's begin - its first output: inner index = src + output
-    u64 key[JM_TILE];  // owner's outer key
-    u64 mark[JM_W];    // bit w: an owner's outputs start at w (bit 0 always)
-    u32 base[JM_W];    // marks in the words before
+    static constexpr int kTile = JB * I, kWords = kTile / 64;
+    u64 src[kTile];    // owner's begin - its first output: inner index = src + output
+    u64 key[kTile];    // owner's outer key
+    u64 mark[kWords];  // bit w: an owner's outputs start at w (bit 0 always)
+    u32 base[kWords];  // marks in the words before
     u64 lo;            // an outer tuple at or before the tile's first owner
 };
 
 // jt.lo = the last outer tuple o with offsets[o] <= t0, by wave 0 (64-way
 // search: 4 rounds of loads at 2M outer tuples).  Every thread calls it.
-__device__ __forceinline__ void join_tile_seek(JoinTile &jt, const u64 *offsets, u64 n_outer,
+template <int I>
+__device__ __forceinline__ void join_tile_seek(JoinTile<I> &jt, const u64 *offsets, u64 n_outer,
                                                u64 t0) {
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
@@ -278,15 +280,68 @@ __device__ __forceinline__ void join_tile_seek(JoinTile &jt, const u64 *offsets,
     __syncthreads();
 }
 
-// The owners of the outputs [t0, t1), t1 - t0 <= JM_TILE; jt.lo from
-// join_tile_seek or from the tile before.  Every thread of a block of JB calls
-// it; ends with a barrier.  jt.lo moves on to the last owner.
-__device__ __forceinline__ void join_tile_owners(JoinTile &jt, const u64 *outer, u64 n_outer,
+// The last outer tuple o of [lo, lo + len) with offsets[o] <= p, when lo's is.
+__device__ __forceinline__ u64 last_at_most(const u64 *offsets, u64 lo, u64 len, u64 p) {
+    while (len > 1) {
+        const u64 half = len >> 1;
+        if (offsets[lo + half] <= p) lo += half;
+        len -= half;
+    }
+    return lo;
+}
+
+// The owners of the outputs [t0, t1) where most outer tuples have none (a walk
+// over all of a tile's, by one block, took 5.6 ms at 1,544 outputs of 2M): every
+// output is marked, its slot its own number.  A thread searches for the owner
+// of the first of its I consecutive outputs, and at the end of a run for the
+// next owner at doubling distances.  Every thread of a block calls it; ends
+// with a barrier.
+template <int I>
+__device__ __forceinline__ void join_tile_search(JoinTile<I> &jt, const u64 *outer, u64 n_outer,
                                                  const u64 *offsets, const u64 *begins, u64 t0,
                                                  u64 t1) {
     const int t = threadIdx.x;
+    const u64 p0 = t0 + (u64)t * I;
+    if (p0 < t1) {
+        u64 o = last_at_most(offsets, 0, n_outer, p0);
+        u64 end = offsets[o + 1], src = begins[o] - offsets[o], key = outer[o];
+#pragma unroll 1
+        for (int r = 0; r < I && p0 + r < t1; ++r) {
+            const u64 p = p0 + r;
+            if (p >= end) {
+                u64 step = 1;
+                ++o;
+                while (o + step < n_outer && offsets[o + step] <= p) {
+                    o += step;
+                    step *= 2;
+                }
+                o = last_at_most(offsets, o, step < n_outer - o ? step : n_outer - o, p);
+                end = offsets[o + 1];
+                src = begins[o] - offsets[o];
+                key = outer[o];
+            }
+            jt.src[t * I + r] = src;
+            jt.key[t * I + r] = key;
+        }
+    }
+    if (t < JoinTile<I>::kWords) {
+        jt.mark[t] = ~0ull;
+        jt.base[t] = 64 * t;
+    }
+    __syncthreads();
+}
+
+// The owners of the outputs [t0, t1), at most a tile; jt.lo from
+// join_tile_seek or from the tile before.  Every thread of a block of JB calls
+// it; ends with a barrier.  jt.lo moves on to the last owner.
+template <int I>
+__device__ __forceinline__ void join_tile_owners(JoinTile<I> &jt, const u64 *outer, u64 n_outer,
+                                                 const u64 *offsets, const u64 *begins, u64 t0,
+                                                 u64 t1) {
+    constexpr int W = JoinTile<I>::kWords;
+    const int t = threadIdx.x;
     const u64 lo = jt.lo;
-    if (t < JM_W) jt.mark[t] = 0;
+    if (t < W) jt.mark[t] = 0;
     __syncthreads();
     // nearly always one outer tuple a thread: its values stay in registers
     u64 b = 0, e = 0, begin = 0, key = 0;
@@ -308,12 +363,12 @@ __device__ __forceinline__ void join_tile_owners(JoinTile &jt, const u64 *outer,
         mark(offsets[o], offsets[o + 1]);
     __syncthreads();
     if (t < 64) {
-        u32 c = t < JM_W ? (u32)__popcll(jt.mark[t]) : 0, x = c;
+        u32 c = t < W ? (u32)__popcll(jt.mark[t]) : 0, x = c;
         for (int d = 1; d < 64; d <<= 1) {
             const u32 y = __shfl_up(x, d, 64);
             if (t >= d) x += y;
         }
-        if (t < JM_W) jt.base[t] = x - c;
+        if (t < W) jt.base[t] = x - c;
     }
     __syncthreads();
     auto place = [&](u64 o, u64 b, u64 e, u64 begin, u64 key) {
@@ -334,7 +389,8 @@ __device__ __forceinline__ void join_tile_owners(JoinTile &jt, const u64 *outer,
 
 // Slot in jt.src / jt.key of the owner of the tile's output w, where the wave's
 // lanes hold w = 64 x + lane.
-__device__ __forceinline__ u32 join_tile_owner(const JoinTile &jt, u32 w) {
+template <int I>
+__device__ __forceinline__ u32 join_tile_owner(const JoinTile<I> &jt, u32 w) {
     const u64 le = (2ull << (w & 63)) - 1ull;  // all ones for bit 63
     return jt.base[w >> 6] + (u32)__popcll(jt.mark[w >> 6] & le) - 1;
 }
@@ -345,19 +401,24 @@ __device__ __forceinline__ u32 join_tile_owner(const JoinTile &jt, u32 w) {
 // keys took 1.81 ms with a binary search per thread, take 1.22 ms, and 1.15 ms
 // with nontemporal stores, which leave the caches to the inner keys (5 GB read
 // and written at 4.4 TB/s; a large copy reaches 4.8).
+template <int I, bool SPARSE>
 __global__ __launch_bounds__(JB) void k_join_materialize(const u64 *inner, const u64 *outer,
                                                          u64 n_outer, const u64 *offsets,
                                                          const u64 *begins, u64 total, u32 per,
                                                          int arity, int s0, int s1, u64 *out) {
-    __shared__ JoinTile jt;
-    u64 t0 = (u64)blockIdx.x * per * JM_TILE;
-    join_tile_seek(jt, offsets, n_outer, t0);
-    for (u32 k = 0; k < per && t0 < total; ++k, t0 += JM_TILE) {
-        const u64 t1 = t0 + JM_TILE < total ? t0 + JM_TILE : total;
-        join_tile_owners(jt, outer, n_outer, offsets, begins, t0, t1);
-        u64 ik[JM_I], ok[JM_I];
+    constexpr int TILE = JoinTile<I>::kTile;
+    __shared__ JoinTile<I> jt;
+    u64 t0 = (u64)blockIdx.x * per * TILE;
+    if constexpr (!SPARSE) join_tile_seek(jt, offsets, n_outer, t0);
+    for (u32 k = 0; k < per && t0 < total; ++k, t0 += TILE) {
+        const u64 t1 = t0 + TILE < total ? t0 + TILE : total;
+        if constexpr (SPARSE)
+            join_tile_search(jt, outer, n_outer, offsets, begins, t0, t1);
+        else
+            join_tile_owners(jt, outer, n_outer, offsets, begins, t0, t1);
+        u64 ik[I], ok[I];
 #pragma unroll
-        for (int r = 0; r < JM_I; ++r) {
+        for (int r = 0; r < I; ++r) {
             const u32 w = r * JB + threadIdx.x;
             if (t0 + w < t1) {
                 const u32 at = join_tile_owner(jt, w);
@@ -366,7 +427,7 @@ __global__ __launch_bounds__(JB) void k_join_materialize(const u64 *inner, const
             }
         }
 #pragma unroll
-        for (int r = 0; r < JM_I; ++r) {
+        for (int r = 0; r < I; ++r) {
             const u32 w = r * JB + threadIdx.x;
             if (t0 + w < t1)
                 __builtin_nontemporal_store(apply_map(ik[r], ok[r], arity, s0, s1), &out[t0 + w]);
@@ -770,7 +831,7 @@ __global__ __launch_bounds__(JB) void k_join_insert_lb(
     const u64 *inner, const u64 *outer, u64 n_outer, const u64 *offsets, const u64 *begins,
     u64 total, u32 per, int arity, int s0, int s1, int pop, int plhs, int prhs, HsSel sel,
     u64 *out, u64 out_cap, u64 out_base, CtxWords *words, u64 *result) {
-    __shared__ JoinTile jt;
+    __shared__ JoinTile<JM_I> jt;
     __shared__ u64 s_stage[JB / 64][kStage];
     __shared__ gdl_hs_seg s_segs[SEG ? kMaxSegs : 1];
     load_segs<SEG>(sel, s_segs);
@@ -980,13 +1041,35 @@ gdl_status join_materialize(gdl_ctx *ctx, const u64 *inner, const u64 *outer, u6
                             const u64 *offsets, const u64 *begins, u64 total, gdl_colmap map,
                             u64 *out) {
     if (total == 0) return GDL_OK;
-    const u64 nt = (total + JM_TILE - 1) / JM_TILE;
-    if (nt > 0x7fffffffull) return fail(ctx, GDL_ERR_OVERFLOW, "join: output too large");
+    if ((total + JM_TILE - 1) / JM_TILE > 0x7fffffffull)
+        return fail(ctx, GDL_ERR_OVERFLOW, "join: output too large");
     KTimer kt(ctx, K_JOIN_MAT, 16.0 * total);
-    const u32 per = tiles_per_block(ctx, nt);
-    hipLaunchKernelGGL(k_join_materialize, dim3(grid_for(nt, per)), dim3(JB), 0, ctx->stream,
-                       inner, outer, n_outer, offsets, begins, total, per, map.arity, map.src[0],
-                       map.arity == 2 ? map.src[1] : 0, out);
+    // Fewer outputs than outer tuples: owners by search, one tile a block, in
+    // as few outputs a thread as leave the chip full (a search is a chain of
+    // ~21 loads).  2M outer tuples, us by walk | I = 1 | 2 | 8, and before the
+    // walk (a search for every 8 outputs, then one tuple after the other):
+    //   16,000 outputs in runs of 8   532 |  8 |  8 | 10, before 10
+    //   20,000 in runs of 1           641 |  8 | 12 | 52, before 882
+    //   320,000 in runs of 8           56 | 12 | 12 | 12, before 12
+    //   800,000 in runs of 8           38 | 28 | 16 | 16, before 17
+    //   1.6M in runs of 8              28 | 51 | 31 | 21, before 26
+    // and where the rule changes over, by walk | I = 2 | 4 | 8:
+    //   2M in runs of 1                32 | 37 | 45 | 65, before 80
+    //   2M in runs of 40               26 | 24 | 17 | 18, before 20
+    // I = 2 also for a few outputs of many tuples: 4M of 20M in runs of 1
+    // 245 us, I = 4 448, before 370; in runs of 40 49, 34, 34.
+    const bool sparse = total < n_outer;
+    auto launch = [&](auto kern, u64 tile) {
+        const u64 nt = (total + tile - 1) / tile;
+        const u32 per = sparse ? 1 : tiles_per_block(ctx, nt);
+        hipLaunchKernelGGL(kern, dim3(grid_for(nt, per)), dim3(JB), 0, ctx->stream, inner, outer,
+                           n_outer, offsets, begins, total, per, map.arity, map.src[0],
+                           map.arity == 2 ? map.src[1] : 0, out);
+    };
+    if (!sparse) launch(k_join_materialize<JM_I, false>, JM_TILE);
+    else if (total <= 1ull << 18) launch(k_join_materialize<1, true>, JB);
+    else if (total <= 1ull << 20 || total < n_outer / 4) launch(k_join_materialize<2, true>, 2 * JB);
+    else launch(k_join_materialize<4, true>, 4 * JB);
     return check_launch(ctx, "k_join_materialize");
 }
 

@@ -70,6 +70,36 @@ JOIN_SHAPES = {
 }
 
 
+def some(n, hits, prefixes, at=None):
+    """n outer tuples of which `hits` find one of `prefixes` runs, the others none."""
+    rng = np.random.default_rng(n + hits)
+    asks = np.full(n, prefixes + 7)
+    asks[rng.choice(n, hits, replace=False) if at is None else at] = \
+        rng.integers(0, prefixes, hits)
+    return asks
+
+
+# fewer outputs than outer tuples: each thread searches for the owner of the
+# first of its 1, 2 or 4 consecutive outputs (up to 2^18 outputs; up to 2^20 or
+# a quarter of the outer tuples; above), tiles of 256 of those
+JOIN_SHAPES.update({
+    "sparse_one": ([1], some(5000, 1, 1, [4999])), "sparse_first": ([1], some(5000, 1, 1, [0])),
+    "sparse_255": ([1], some(9000, 255, 1)), "sparse_256": ([1], some(9000, 256, 1)),
+    "sparse_257": ([1], some(9000, 257, 1)), "sparse_ends": ([256, 1, 2], some(4000, 9, 3)),
+    "sparse_block": ([1], some(70_000, 300, 1, np.arange(65_000, 65_300))),
+    "sparse_hub": ([90_000, 1, 3], some(200_000, 3, 3)),
+    "sparse_runs": ([(i * 7) % 23 for i in range(500)], some(100_000, 4000, 500)),
+    "sparse_2^18": ([1], some(300_000, 1 << 18, 1)),
+    "sparse_two": ([1], some(300_000, (1 << 18) + 1, 1)),
+    "sparse_two_runs": ([3, 1, 8, 2], some(400_000, 99_999, 4)),
+    "sparse_2^20": ([1], some(1_100_000, 1 << 20, 1)),
+    "sparse_four": ([1], some(1_100_000, (1 << 20) + 1, 1)),
+    "sparse_four_runs": ([9, 1, 40], some(2_000_000, 70_000, 3)),
+    "sparse_quarter": ([1, 2], some(5_000_000, 750_000, 2)),
+    "as_many_as_outer": ([2], some(200_000, 100_000, 1)),
+})
+
+
 @pytest.mark.parametrize("name", JOIN_SHAPES)
 def test_join_outputs_at_tile_edges(ctx, name):
     lengths, asks = JOIN_SHAPES[name]
@@ -78,6 +108,27 @@ def test_join_outputs_at_tile_edges(ctx, name):
     ik, ok, _ = np_join_runs(inner, outer)
     got = ctx.join(inner, outer, (1, 3))  # (inner c1, outer c1)
     assert np.array_equal(got, ((ik & M32) << np.uint64(32)) | (ok & M32))
+
+
+# outputs that few of the outer tuples have take less time than outputs of all
+def test_join_time_where_most_outer_tuples_miss(ctx):
+    inner, n = runs_of([8] * 50_000), 2_000_000
+
+    def ms(hits):
+        outer = gdl.pack(some(n, hits, 50_000), np.arange(n))
+        best = 1e9
+        for _ in range(3):
+            ctx.stats_reset()
+            ctx.join(inner, outer, (1, 3))
+            best = min(best, ctx.stats()["join_materialize"]["total_ms"])
+        return best
+
+    ctx.stats_enable(True)
+    try:
+        assert ms(200) < ms(n)
+    finally:
+        ctx.stats_enable(False)
+        ctx.stats_reset()
 
 
 def _sorted(rng, n, hi):
