@@ -47,11 +47,13 @@ __device__ __forceinline__ u64 wave_sum(u64 v) {
 // column with kb-bit columns) to out[base ..), in bit order.  Each lane puts
 // the round-local numbers of its bits in the wave's LDS list (buf, 4096
 // entries) from its exclusive count on; the wave then stores the keys with
-// consecutive lanes on consecutive positions, past the caches with NT (nothing
-// reads them soon).  Returns the round's total (the same in every lane).
+// consecutive lanes on consecutive positions.  Returns the round's total (the
+// same in every lane).
 // (Words of more than 8 bits put in the list by the whole wave, a bit per
-// lane: 0.40 against 0.32 ms for 68M keys of 2^30 bits.)
-template <bool NT>
+// lane: 0.40 against 0.32 ms for 68M keys of 2^30 bits.  Nontemporal stores,
+// whose lines two rounds share, are slower where many bits are set: 2^30 bits,
+// half of them set 1.03 against 0.77 ms, a quarter 0.60 against 0.48; 3 %
+// 0.124 against 0.139.)
 __device__ __forceinline__ u64 stage_write(u64 wd, u64 bitbase, int kb, u64 *out, u64 base,
                                            u64 out_cap, uint16_t *buf) {
     const int lane = threadIdx.x & 63;
@@ -75,10 +77,7 @@ __device__ __forceinline__ u64 stage_write(u64 wd, u64 bitbase, int kb, u64 *out
     for (u32 t = lane; t < total; t += 64) {
         const u64 bit = bitbase + buf[t];
         const u64 key = ((bit >> kb) << 32) | (bit & lo_mask);
-        if (base + t < out_cap) {
-            if constexpr (NT) __builtin_nontemporal_store(key, &out[base + t]);
-            else out[base + t] = key;
-        }
+        if (base + t < out_cap) out[base + t] = key;
     }
     wave_sync_lds();  // the list is rewritten by the next round
     return total;
@@ -149,7 +148,7 @@ __global__ __launch_bounds__(DB) void k_xt_write(const u64 *words, u64 n_words, 
     u64 base = tile_offsets[tile];
 #pragma unroll
     for (int r = 0; r < R; ++r)
-        base += stage_write<true>(w[r], (t0 + (u64)r * 64) * 64, kb, out, base, out_cap,
+        base += stage_write(w[r], (t0 + (u64)r * 64) * 64, kb, out, base, out_cap,
                             s_buf[threadIdx.x >> 6]);
 }
 
@@ -834,7 +833,7 @@ __global__ __launch_bounds__(DB) void k_dense_append(DenseArgs a, const u32 *pop
         if (pop[x] == 0) continue;
         const u64 w0 = (i % cpr) * 64, w = w0 + lane;
         const u64 v = w < a.rw ? D[(u64)x * a.rw + w] : 0ull;
-        at += stage_write<false>(v, ((u64)x << kb) + w0 * 64, kb, a.log, at, ~0ull, s_buf[wv]);
+        at += stage_write(v, ((u64)x << kb) + w0 * 64, kb, a.log, at, ~0ull, s_buf[wv]);
     }
     __syncthreads();
     if (threadIdx.x == 0 && last_of_groups(st, &DenseGroup::append_done, &st->append_groups)) {
