@@ -100,7 +100,8 @@ struct CtxWords {
     alignas(128) unsigned long long bits[3];   // OR of each column, blocks done
     alignas(128) unsigned long long cursor;    // new keys, and blocks done from bit 50 on
     unsigned long long outside;                // a key was outside the id bound
-    alignas(128) u32 sort[2][kSortWords];      // a sort uses one and clears the other
+    // a sort uses one of the first two and clears the other; recorded ones the third
+    alignas(128) u32 sort[3][kSortWords];
     alignas(128) unsigned long long produced[kMaxEndBlocks];  // a word per block, set before read
 };
 

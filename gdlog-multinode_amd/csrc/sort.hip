@@ -454,14 +454,14 @@ static gdl_status tile_passes_of(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bi
     Scratch scr(ctx);
     S *state;
     u64 *tmp = nullptr;
-    const u64 states = 2 * (u64)R * nb;
-    GDL_TRY(scr.get(states + kSortWords, &state));
     if (passes > 1) GDL_TRY(scr.get(n, &tmp));
+    GDL_TRY(scr.get(2 * (u64)R * nb, &state));  // last: larger tiles need less
     // A recorded sort replays with the set it was recorded with, whatever sorts
-    // ran in between: it has counts of its own (behind the states, so that it
-    // allocates no more than an eager one) and clears them itself.
+    // ran in between: recorded sorts share one that no other sort uses, and each
+    // clears it itself (they follow each other on the stream: their scratch is
+    // one block of the pool, too).
     const bool recorded = records_graph(ctx);
-    u32 *hist = (u32 *)(state + states), *other = nullptr;
+    u32 *hist = ctx->words->sort[2], *other = nullptr;
     if (recorded) {
         hipLaunchKernelGGL(k_rs_clear, dim3((kSortWords + 255) / 256), dim3(256), 0, ctx->stream,
                            hist);
@@ -508,14 +508,19 @@ static gdl_status tile_passes(gdl_ctx *ctx, const u64 *d_in, u64 n, int lo_bits,
     // thread, so a wave's serial ranking is short.  Measured, us for 4 passes:
     // 100,000 keys 40 (256 threads x 8: 43), 1M 70 (512 x 8: 72), 2.5M 101 (4096
     // keys a tile: 117), 41M 895 (512 x 16: 928).  A digit's running count fits
-    // 30 bits below 2^30 keys.
+    // 30 bits below 2^30 keys; from there the words are of 64 bits, and tiles of
+    // 16384 keys halve their number (2^30 keys 23.9 ms, in tiles of 8192 30.5).
+    // Smaller tiles need more memory for their words: where it does not hold
+    // them, tiles of 8192 keys are taken.
+    gdl_status st = GDL_ERR_OUT_OF_MEMORY;
     if (n <= 1ull << 18)
-        return tile_passes_of<RB, 512, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
-    if (n <= 1ull << 20)
-        return tile_passes_of<RB, 1024, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+        st = tile_passes_of<RB, 512, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+    else if (n <= 1ull << 20)
+        st = tile_passes_of<RB, 1024, 4, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+    if (st != GDL_ERR_OUT_OF_MEMORY) return st;
     if (n < 1ull << 30)
         return tile_passes_of<RB, 1024, 8, u32>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
-    return tile_passes_of<RB, 1024, 8, u64>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
+    return tile_passes_of<RB, 1024, 16, u64>(ctx, d_in, n, lo_bits, xf, dbits, passes, d_out);
 }
 
 // Shared driver of sort and sort+unique.  For n <= 4096 with `unique`,

@@ -86,3 +86,82 @@ def test_tile_words_of_a_large_merge_are_counted(ctx):
         assert diff(1 << 20) == 0 and np.array_equal(d.numpy(m.value), want)
     for x in (f, t, d):
         x.free()
+
+
+def block(nbytes):
+    """The allocator's block for a request of a call's scratch."""
+    nbytes += 16
+    step = 1 << max(nbytes.bit_length() - 4, 0)
+    return 512 if nbytes <= 512 else -(-nbytes // step) * step
+
+
+# A sort of n keys fits room for a second buffer of them, a count per digit (9
+# bits) and 4096 keys, and the digits' totals (and an eighth of the counts, the
+# step of the allocator's blocks).
+def sort_room(n):
+    counts = 4 * 512 * -(-n // 4096)
+    return block(8 * n) + block(counts) + counts // 8 + block(4 * 512)
+
+
+@pytest.mark.parametrize("n", [4097, 12_289, 100_000, 1 << 18, (1 << 18) + 1, 700_001, 1 << 20,
+                               1_500_000])
+def test_sort_in_little_scratch(ctx, n):
+    keys = gdl.pack(*np.random.default_rng(n).integers(0, 1 << 18, (2, n)))
+    d, o = ctx.to_device(keys), ctx.alloc(n)
+    ctx.release_cached()
+    ctx.set_mem_cap(ctx.mem_info()["in_use"] + sort_room(n))
+    try:
+        for _ in range(2):
+            ctx._check(ctx.eng.gdl_sort_u64(ctx.h, d.ptr, n, 18, 18, o.ptr), "sort")
+    finally:
+        ctx.set_mem_cap(0)
+    assert np.array_equal(o.numpy(), np.sort(keys))
+    d.free(); o.free()
+
+
+# From 2^30 keys on a tile's digit counts take 64-bit words (tiles of 16384
+# keys); the recorded form replays with other keys.
+@pytest.mark.parametrize("recorded", [False, True])
+def test_sort_of_more_than_2_to_the_30_keys(ctx, recorded):
+    torch = pytest.importorskip("torch")
+    n = (1 << 30) + 12_345
+    if torch.cuda.mem_get_info()[0] < 120 << 30:
+        pytest.skip("needs 120 GB of device memory")
+    ctx.stats_enable(False)
+    ctx.release_cached()
+    keys = torch.empty(n, dtype=torch.int64, device="cuda")
+    out = torch.empty_like(keys)
+
+    def draw(seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        torch.randint(0, 1 << 36, (n,), device="cuda", generator=g, out=keys)
+        keys.copy_(((keys >> 18) << 32) | (keys & 0x3ffff))
+        out.zero_()
+        torch.cuda.synchronize()
+
+    def sort():
+        ctx._check(ctx.eng.gdl_sort_u64(ctx.h, keys.data_ptr(), n, 18, 18, out.data_ptr()), "sort")
+
+    def right():
+        ctx.sync()
+        return bool(torch.equal(out, torch.sort(keys)[0]))
+
+    draw(1)
+    ctx.set_mem_cap(ctx.mem_info()["in_use"] + sort_room(n))
+    try:
+        sort()
+    finally:
+        ctx.set_mem_cap(0)
+    assert right()
+    if recorded:
+        ctx.graph_begin()
+        sort()
+        g = ctx.graph_end()
+        for seed in (2, 3):
+            draw(seed)
+            ctx.graph_launch(g)
+            assert right()
+        ctx.graph_destroy(g)
+    del keys, out
+    torch.cuda.empty_cache()
+    ctx.release_cached()
