@@ -310,7 +310,7 @@ static gdl_status compact_impl(gdl_ctx *ctx, const u64 *d_in, u64 n, F flag, u64
     TileLook look;
     GDL_TRY(tile_look(ctx, nt, &scr, &look));
     {
-        KTimer kt(ctx, K_COMPACT, 16.0 * n);
+        KTimer kt(ctx, K_COMPACT, 8.0 * n);  // and the kept keys' writes, below
         auto launch = [&](auto kern, int block) {
             hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(block), 0, ctx->stream, d_in, n,
                                flag, look, d_out, result_words(ctx));
@@ -319,7 +319,9 @@ static gdl_status compact_impl(gdl_ctx *ctx, const u64 *d_in, u64 n, F flag, u64
         else launch(k_compact<TB, F>, TB);
         GDL_TRY(check_launch(ctx, "k_compact"));
     }
-    return read_result(ctx, n_out);
+    GDL_TRY(read_result(ctx, n_out));
+    ctx->stats[K_COMPACT].alg_bytes += 8.0 * (double)*n_out;
+    return GDL_OK;
 }
 
 gdl_status unique_keys(gdl_ctx *ctx, const u64 *d_in, u64 n, u64 *d_out, u64 *n_out) {

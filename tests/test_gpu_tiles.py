@@ -175,6 +175,17 @@ def test_compaction_at_tile_edges(ctx, n, kind):
     assert np.array_equal(ctx.filter(keys, gdl.PRED_EQ | 0x100, 0, 7), keys[keep])
 
 
+# what a compaction reads, and the keys it keeps
+@pytest.mark.parametrize("n,kept", [(1000, 1), (50_000, 50_000), (1_200_000, 240_000)])
+def test_compaction_counts_the_bytes_it_moves(ctx, n, kept):
+    keys = (np.arange(n) // (n // kept)).astype(np.uint64)
+    ctx.stats_reset()
+    assert ctx.unique(keys).size == kept
+    s = ctx.stats()["compact"]
+    ctx.stats_reset()
+    assert s["launches"] == 1 and s["alg_bytes"] == 8 * (n + kept)
+
+
 # one launch up to 2^22 values, three above; 2048 values a tile
 @pytest.mark.parametrize("n", [1, 8, 2047, 2048, 2049, 100_000, 1 << 22, (1 << 22) + 1])
 def test_join_offsets_at_tile_edges(ctx, n):
