@@ -298,6 +298,24 @@ def test_dense_sg_bodies_two_relations(ctx, kb, mode, same):
     _check_run(got, want, delta, fs)
 
 
+# the largest domain: its row offsets are read back by a copy (more than 1 MB),
+# beside ranges that one launch gathers
+@pytest.mark.gpu
+@pytest.mark.parametrize("kb", [16, 17])
+def test_dense_tc_bodies_over_the_largest_domains(ctx, kb):
+    rng = np.random.default_rng(kb)
+    ids = np.append(rng.choice((1 << kb) - 1, 1999, replace=False), (1 << kb) - 1)
+    e = np.unique(gdl.pack(ids[rng.integers(0, 2000, 2200)], ids[rng.integers(0, 2000, 2200)]))
+    want, fs = tc_bodies(reverse(e), e, e, max_bodies=6)
+    ctx.set_dense_mode(2)
+    try:
+        got = ctx.fixpoint_dense(gdl.DENSE_TC, kb, e, e, reverse(e), max_bodies=6)
+    finally:
+        ctx.set_dense_mode(1)
+    _check_run(got, want, e, fs)
+    ctx.release_cached()
+
+
 @pytest.mark.gpu
 def test_dense_bodies_stop_at_max_bodies_and_resume(ctx):
     e = np.unique(GRAPHS["er_1000"]())

@@ -136,12 +136,16 @@ def _sorted(rng, n, hi):
         np.zeros(0, np.uint64)
 
 
-# tiles are 2048 keys of the merged sequence; a tile may hold one side only,
-# and a duplicate may be the first key of a tile
+# tiles are 2048 keys of the merged sequence, 8192 from 2^19 on; a tile may hold
+# one side only, and a duplicate may be the first key of a tile
+BIG = 1 << 18
 @pytest.mark.parametrize("na,nb,hi", [
     (0, 1, 9), (1, 0, 9), (1, 1, 1), (2047, 1, 5000), (1024, 1024, 2048), (1024, 1024, 1024),
     (2048, 2048, 2048), (2049, 2047, 4097), (5000, 5000, 5500), (100_000, 10, 10**6),
-    (10, 100_000, 10**6), (300_001, 299_999, 600_000), (700_000, 700_000, 700_000)])
+    (10, 100_000, 10**6), (300_001, 299_999, 600_000), (700_000, 700_000, 700_000),
+    (BIG, BIG - 1, 2 * BIG), (BIG, BIG, BIG), (BIG + 4096, BIG + 4095, 600_000),
+    (BIG + 4096, BIG + 4096, BIG + 4096), (BIG + 4097, BIG + 4096, 600_000),
+    (2 * BIG + 8192, 1, 600_000), (1, 2 * BIG + 8192, 600_000)])
 def test_merge_at_tile_edges(ctx, na, nb, hi):
     rng = np.random.default_rng(na * 7 + nb)
     a, b = _sorted(rng, na, hi), _sorted(rng, nb, hi)
@@ -164,12 +168,12 @@ def test_tile_words_are_tagged_anew(ctx):
 
 # tiles of 4096 keys, of 16384 from 2^20 keys on
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 4095, 4096, 4097, 12_289, (1 << 20) - 1, 1 << 20,
-                               (1 << 20) + 1, 2_000_003])
+                               (1 << 20) + 1, (1 << 20) + 16_383, (1 << 20) + 16_385, 2_000_003])
 @pytest.mark.parametrize("kind", ["none", "all", "half", "last", "tile_firsts"])
 def test_compaction_at_tile_edges(ctx, n, kind):
     i = np.arange(n)
     keep = {"none": i < 0, "all": i >= 0, "half": i % 2 == 1, "last": i == n - 1,
-            "tile_firsts": i % 4096 == 0}[kind]
+            "tile_firsts": i % (4096 if n < 1 << 20 else 16_384) == 0}[kind]
     # c0 == 7 where kept (a predicate on a column), c1 tells the keys apart
     keys = gdl.pack(np.where(keep, 7, 8), i)
     assert np.array_equal(ctx.filter(keys, gdl.PRED_EQ | 0x100, 0, 7), keys[keep])
@@ -186,9 +190,24 @@ def test_compaction_counts_the_bytes_it_moves(ctx, n, kept):
     assert s["launches"] == 1 and s["alg_bytes"] == 8 * (n + kept)
 
 
-# one launch up to 2^22 values, three above; 2048 values a tile
-@pytest.mark.parametrize("n", [1, 8, 2047, 2048, 2049, 100_000, 1 << 22, (1 << 22) + 1])
+# one launch up to 2^22 values, three above; 2048 values a tile, 8192 from 2^18 on
+SCAN_SIZES = [1, 8, 2047, 2048, 2049, 100_000, BIG - 1, BIG, BIG + 1, BIG + 8191, BIG + 8193,
+              1 << 22, (1 << 22) + 1]
+
+
+# a join's run starts and their scan: the same sizes of the outer relation
+@pytest.mark.parametrize("n", SCAN_SIZES)
 def test_join_offsets_at_tile_edges(ctx, n):
+    lengths = [i % 4 for i in range(1000)]
+    inner = runs_of(lengths)
+    outer = gdl.pack((np.arange(n) * 7919) % 1009, np.arange(n))
+    ik, ok, _ = np_join_runs(inner, outer)
+    got = ctx.join(inner, outer, (1, 3))
+    assert np.array_equal(got, ((ik & M32) << np.uint64(32)) | (ok & M32))
+
+
+@pytest.mark.parametrize("n", SCAN_SIZES)
+def test_scan_at_tile_edges(ctx, n):
     import ctypes
     counts = (np.arange(n, dtype=np.uint64) * np.uint64(2654435761) & M32).astype(np.uint32)
     counts[::3] = 0
@@ -223,9 +242,10 @@ def test_sort_at_tile_edges(ctx, n, kind):
 
 
 # a linear body's blocks hand over their counts packed in one word up to 2^27
-# produced tuples and 1023 blocks of 1024 outer tuples, in words of their own
-# above; the ids need a hash set
-@pytest.mark.parametrize("paths", [1, 1023, 1025, 400_000, 1_200_000])
+# produced tuples and 1023 blocks (of 256 outer tuples up to 2^16 of them, of
+# 512 above), in words of their own above; the ids need a hash set
+@pytest.mark.parametrize("paths", [1, 1023, 1025, 21_845, 21_846, 174_592, 174_593, 400_000,
+                                   1_200_000])
 def test_linear_bodies_of_disjoint_paths(ctx, paths):
     # node j of path i is i + j * paths + 2^19: three edges a path, in any order
     i = np.arange(paths, dtype=np.uint64) + np.uint64(1 << 19)
@@ -237,6 +257,23 @@ def test_linear_bodies_of_disjoint_paths(ctx, paths):
     assert np.array_equal(got["out"], want)
     assert [t[3] for t in got["trace"]] == [2 * paths, paths, 0]
     assert [t[2] for t in got["trace"]] == [2 * paths, paths, 0]
+
+
+# with runs of up to 1000 the limit of 2^27 produced tuples is a delta of
+# 134,217: first deltas on both sides of it, and one that grows past it
+@pytest.mark.parametrize("first", [134_216, 134_217, 134_218, 1200])
+def test_linear_bodies_around_the_packed_limit(ctx, first):
+    base, ins, outs = 1 << 19, np.arange(1000), np.arange(100 if first > 1200 else 200)
+    hub, extra = 0, np.arange(first - ins.size - outs.size)
+    into = gdl.pack(base + 1 + ins, np.full(ins.size, base + hub))
+    out = gdl.pack(np.full(outs.size, base + hub), base + 5000 + outs)
+    alone = gdl.pack(base + 10_000 + 2 * extra, base + 10_001 + 2 * extra)
+    edges = np.concatenate([into, out, alone])
+    pairs = gdl.pack(np.repeat(base + 1 + ins, outs.size), np.tile(base + 5000 + outs, ins.size))
+    got = ctx.run_tc(edges, out_cap=edges.size + pairs.size)
+    assert np.array_equal(got["out"], np.sort(np.concatenate([edges, pairs])))
+    assert [t[3] for t in got["trace"]] == [pairs.size, 0]
+    assert [t[2] for t in got["trace"]] == [pairs.size, 0]
 
 
 # a result of n keys goes straight into a buffer that holds it; a smaller one
