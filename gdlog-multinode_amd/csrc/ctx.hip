@@ -222,7 +222,10 @@ gdl_status Staging::send() {
         u64 words = 0;
         for (; sent_ < pending_.size() && a.count < kGather; ++sent_) {
             const Pending &p = pending_[sent_];
-            // (places in the buffer are 256-byte aligned)
+            // (places in the buffer are 256-byte aligned; a dense set-up over
+            // 2^15 and 2^16 ids, whose ranges are of 128 to 512 kB, takes 20-30
+            // us longer with a copy command for those above 64 kB, one over
+            // 2^17, of 1 MB, the same)
             if (p.n % 4 || p.n > (1u << 20)) {
                 GDL_HIP(ctx_, hipMemcpyAsync(ctx_->h_stage + p.at, p.d_src, p.n,
                                              hipMemcpyDeviceToHost, ctx_->stream));

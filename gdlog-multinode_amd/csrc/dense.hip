@@ -226,7 +226,8 @@ static gdl_status bitmap_extract_sorted(gdl_ctx *ctx, const u64 *words, int kb, 
 // The counters of the running body, one set per group of blocks (blockIdx mod
 // kGroups), each on a line of its own: atomics on one line take 11 ns one after
 // another, and with a single set the counters of a body's 2048 combine, 2048
-// row-OR and 4096 transpose blocks took 50-110 us of its time.
+// row-OR and 4096 transpose blocks took 50-110 us of its time.  A few TC bodies
+// over 2^13 ids: 488 us with 8 groups, 437 with 16, 418 with 32 and with 64.
 constexpr u32 kGroups = 32;
 enum DenseCounter {
     DC_NEW,       // new tuples
@@ -311,8 +312,10 @@ __device__ __forceinline__ void group_add(DenseState *st, DenseCounter c, u64 v)
 // Counts this block as finished in its group and the group, when it is its
 // last block, among the groups (one thread of each block); true for the last
 // block of all.  *mine is back at 0 after the last block of its group.  A grid
-// of up to kOneGroup blocks is one group: one atomic less in a row.
+// of up to kOneGroup blocks is one group: one atomic less in a row (32 the same
+// within 2 %, 256 slower by 2 % over 2^13 ids).
 constexpr u32 kOneGroup = 64;
+static_assert(kOneGroup + 1 >= kGroups, "above it every group has a block");
 __device__ __forceinline__ bool last_of_groups(DenseState *st, u32 DenseGroup::*done,
                                                u32 *groups) {
     order_memory();
@@ -1152,7 +1155,10 @@ __global__ __launch_bounds__(DB) void k_dense_planes(const u64 *off, u64 rw, int
 // A block counts `per` * DB keys in an LDS table of rows (per at most kMarkPer)
 // and adds each row once (a row that finds no place adds directly): a hub row's
 // keys all add to one word, 11 ns each, which took 0.25-0.37 ms for the first
-// delta of SG on an R-MAT graph of 40,000 edges.
+// delta of SG on an R-MAT graph of 40,000 edges.  Set-up over 2^15 ids, 2M keys
+// of skewed rows in any order: 498 us with up to 4 * DB keys a block, 258 with
+// 16 and with 64 (4M keys in order 175, 172, 181); 273 us with 1024 rows in the
+// table, 258 with 4096, 320 with 8192, whose blocks are fewer per CU.
 constexpr int kMarkPer = 16;
 constexpr u32 kMarkSlots = 4096, kNoRow = ~0u;
 __global__ __launch_bounds__(DB) void k_dense_mark(const u64 *keys, u64 n, int per, u32 slot_mask,
@@ -2209,7 +2215,8 @@ gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
             const double row = 8.0 * (double)rw;
             // combine: the pred rows read (D, and SG's U), FULL's row read,
             // the new delta row written, new words set in FULL
-            ctx->stats[K_DENSE_COMBINE].alg_bytes += row * (double)cb[DC_ROWS_IO] + 8.0 * (double)cb[0];
+            ctx->stats[K_DENSE_COMBINE].alg_bytes +=
+                row * (double)cb[DC_ROWS_IO] + 8.0 * (double)cb[0];
             // expansion bit by bit: the delta row read, U's row written, one
             // 16-byte entry per delta bit; by columns: the 64-byte segments
             // the transposes read and wrote, the OR's row reads and writes
@@ -2220,7 +2227,8 @@ gdl_status dense_run(gdl_ctx *ctx, const gdl_dense_rule *rule, gdl_hashset *hs,
             ctx->stats[K_DENSE_ORROWS].alg_bytes += row * (double)cb[DC_OR_IO];
             // append: the rows with new tuples read, their keys written
             if (!log_last)
-                ctx->stats[K_DENSE_APPEND].alg_bytes += row * (double)cb[DC_ROWS_NEW] + 8.0 * (double)cb[0];
+                ctx->stats[K_DENSE_APPEND].alg_bytes +=
+                    row * (double)cb[DC_ROWS_NEW] + 8.0 * (double)cb[0];
             in_delta = cb[0];
             last_rows = cb[DC_ROWS_NEW];
             hs->size += cb[0];

@@ -88,7 +88,9 @@ __device__ __forceinline__ u32 span_runs(const u64 *keys, u64 n, int shift, u64 
 }
 
 // Spans of 1024 keys a wave (R = 16) for large arrays; of 256 below 2^22 keys,
-// where the longer ones leave CUs without a wave.  The hash build takes 256
+// where the longer ones leave CUs without a wave: count and build of 2M keys 48
+// us with short spans and 54 with long, of 4M 60 and 63, of 4.2M 61-63 and
+// 60-64, of 8M 73-75 and 76-79, of 16M 119 and 102.  The hash build takes 256
 // and 64: its lanes insert one run after another, a chain of atomics that
 // grows with the span (1M keys in 400k runs: 37 us with 64 or 256).
 constexpr u64 kLongSpan = 1ull << 22;
@@ -1405,15 +1407,16 @@ gdl_status gdl_fixpoint_linear(gdl_ctx *ctx, const uint64_t *d_inner, uint64_t n
     // at most 128 bodies per host wait (on the 200k-node tree 128 beat 32 by
     // 2.5 %; 64 did not; a chunk that stops early leaves no-op launches)
     constexpr int kChunk = 128;
-    // a body is bound by the latency of each tuple's chain of dependent
-    // accesses (~0.6 us a load) and by the set's atomics (25e9 a second at
-    // random places, whatever their scope: 8 of the 21 us of a body of 190k
-    // outer tuples; its key 5, the end of its blocks 1.4, its launch 4), so every outer tuple gets its own
-    // lane (more chains in flight).  Blocks of 512 (each ends with an atomic on
-    // the shared cursor, 11 ns one after another, but also waits for its
-    // slowest wave): 17.1 us a body on the 200k-node tree, 18.0 with 256 and
-    // 18.4 with 1024; of 256 up to 2^16 outer tuples (50,000 nodes: 9.4
-    // against 10.3 us)
+    // a body is bound by its launch and the latency of each tuple's chain of
+    // dependent accesses (~0.6 us a load): of the 21 us of a body of 190k outer
+    // tuples the launch takes 4, the key 5, the insert 8 (what its atomics take
+    // at their rate, 25e9 a second at random places whatever their scope; 4 of
+    // the 17 us of the tree's average body), the end of its blocks 1.4.  So
+    // every outer tuple gets its own lane (more chains in flight).  Blocks of 512
+    // (each ends with an atomic on the shared cursor, 11 ns one after another,
+    // but also waits for its slowest wave): 17.1 us a body on the 200k-node tree,
+    // 18.0 with 256 and 18.4 with 1024; of 256 up to 2^16 outer tuples (50,000
+    // nodes: 9.4 against 10.3 us)
     const int shift = inner_idx->prefix_cols >= 2 ? 0 : 32;
     const u64 mr = std::max<u64>(inner_idx->max_run, 1);
     Scratch scr(ctx);

@@ -5,8 +5,9 @@
 // A B-key is a duplicate exactly when the A-key consumed just before it is
 // equal (equal keys are adjacent in merge order and A goes first).
 //
-// One launch: a block takes a tile of keys of the merged sequence, finds where its B-keys go among its A-keys, counts the duplicates, learns how many
-// the tiles before hold (tile_before), and writes its part of U and D.
+// One launch: a block takes a tile of keys of the merged sequence, finds where
+// its B-keys go among its A-keys, counts the duplicates, learns how many the
+// tiles before hold (tile_before), and writes its part of U and D.
 #include "gdl_internal.hpp"
 
 namespace gdl {
@@ -176,7 +177,8 @@ static gdl_status merge_impl(gdl_ctx *ctx, const u64 *A, u64 na, const u64 *B, u
     }
     // Tickets come at 11 ns each (atomics on one word), so 41M + 2M keys in
     // tiles of 2048 took 395 us, 240 of them in 21,000 tickets; in tiles of
-    // 8192 keys it takes 235 us.  Below 2^19 keys the smaller tiles spread over more CUs.
+    // 8192 keys it takes 235 us.  Below 2^19 keys the smaller tiles spread over
+    // more CUs.
     const bool big = tot >= 1ull << 19;
     const u64 tile = (big ? 1024 : 256) * MG_I, nt = (tot + tile - 1) / tile;
     if (nt > 0x7fffffffull) return fail(ctx, GDL_ERR_OVERFLOW, "merge: too many tiles");

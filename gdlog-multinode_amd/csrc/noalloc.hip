@@ -20,8 +20,8 @@ namespace gdl {
 
 static constexpr uint64_t kNoallocMaxKeys = GDL_NOALLOC_MAX_KEYS;
 // Worst case for kNoallocMaxKeys keys: the sorted copy (8n) and the radix
-// ping-pong buffer (8n), two arrays of 2^9 digit counts per 4096-key tile, and
-// the passes' digit counts, each piece 256-byte aligned.
+// ping-pong buffer (8n), and two arrays of 2^9 digit counts per 4096-key tile
+// (2048-key tiles of up to 2^18 keys need less), each piece 256-byte aligned.
 static constexpr size_t kScratchBytes = 18u << 20;
 static_assert(kScratchBytes >= 16 * GDL_NOALLOC_MAX_KEYS +
                                    2 * 4 * 512 * (GDL_NOALLOC_MAX_KEYS / 4096) + (64u << 10),

@@ -148,9 +148,9 @@ struct PrefixDiffFlag {
 
 // Writes the kept keys of a tile after those of the tiles before it
 // (tile_before), the total to *n_out: one read of the keys in one launch.
-// 41M sorted keys, 31M distinct: 0.146 ms, 3.9 TB/s (a count launch, a scan and a write
-// launch took 0.078 + 0.008 + 0.131); CSPA's small ones 7.2 us instead of
-// 7.1 + 3 + 6.
+// 41M sorted keys, 31M distinct: 0.146 ms, 3.9 TB/s (a count launch, a scan and
+// a write launch took 0.078 + 0.008 + 0.131); CSPA's small ones 7.2 us instead
+// of 7.1 + 3 + 6.
 template <int B, typename F>
 __global__ __launch_bounds__(B) void k_compact(const u64 *in, u64 n, F flag, TileLook look,
                                                u64 *out, u64 *n_out) {

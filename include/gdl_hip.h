@@ -486,7 +486,11 @@ typedef struct gdl_kernel_stat {
 gdl_status gdl_stats_enable(gdl_ctx *ctx, int enable);
 gdl_status gdl_stats_reset(gdl_ctx *ctx);
 /* Resolves pending events (synchronises) and returns the number of kernel
- * classes; fills up to `cap` entries. */
+ * classes; fills up to `cap` entries.  The names are those of the engine's
+ * present kernels and change with them (a sort is "rs_hist" and "rs_pass", a
+ * merge "merge", a unique or filter "compact", a scan "scan_one" or
+ * "scan_reduce" / "scan_top" / "scan_down"): look a class up by name only with
+ * a default for one that is not there. */
 gdl_status gdl_stats_get(gdl_ctx *ctx, gdl_kernel_stat *out, int cap, int *n_out);
 
 #ifdef __cplusplus
