@@ -333,6 +333,42 @@ def test_sort_in_a_graph(ctx, n):
     d.free(); o.free()
 
 
+# recorded sorts share one set of digit counts: two in one graph, and two graphs
+# in turn, with a sort between
+def test_recorded_sorts_take_turns(ctx):
+    ctx.stats_enable(False)
+    rng = np.random.default_rng(3)
+    sizes = [5000, 300_000, 40_000]
+    d, o = [ctx.alloc(n) for n in sizes], [ctx.alloc(n) for n in sizes]
+
+    def sort(i):
+        ctx._check(ctx.eng.gdl_sort_u64(ctx.h, d[i].ptr, sizes[i], 18, 18, o[i].ptr), "sort")
+
+    for i in range(3):
+        sort(i)
+    ctx.sync()
+    graphs = []
+    for which in ((0, 1), (2,)):
+        ctx.graph_begin()
+        for i in which:
+            sort(i)
+        graphs.append(ctx.graph_end())
+    for _ in range(4):
+        keys = [gdl.pack(rng.integers(0, 1 << 18, n), rng.integers(0, 1 << 18, n)) for n in sizes]
+        for i in range(3):
+            ctx._check(ctx.eng.gdl_memcpy_h2d(ctx.h, d[i].ptr, keys[i].ctypes.data,
+                                              keys[i].nbytes), "h2d")
+        ctx.graph_launch(graphs[0])
+        ctx.graph_launch(graphs[1])
+        assert np.array_equal(ctx.sort(keys[1], 18, 18), np.sort(keys[1]))
+        for i in range(3):
+            assert np.array_equal(o[i].numpy(), np.sort(keys[i]))
+    for g in graphs:
+        ctx.graph_destroy(g)
+    for x in d + o:
+        x.free()
+
+
 # a block takes 4096 slots a round, the last round holds the word of the key ~0
 @pytest.mark.parametrize("n", [0, 1, 700, 5000, 300_000])
 @pytest.mark.parametrize("top", [False, True])
